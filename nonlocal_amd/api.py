@@ -399,17 +399,17 @@ class preconditioner:
         return dict(ok=bool(ok.value), shift=shift.value, fw_levels=fw.value, bw_levels=bw.value, seconds=sec.value)
 
     def sweep_info(self):
-        """ILLT sweep layout (nlf_precond_sweep_info): per sweep the levels as swept, the compute
-        width, the levels of the LDS dependency window and the kernel (0 packed, 1 ELL one level at a
-        time, 2 ELL with prefetch)."""
+        """ILLT sweep layout (nlf_precond_sweep_info): per sweep the levels as swept, their width, the
+        steps of the LDS dependency window and the kernel (2 chunks of rows side by side, 0 one
+        workgroup)."""
         out = (C.c_int32 * 8)()
         self.ctx.check(load().nlf_precond_sweep_info(self.h, out))
         keys = ("levels", "width", "window_levels", "kernel")
         return {"forward": dict(zip(keys, out[0:4])), "backward": dict(zip(keys, out[4:8]))}
 
     def blocks(self):
-        """Independent diagonal blocks of an ILLT's matrix, each factored and swept by a workgroup
-        of its own (nlf_precond_blocks)."""
+        """Independent diagonal blocks of an ILLT's matrix, each factored by a workgroup of its own
+        and swept in chunks of its own (nlf_precond_blocks)."""
         out = C.c_int32()
         self.ctx.check(load().nlf_precond_blocks(self.h, C.byref(out)))
         return out.value

@@ -425,7 +425,7 @@ i64 batch_cg(nlf_batch B, const V* val, const double* b, double* x, double tol, 
         batch_spmv<double, false>(P, A, A->val.p, x, q.p, nullptr, start ? nullptr : st.p, s);
         if (M) {
             hipLaunchKernelGGL(k_bsub, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, b, q.p, rt.p);
-            precond_apply<double>(M, n, rt.p, zt.p, nullptr, s);
+            precond_apply(M, n, rt.p, zt.p, nullptr, s);
         }
         hipLaunchKernelGGL(k_bresidual, dim3(P.v_blocks), dim3(BATCH_VROWS), 0, s, P.v_inst.p, P.v_row0.p, P.row_begin.p, b,
                            q.p, r.p, z.p, p.p, B->invd.p, M ? (const double*)zt.p : nullptr, pa.p, pb.p, pc.p, pd.p, pe.p,
@@ -442,7 +442,7 @@ i64 batch_cg(nlf_batch B, const V* val, const double* b, double* x, double tol, 
         hipLaunchKernelGGL(k_bupdate, dim3(P.v_blocks), dim3(BATCH_VROWS), 0, s, P.v_inst.p, P.v_row0.p, P.row_begin.p, x,
                            r.p, p.p, q.p, z.p, M ? (const double*)nullptr : B->invd.p, pb.p, st.p);
         if (M) {
-            precond_apply<double>(M, n, r.p, z.p, nullptr, s);
+            precond_apply(M, n, r.p, z.p, nullptr, s);
             hipLaunchKernelGGL(k_bdot, dim3(P.v_blocks), dim3(BATCH_VROWS), 0, s, P.v_inst.p, P.v_row0.p, P.row_begin.p, r.p,
                                z.p, pb.p, (const BatchState*)st.p);
         }

@@ -7,10 +7,10 @@
 // with no host synchronisation; the host reads the state every few iterations.
 //
 // ILLT: IC(0) of the local matrix, diagonal scaling s = 1/sqrt|a_ii| and shift retries (our choice:
-// Eigen::IncompleteCholesky is not vendored, so its factor is not reproduced).  Factorisation and
-// both triangular solves are level-scheduled: rows are grouped by dependency level (computed once on
-// the host from the pattern) and one persistent 1024-thread workgroup sweeps the levels with a
-// barrier between them.
+// Eigen::IncompleteCholesky is not vendored, so its factor is not reproduced).  Rows are grouped by
+// dependency level (computed once on the host from the pattern).  The factorisation is one persistent
+// 1024-thread workgroup per independent block with a barrier between levels; the triangular sweeps run
+// as a dataflow over chunks of rows (nlf_sweep.inl).
 #include "nlf_internal.hpp"
 
 #include <mutex>
@@ -506,36 +506,34 @@ __global__ __launch_bounds__(LEVEL_THREADS) void k_ic_factor(LevelArgs a, const 
     }
 }
 
-// One triangular sweep in level order.  Records (one per row) are stored contiguously in level
+// One triangular sweep in level order, for rows with more dependencies than the chunked sweeps take.  Records (one per row) are stored contiguously in level
 // order so a level's loads are coalesced; a dependency on a row solved at most K levels earlier is
 // read from an LDS window of K x W slots (slot = (level mod K) * W + position in level), otherwise
 // (dep < 0) from global memory.
-template<class X>
 struct PackedSweep {
     int levels, K, W;
     const i32* lptr;      // [levels+1] record offsets
     const i32* row;       // row of each record
     const i32* off;       // [records+1] entry offsets
     const i32* dep;       // window slot, or -(row+1)
-    const X* val;         // factor entries
-    const X* dinv;        // 1 / U_kk
-    const X* scale;       // s_k
+    const double* val;         // factor entries
+    const double* dinv;        // 1 / U_kk
+    const double* scale;       // s_k
 };
 
 // z = S U^-1 U^-T S r : forward U^T y = S r, backward U z' = y, z = S z'.  One workgroup.
-template<class X>
-__global__ __launch_bounds__(LEVEL_THREADS) void k_ic_solve(PackedSweep<X> fw, PackedSweep<X> bw, const X* __restrict__ r,
-                                                            X* __restrict__ y, X* __restrict__ z,
+__global__ __launch_bounds__(LEVEL_THREADS) void k_ic_solve(PackedSweep fw, PackedSweep bw, const double* __restrict__ r,
+                                                            double* __restrict__ y, double* __restrict__ z,
                                                             const CGState* __restrict__ st) {
     extern __shared__ unsigned char smem_raw[];
-    X* win = reinterpret_cast<X*>(smem_raw);
+    double* win = reinterpret_cast<double*>(smem_raw);
     if (st && st->done) return;
     for (int L = 0; L < fw.levels; ++L) {
         const i32 b = fw.lptr[L], cnt = fw.lptr[L + 1] - b;
         for (i32 t = threadIdx.x; t < cnt; t += blockDim.x) {
             const i32 rec = b + t;
             const i32 k = fw.row[rec];
-            X v = fw.scale[rec] * r[k];
+            double v = fw.scale[rec] * r[k];
             for (i32 e = fw.off[rec]; e < fw.off[rec + 1]; ++e) {
                 const i32 d = fw.dep[e];
                 v -= fw.val[e] * (d >= 0 ? win[d] : y[-d - 1]);
@@ -551,7 +549,7 @@ __global__ __launch_bounds__(LEVEL_THREADS) void k_ic_solve(PackedSweep<X> fw, P
         for (i32 t = threadIdx.x; t < cnt; t += blockDim.x) {
             const i32 rec = b + t;
             const i32 k = bw.row[rec];
-            X v = y[k];
+            double v = y[k];
             for (i32 e = bw.off[rec]; e < bw.off[rec + 1]; ++e) {
                 const i32 d = bw.dep[e];
                 v -= bw.val[e] * (d >= 0 ? win[d] : y[-d - 1]);
@@ -565,276 +563,17 @@ __global__ __launch_bounds__(LEVEL_THREADS) void k_ic_solve(PackedSweep<X> fw, P
     }
 }
 
-// ELL form of one sweep for the fast path: every level is a block of `cnt` records with exactly WE
-// entry slots each, stored record-major (entry j of record rec at WE * rec + j), so that a lane
-// loads a record's values and dependency slots with 16-byte loads and a wave's loads of one level
-// cover one contiguous span; padding slots carry value 0 and a dependency on slot 0 of the
-// (zero-initialised) window.
-template<class X>
-struct EllSweep {
-    int levels, K, W;
-    const i32* lptr;
-    const i32* row;
-    const i32* dep;          // window slot (K > 0) or -(row + 1) of a dependency read from the output
-    const X* val;
-    const X* dinv;
-};
-
-
-// rhs_lvl[rec] = scale[rec] * r[row[rec]] (forward) or y[row[rec]] (backward, scale == nullptr);
-// also clears `clear` (the sweep's output, read through global dependencies).
-template<class X>
-__global__ void k_sweep_gather(i64 n, const i32* __restrict__ row, const X* __restrict__ scale, const X* __restrict__ src,
-                               X* __restrict__ rhs_lvl, X* __restrict__ clear, const CGState* __restrict__ st) {
-    if (st && st->done) return;
-    for (i64 t = i64(blockIdx.x) * blockDim.x + threadIdx.x; t < n; t += i64(gridDim.x) * blockDim.x) {
-        const i32 k = row[t];
-        rhs_lvl[t] = scale ? scale[t] * src[k] : src[k];
-        if (clear) clear[t] = X(0);
-    }
-}
-
-// One level-scheduled triangular sweep by one workgroup.  The first `ct` threads (ct = blockDim - 64
-// SW, at least the widest level) compute: thread t owns record t of every level, and the record data
-// of level L + D (right-hand side, 1/U_kk, the WE entries and their dependency slots) are loaded D
-// levels ahead into a ring of D register slots, while the level offsets and every dependency live in
-// LDS; a level's critical path is the LDS reads of its dependencies, a few FMAs, the LDS write and
-// the barrier.  The last SW waves store: after the barrier of level L they copy the level's values
-// from the LDS window to out_lvl (level order), while level L + 1 is computed.
-//
-// Why the split: a wave's vector-memory counter covers loads and stores alike, and loads and stores
-// may complete out of order relative to each other, so while a wave has stores in flight any wait
-// for one of its loads must wait for everything (vmcnt 0), which drains the prefetch ring.  Compute
-// waves that never store wait for exactly the level they need.  For the same reason no load of the
-// level loop goes through a generic (flat) address.  The arithmetic of a record is unchanged; the
-// row-order results come from k_sweep_scatter.
-constexpr size_t SWEEP_LDS_BYTES = 64 * 1024;
-// Compute widths of the two prefetching sweeps and their store waves (workgroups of CT + 64 SW).
-#ifndef NLF_SWEEP_SW_SMALL
-#define NLF_SWEEP_SW_SMALL 2
-#endif
-#ifndef NLF_SWEEP_SW_LARGE
-#define NLF_SWEEP_SW_LARGE 2
-#endif
-constexpr int SWEEP_SW_SMALL = NLF_SWEEP_SW_SMALL, SWEEP_SW_LARGE = NLF_SWEEP_SW_LARGE;
-constexpr int SWEEP_CT_SMALL = 512, SWEEP_CT_LARGE = 1024 - 64 * SWEEP_SW_LARGE;
-
-// Levels the ring holds, sized so that the ring and the rest of a compute lane fit the registers a
-// lane has with CT compute lanes plus the store waves per workgroup (168 VGPRs up to 12 waves, 128
-// at 16) without spilling.
-template<int WE, int CT>
-constexpr int sweep_depth() {
-    return CT <= SWEEP_CT_SMALL ? (WE <= 4 ? 8 : WE <= 8 ? 4 : WE <= 16 ? 2 : 1) : (WE <= 4 ? 4 : WE <= 8 ? 2 : 1);
-}
-
-// N consecutive elements of type T by 16-byte loads (8-byte when N * sizeof(T) is 8); p is aligned
-// to the load size
-template<class T, int N>
-__device__ __forceinline__ void load16(const T* __restrict__ p, T (&v)[N]) {
-    constexpr int B = int(N * sizeof(T));
-    static_assert(B == 8 || B % 16 == 0, "record slots are whole 8- or 16-byte words");
-    if constexpr (B == 8) {
-        const uint2 w = *reinterpret_cast<const uint2*>(p);
-        __builtin_memcpy(v, &w, 8);
-    } else {
-        const uint4* q = reinterpret_cast<const uint4*>(p);
-#pragma unroll
-        for (int k = 0; k < B / 16; ++k) {
-            const uint4 w = q[k];
-            __builtin_memcpy(reinterpret_cast<unsigned char*>(v) + 16 * k, &w, 16);
-        }
-    }
-}
-
-template<class X, int WE, int CT, int SW>
-__global__ __launch_bounds__(CT + 64 * SW) void k_ic_sweep(EllSweep<X> s, const SweepBlock* __restrict__ blk,
-                                                           const X* __restrict__ rhs, X* __restrict__ out_lvl,
-                                                           const CGState* __restrict__ st) {
-    // blk: one sweep per workgroup over the records of independent diagonal blocks (a batch's
-    // instances).  Only the counts and the level offset come from memory: the record pointers stay
-    // kernel arguments, known global, so that their loads are not flat ones.
-    if (blk) {
-        const SweepBlock b = blk[blockIdx.x];
-        s.levels = b.levels;
-        s.K = b.K;
-        s.lptr += b.lptr_off;
-    }
-    constexpr int D = sweep_depth<WE, CT>();
-    extern __shared__ unsigned char smem_raw[];
-    X* win = reinterpret_cast<X*>(smem_raw);
-    i32* lp = reinterpret_cast<i32*>(smem_raw + ((size_t(s.K) * size_t(s.W) * sizeof(X) + 15) & ~size_t(15)));
-    if (st && st->done) return;
-    const int t = threadIdx.x;
-    const int ct = int(blockDim.x) - 64 * SW;
-    for (int i = t; i < s.K * s.W; i += blockDim.x) win[i] = X(0);
-    for (int i = t; i <= s.levels; i += blockDim.x) lp[i] = s.lptr[i];
-    __syncthreads();
-    // the compute waves run whole trips of D levels (the phantom levels past the last one recompute
-    // the last level's records into window slots no record reads): an exit inside the unrolled trip
-    // would make the compiler wait for every prefetched load at the top of each trip
-    const int padded = (s.levels + D - 1) / D * D;
-    if (t >= ct) {
-        // store waves: one barrier per level, like the compute waves, then that level's values
-        constexpr int PER = (CT + 64 * SW - 1) / (64 * SW);
-        const int lane = t - ct;
-        for (int L = 0; L < padded; ++L) {
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            if (L >= s.levels) continue;
-            const i32 b = lp[L], cnt = lp[L + 1] - b;
-            const X* src = win + (L % s.K) * s.W;
-            X v[PER];
-#pragma unroll
-            for (int k = 0; k < PER; ++k) {
-                const int i = lane + k * 64 * SW;
-                v[k] = i < cnt ? src[i] : X(0);
-            }
-#pragma unroll
-            for (int k = 0; k < PER; ++k) {
-                const int i = lane + k * 64 * SW;
-                if (i < cnt) out_lvl[b + i] = v[k];
-            }
-        }
-        return;
-    }
-    // The ring.  The loads of a level are issued by every compute thread (past the level's width a
-    // thread reads the level's last record again), so that each thread issues the same loads in the
-    // same order.  (Masking the idle lanes' loads and 16-bit dependency slots were both measured
-    // slower: the loads cost per instruction, and unpacking the slots lengthens the level.)
-    X r_rhs[D], r_dinv[D], r_val[D][WE];
-    i32 r_dep[D][WE];
-    auto load_at = [&](i32 b, i32 cnt, X& rv, X& dv, X (&vv)[WE], i32 (&dd)[WE]) {
-        const i32 rec = b + (t < cnt ? t : cnt - 1);
-        rv = rhs[rec];
-        dv = s.dinv[rec];
-        load16(s.val + i64(WE) * rec, vv);
-        load16(s.dep + i64(WE) * rec, dd);
-    };
-    auto load = [&](int L, X& rv, X& dv, X (&vv)[WE], i32 (&dd)[WE]) {
-        load_at(lp[L], lp[L + 1] - lp[L], rv, dv, vv, dd);
-    };
-    // the prologue issues the ring in slot order (the scheduling barrier keeps the compiler from
-    // grouping the loads by kind): the wait for slot u in the loop then counts only later slots
-#pragma unroll
-    for (int u = 0; u < D; ++u) {
-        load(min(u, s.levels - 1), r_rhs[u], r_dinv[u], r_val[u], r_dep[u]);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    // at least one trip (levels >= 1): a do-while has no zero-trip test, so no block for the
-    // optimiser to sink the prologue's loads into, out of slot order
-    int L0 = 0;
-    do {
-#pragma unroll
-        for (int u = 0; u < D; ++u) {
-            const int L = L0 + u;
-            // offsets of the level this slot is refilled with, read beside the dependencies
-            const int Ln = min(L + D, s.levels - 1);
-            const i32 nb = lp[Ln], ncnt = lp[Ln + 1] - nb;
-            // branch-free: a lane past the level's width holds the level's last record and computes
-            // that record's value again into its own window slot t >= width, which no record reads
-            // (the window stride is the compute width); the store waves copy only the first cnt
-            X v = r_rhs[u];
-#pragma unroll
-            for (int j = 0; j < WE; ++j) v -= r_val[u][j] * win[r_dep[u][j]];
-            v *= r_dinv[u];
-            win[(L % s.K) * s.W + t] = v;
-            // the slot is free once its level is computed: refill it before the barrier, so the
-            // address arithmetic and the load issue overlap the wait for the other waves
-            load_at(nb, ncnt, r_rhs[u], r_dinv[u], r_val[u], r_dep[u]);
-            // every dependency lives in the LDS window: wait for LDS traffic only, so the global
-            // loads prefetched for the next levels stay in flight across the barrier.  The
-            // scheduling barriers keep the compiler from hoisting a later level's address
-            // arithmetic above it, which would wait for that level's loads here.
-            __builtin_amdgcn_sched_barrier(0);
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        L0 += D;
-    } while (L0 < padded);
-}
-
-// Level order to row order: out[row[rec]] = v_lvl[rec]; out2[row[rec]] = scale2[rec] * v_lvl[rec].
-template<class X>
-__global__ void k_sweep_scatter(i64 n, const i32* __restrict__ row, const X* __restrict__ lvl,
-                                const X* __restrict__ scale2, X* __restrict__ out, X* __restrict__ out2,
-                                const CGState* __restrict__ st) {
-    if (st && st->done) return;
-    for (i64 t = i64(blockIdx.x) * blockDim.x + threadIdx.x; t < n; t += i64(gridDim.x) * blockDim.x) {
-        const i32 k = row[t];
-        const X v = lvl[t];
-        out[k] = v;
-        if (out2) out2[k] = scale2[t] * v;
-    }
-}
-
-// The same sweep when the dependency window or the level offsets do not fit LDS: dependencies
-// outside the window are read back from `out` (written by earlier levels of this workgroup), one
-// level at a time with no prefetch.
-template<class X, int WE>
-__global__ __launch_bounds__(LEVEL_THREADS) void k_ic_sweep_generic(EllSweep<X> s, const SweepBlock* __restrict__ blk,
-                                                                    const X* __restrict__ rhs, X* __restrict__ out,
-                                                                    X* __restrict__ out2, const X* __restrict__ scale2,
-                                                                    const CGState* __restrict__ st) {
-    if (blk) {
-        const SweepBlock b = blk[blockIdx.x];
-        s.levels = b.levels;
-        s.K = b.K;
-        s.lptr += b.lptr_off;
-    }
-    extern __shared__ unsigned char smem_raw[];
-    X* win = reinterpret_cast<X*>(smem_raw);
-    if (st && st->done) return;
-    const int t = threadIdx.x;
-    for (int i = t; i < s.K * s.W; i += blockDim.x) win[i] = X(0);
-    __syncthreads();
-    for (int L = 0; L < s.levels; ++L) {
-        const i32 b = s.lptr[L], cnt = s.lptr[L + 1] - b;
-        if (t < cnt) {
-            const i32 rec = b + t;
-            X v = rhs[rec];
-#pragma unroll
-            for (int j = 0; j < WE; ++j) {
-                const i32 d = s.dep[i64(WE) * rec + j];
-                v -= s.val[i64(WE) * rec + j] * (s.K ? win[d] : out[-d - 1]);
-            }
-            v *= s.dinv[rec];
-            if (s.K) win[(L % s.K) * s.W + t] = v;
-            const i32 k = s.row[rec];
-            out[k] = v;
-            if (out2) out2[k] = scale2[rec] * v;
-        }
-        __syncthreads();
-    }
-}
-
-__global__ void k_pack_ell(i64 n, const i64* __restrict__ src, const double* __restrict__ F, double* __restrict__ v64,
-                           float* __restrict__ v32) {
-    for (i64 e = i64(blockIdx.x) * blockDim.x + threadIdx.x; e < n; e += i64(gridDim.x) * blockDim.x) {
-        const double v = src[e] >= 0 ? F[src[e]] : 0.0;
-        v64[e] = v;
-        v32[e] = float(v);
-    }
-}
-
 // Gathers the factor into the packed sweep layout (values by source position, per-record 1/U_kk, s_k).
-__global__ void k_pack_entries(i64 n, const i64* __restrict__ src, const double* __restrict__ F, double* __restrict__ v64,
-                               float* __restrict__ v32) {
-    for (i64 e = i64(blockIdx.x) * blockDim.x + threadIdx.x; e < n; e += i64(gridDim.x) * blockDim.x) {
-        const double v = F[src[e]];
-        v64[e] = v;
-        v32[e] = float(v);
-    }
+__global__ void k_pack_entries(i64 n, const i64* __restrict__ src, const double* __restrict__ F, double* __restrict__ v) {
+    for (i64 e = i64(blockIdx.x) * blockDim.x + threadIdx.x; e < n; e += i64(gridDim.x) * blockDim.x) v[e] = F[src[e]];
 }
 
 __global__ void k_pack_rows(i64 n, const i32* __restrict__ row, const i64* __restrict__ diag, const double* __restrict__ F,
-                            const double* __restrict__ s, double* __restrict__ dinv64, float* __restrict__ dinv32,
-                            double* __restrict__ s64, float* __restrict__ s32) {
+                            const double* __restrict__ s, double* __restrict__ dinv, double* __restrict__ scale) {
     for (i64 t = i64(blockIdx.x) * blockDim.x + threadIdx.x; t < n; t += i64(gridDim.x) * blockDim.x) {
         const i32 k = row[t];
-        const double d = 1.0 / F[diag[k]];
-        dinv64[t] = d;
-        dinv32[t] = float(d);
-        s64[t] = s[k];
-        s32[t] = float(s[k]);
+        dinv[t] = 1.0 / F[diag[k]];
+        scale[t] = s[k];
     }
 }
 
@@ -858,7 +597,11 @@ __global__ void k_zero(i64 n, X* __restrict__ x) {
     for (i64 i = i64(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += i64(gridDim.x) * blockDim.x) x[i] = X(0);
 }
 
+unsigned grid_stride_blocks(i64 n) { return unsigned(std::min<i64>(std::max<i64>((n + 255) / 256, 1), 4096)); }
+
 }  // namespace nlf
+
+#include "nlf_sweep.inl"
 
 // ---- preconditioner object ---------------------------------------------------------------------
 struct nlf_precond_s {
@@ -873,43 +616,27 @@ struct nlf_precond_s {
     nlf::DevBuf<float> invd32;
     // ILLT
     nlf::DevBuf<nlf::i64> outer, diag, tpos;
-    nlf::DevBuf<nlf::i32> cols, fw_rows, fw_ptr, bw_rows, bw_ptr;
+    nlf::DevBuf<nlf::i32> cols, fw_rows, fw_ptr;
     int fw_levels = 0, bw_levels = 0;
     // independent diagonal blocks (more than one: fw_rows / fw_ptr hold each block's levels in turn,
     // and the factorisation runs a workgroup per block)
     int blocks = 1;
     nlf::DevBuf<nlf::SweepBlock> fw_blocks;
-    nlf::DevBuf<double> F, scale, work;
-    nlf::DevBuf<float> work32;
-    struct Sweep {
+    nlf::DevBuf<double> F, scale;
+    // the chunked sweeps with their value buffers (by record) and tickets
+    bool chunked = false;
+    nlf::Sweep sw_fw, sw_bw;
+    nlf::DevBuf<double> fw_lvl, bw_lvl;
+    nlf::DevBuf<nlf::i32> ticket;
+    // the packed sweeps (one workgroup)
+    struct Packed {
         int levels = 0, K = 0, W = 0;
         nlf::DevBuf<nlf::i32> lptr, row, off, dep;
         nlf::DevBuf<double> val, dinv, scale;
-        nlf::DevBuf<float> val32, dinv32, scale32;
-        nlf::PackedSweep<double> f64() const {
-            return {levels, K, W, lptr.p, row.p, off.p, dep.p, val.p, dinv.p, scale.p};
-        }
-        nlf::PackedSweep<float> f32() const {
-            return {levels, K, W, lptr.p, row.p, off.p, dep.p, val32.p, dinv32.p, scale32.p};
-        }
+        nlf::PackedSweep args() const { return {levels, K, W, lptr.p, row.p, off.p, dep.p, val.p, dinv.p, scale.p}; }
     } fw, bw;
     int solve_threads = 64;
-    struct Ell {
-        int levels = 0, K = 0, W = 0, WE = 0, threads = 64;
-        nlf::i64 rows = 0;
-        nlf::DevBuf<nlf::i32> lptr, row, dep;
-        nlf::DevBuf<double> val, dinv, scale;
-        nlf::DevBuf<float> val32, dinv32, scale32;
-        // blocks > 1: independent diagonal blocks, one sweep each (one workgroup per block): bdesc
-        // holds each block's levels, window depth and first level offset; levels and K above are
-        // the largest
-        int blocks = 1;
-        nlf::DevBuf<nlf::SweepBlock> bdesc;
-        template<class X> nlf::EllSweep<X> get() const;
-    } efw, ebw;
-    bool ell = false;
-    nlf::DevBuf<double> rhs_lvl, y_lvl, y1, y2;
-    nlf::DevBuf<float> rhs_lvl32, y_lvl32, y1_32, y2_32;
+    nlf::DevBuf<double> work;
     // learned (set by nlf_learned.hip)
     void* learned = nullptr;
     void (*learned_destroy)(void*) = nullptr;
@@ -918,22 +645,11 @@ struct nlf_precond_s {
     }
 };
 
-template<> nlf::EllSweep<double> nlf_precond_s::Ell::get<double>() const {
-    return {levels, K, W, lptr.p, row.p, dep.p, val.p, dinv.p};
-}
-template<> nlf::EllSweep<float> nlf_precond_s::Ell::get<float>() const {
-    return {levels, K, W, lptr.p, row.p, dep.p, val32.p, dinv32.p};
-}
-
 namespace nlf {
 
 static LevelArgs fw_args(const nlf_precond_s* P) {
     return LevelArgs{P->rows, P->fw_levels, P->outer.p, P->cols.p, P->diag.p, P->tpos.p, P->fw_rows.p, P->fw_ptr.p};
 }
-static LevelArgs bw_args(const nlf_precond_s* P) {
-    return LevelArgs{P->rows, P->bw_levels, P->outer.p, P->cols.p, P->diag.p, P->tpos.p, P->bw_rows.p, P->bw_ptr.p};
-}
-
 // Level sets of the lower (forward) and upper (backward) dependency DAGs of a symmetric pattern.
 static void level_sets(const std::vector<i64>& outer, const std::vector<i32>& cols, const std::vector<i64>& diag,
                        std::vector<i32>& fr, std::vector<i32>& fp, std::vector<i32>& br, std::vector<i32>& bp) {
@@ -967,8 +683,6 @@ static void level_sets(const std::vector<i64>& outer, const std::vector<i32>& co
     bucket(nl, br, bp, false);
 }
 
-unsigned grid_stride_blocks(i64 n) { return unsigned(std::min<i64>(std::max<i64>((n + 255) / 256, 1), 4096)); }
-
 constexpr size_t IC_WINDOW_BYTES = 64 * 1024;
 
 // Builds one packed sweep: records in level order, entries (lower part for the forward sweep,
@@ -976,7 +690,7 @@ constexpr size_t IC_WINDOW_BYTES = 64 * 1024;
 // device from the factor by source position.
 static void build_sweep(const std::vector<i64>& outer, const std::vector<i32>& cols, const std::vector<i64>& diag,
                         const std::vector<i32>& lrows, const std::vector<i32>& lptr, bool forward, const double* F,
-                        const double* scale, const i64* d_diag, nlf_precond_s::Sweep& sw, hipStream_t s) {
+                        const double* scale, const i64* d_diag, nlf_precond_s::Packed& sw, hipStream_t s) {
     const i64 n = i64(diag.size());
     const int levels = int(lptr.size()) - 1;
     std::vector<i32> level_of(n), pos_of(n);
@@ -1019,106 +733,15 @@ static void build_sweep(const std::vector<i64>& outer, const std::vector<i32>& c
     DevBuf<i64> d_src;
     upload(d_src, src.data(), std::max<size_t>(src.size(), 1), s);
     const size_t ne = std::max<size_t>(src.size(), 1);
-    sw.val.alloc(ne); sw.val32.alloc(ne);
-    sw.dinv.alloc(size_t(n)); sw.dinv32.alloc(size_t(n)); sw.scale.alloc(size_t(n)); sw.scale32.alloc(size_t(n));
+    sw.val.alloc(ne);
+    sw.dinv.alloc(size_t(n)); sw.scale.alloc(size_t(n));
     if (!src.empty())
         hipLaunchKernelGGL(k_pack_entries, dim3(grid_stride_blocks(i64(src.size()))), dim3(256), 0, s, i64(src.size()),
-                           d_src.p, F, sw.val.p, sw.val32.p);
+                           d_src.p, F, sw.val.p);
     hipLaunchKernelGGL(k_pack_rows, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, sw.row.p, d_diag, F, scale,
-                       sw.dinv.p, sw.dinv32.p, sw.scale.p, sw.scale32.p);
+                       sw.dinv.p, sw.scale.p);
     NLF_HIP(hipGetLastError());
     NLF_HIP(hipStreamSynchronize(s));
-}
-
-// ELL sweep for the fast kernel; false when a level is wider than one workgroup or rows have too
-// many entries (the generic packed sweep is used then).
-static bool build_ell(const std::vector<i64>& outer, const std::vector<i32>& cols, const std::vector<i64>& diag,
-                      const std::vector<i32>& lrows, const std::vector<i32>& level_ptr, bool forward, const double* F,
-                      const double* scale, const i64* d_diag, nlf_precond_s::Ell& el, hipStream_t s) {
-    const i64 n = i64(diag.size());
-    // Levels wider than the sweep's compute width are split into consecutive parts: the records of a
-    // level are independent, so any split keeps the dependency order.  The widest level is often
-    // level 0, the rows with no dependency at all (first-kind rows among them), several times wider
-    // than the rest.  The width is the one of the two prefetching sweeps that needs fewer levels,
-    // preferring the narrower (deeper prefetch) unless it needs over 25% more.
-    std::vector<i32> lptr(1, 0);
-    {
-        i64 c_small = 0, c_large = 0;
-        for (size_t L = 0; L + 1 < level_ptr.size(); ++L) {
-            const i64 w = level_ptr[L + 1] - level_ptr[L];
-            c_small += (w + SWEEP_CT_SMALL - 1) / SWEEP_CT_SMALL;
-            c_large += (w + SWEEP_CT_LARGE - 1) / SWEEP_CT_LARGE;
-        }
-        const i32 cap = 4 * c_small <= 5 * c_large ? SWEEP_CT_SMALL : SWEEP_CT_LARGE;
-        for (size_t L = 0; L + 1 < level_ptr.size(); ++L) {
-            for (i32 x = level_ptr[L] + cap; x < level_ptr[L + 1]; x += cap) lptr.push_back(x);
-            lptr.push_back(level_ptr[L + 1]);
-        }
-    }
-    const int levels = int(lptr.size()) - 1;
-    std::vector<i32> level_of(n), pos_of(n);
-    int W = 1, WEmax = 0;
-    for (int L = 0; L < levels; ++L) {
-        W = std::max(W, lptr[L + 1] - lptr[L]);
-        for (i32 t = lptr[L]; t < lptr[L + 1]; ++t) { level_of[lrows[t]] = L; pos_of[lrows[t]] = t - lptr[L]; }
-    }
-    int K = 1;
-    for (i64 t = 0; t < n; ++t) {
-        const i32 k = lrows[t];
-        const i64 b = forward ? outer[k] : diag[k] + 1, e = forward ? diag[k] : outer[k + 1];
-        WEmax = std::max(WEmax, int(e - b));
-        for (i64 p = b; p < e; ++p) K = std::max(K, level_of[k] - level_of[cols[p]]);
-    }
-    K += 1;
-    int WE = 4;
-    while (WE < WEmax) WE *= 2;
-    if (W > LEVEL_THREADS || WE > 32) return false;
-    // one thread per record of the widest level; the window's slot blocks are one workgroup wide,
-    // so that the sweep's lanes past a level's width have slots of their own to write
-    const int threads = std::min(LEVEL_THREADS, std::max(64, (W + 63) / 64 * 64));
-    W = threads;
-    const bool window = size_t(K) * size_t(W) * sizeof(double) <= IC_WINDOW_BYTES;
-    std::vector<i32> dep(size_t(WE) * n);
-    std::vector<i64> src(size_t(WE) * n, -1);
-    for (int L = 0; L < levels; ++L) {
-        const i32 b = lptr[L], cnt = lptr[L + 1] - b;
-        for (i32 t = 0; t < cnt; ++t) {
-            const i32 k = lrows[b + t];
-            const i64 pb = forward ? outer[k] : diag[k] + 1, pe = forward ? diag[k] : outer[k + 1];
-            for (int j = 0; j < WE; ++j) {
-                const size_t e = size_t(WE) * size_t(b + t) + size_t(j);
-                if (pb + j < pe) {
-                    const i32 i = cols[pb + j];
-                    dep[e] = window ? (level_of[i] % K) * W + pos_of[i] : -(i + 1);
-                    src[e] = pb + j;
-                } else {
-                    dep[e] = window ? 0 : -1;       // value 0 times a finite slot
-                }
-            }
-        }
-    }
-    el.levels = levels;
-    el.K = window ? K : 0;
-    el.W = W;
-    el.WE = WE;
-    el.threads = threads;
-    el.rows = n;
-    el.blocks = 1;                                   // one sweep (a blocked layout tried before is replaced)
-    el.bdesc.release();
-    upload(el.lptr, lptr.data(), lptr.size(), s);
-    upload(el.row, lrows.data(), lrows.size(), s);
-    upload(el.dep, dep.data(), dep.size(), s);
-    DevBuf<i64> d_src;
-    upload(d_src, src.data(), src.size(), s);
-    el.val.alloc(src.size()); el.val32.alloc(src.size());
-    hipLaunchKernelGGL(k_pack_ell, dim3(grid_stride_blocks(i64(src.size()))), dim3(256), 0, s, i64(src.size()), d_src.p,
-                       F, el.val.p, el.val32.p);
-    el.dinv.alloc(size_t(n)); el.dinv32.alloc(size_t(n)); el.scale.alloc(size_t(n)); el.scale32.alloc(size_t(n));
-    hipLaunchKernelGGL(k_pack_rows, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, el.row.p, d_diag, F, scale, el.dinv.p,
-                       el.dinv32.p, el.scale.p, el.scale32.p);
-    NLF_HIP(hipGetLastError());
-    NLF_HIP(hipStreamSynchronize(s));
-    return true;
 }
 
 // Contiguous row ranges with no entry between them: the diagonal blocks of a block-diagonal pattern
@@ -1180,221 +803,24 @@ static BlockLevels block_levels(const std::vector<i32>& lrows, const std::vector
     return bl;
 }
 
-// The ELL layout for a factor made of independent diagonal blocks: every block gets its own levels
-// and its own sweep, one workgroup each, so that the blocks' levels run side by side instead of one
-// after another.  Records are block after block; all blocks share the compute width W (their widest
-// split level) and the record arrays, each has its level offsets and window depth.  Each record's
-// arithmetic is the single-sweep one, so the results are the same bits.
-static bool build_ell_blocks(const std::vector<i64>& outer, const std::vector<i32>& cols, const std::vector<i64>& diag,
-                             const BlockLevels& bl, bool forward, const double* F, const double* scale, const i64* d_diag,
-                             nlf_precond_s::Ell& el, hipStream_t s) {
-    const i64 n = i64(diag.size());
-    const int B = int(bl.levels.size());
-    for (int b = 0; b < B; ++b)
-        if (bl.levels[size_t(b)] == 0) return false;                // an empty block
-    // the split width, as in build_ell, over every block's levels
-    i32 cap;
-    {
-        i64 c_small = 0, c_large = 0;
-        for (int b = 0; b < B; ++b)
-            for (i64 L = bl.seg[size_t(b)]; L + 1 < bl.seg[size_t(b) + 1]; ++L) {
-                const i64 w = bl.ptr[size_t(L) + 1] - bl.ptr[size_t(L)];
-                c_small += (w + SWEEP_CT_SMALL - 1) / SWEEP_CT_SMALL;
-                c_large += (w + SWEEP_CT_LARGE - 1) / SWEEP_CT_LARGE;
-            }
-        cap = 4 * c_small <= 5 * c_large ? SWEEP_CT_SMALL : SWEEP_CT_LARGE;
-    }
-    // split levels; records keep the block-major order of bl.rows
-    std::vector<i32> lptr;
-    std::vector<i64> seg(static_cast<size_t>(B) + 1, 0);
-    std::vector<int> blevels(static_cast<size_t>(B), 0);
-    std::vector<i32> level_of(static_cast<size_t>(n)), pos_of(static_cast<size_t>(n));
-    int W = 1;
-    for (int b = 0; b < B; ++b) {
-        seg[size_t(b)] = i64(lptr.size());
-        lptr.push_back(bl.ptr[size_t(bl.seg[size_t(b)])]);
-        int lv = 0;
-        for (i64 L = bl.seg[size_t(b)]; L + 1 < bl.seg[size_t(b) + 1]; ++L) {
-            const i32 end = bl.ptr[size_t(L) + 1];
-            for (i32 x = bl.ptr[size_t(L)]; x < end; x += cap) {
-                const i32 y = std::min(x + cap, end);
-                for (i32 t = x; t < y; ++t) {
-                    level_of[size_t(bl.rows[size_t(t)])] = lv;
-                    pos_of[size_t(bl.rows[size_t(t)])] = t - x;
-                }
-                W = std::max(W, y - x);
-                lptr.push_back(y);
-                ++lv;
-            }
-        }
-        blevels[size_t(b)] = lv;
-    }
-    seg[size_t(B)] = i64(lptr.size());
-    int K = 1, WEmax = 0;
-    std::vector<int> bK(static_cast<size_t>(B), 1);
-    for (i64 t = 0; t < n; ++t) {
-        const i32 k = bl.rows[size_t(t)];
-        const int b = bl.blk[size_t(k)];
-        const i64 pb = forward ? outer[k] : diag[k] + 1, pe = forward ? diag[k] : outer[k + 1];
-        WEmax = std::max(WEmax, int(pe - pb));
-        for (i64 p = pb; p < pe; ++p) {
-            if (bl.blk[size_t(cols[p])] != b) return false;         // not block diagonal
-            bK[size_t(b)] = std::max(bK[size_t(b)], level_of[size_t(k)] - level_of[size_t(cols[p])] + 1);
-        }
-    }
-    for (int b = 0; b < B; ++b) K = std::max(K, bK[size_t(b)]);
-    int WE = 4;
-    while (WE < WEmax) WE *= 2;
-    if (W > LEVEL_THREADS || WE > 32) return false;
-    const int threads = std::min(LEVEL_THREADS, std::max(64, (W + 63) / 64 * 64));
-    W = threads;
-    const bool window = size_t(K) * size_t(W) * sizeof(double) <= IC_WINDOW_BYTES;
-    std::vector<i32> dep(size_t(WE) * size_t(n));
-    std::vector<i64> src(size_t(WE) * size_t(n), -1);
-    for (i64 t = 0; t < n; ++t) {
-        const i32 k = bl.rows[size_t(t)];
-        const int Kb = bK[size_t(bl.blk[size_t(k)])];
-        const i64 pb = forward ? outer[k] : diag[k] + 1, pe = forward ? diag[k] : outer[k + 1];
-        for (int j = 0; j < WE; ++j) {
-            const size_t e = size_t(WE) * size_t(t) + size_t(j);
-            if (pb + j < pe) {
-                const i32 i = cols[pb + j];
-                dep[e] = window ? (level_of[size_t(i)] % Kb) * W + pos_of[size_t(i)] : -(i + 1);
-                src[e] = pb + j;
-            } else {
-                dep[e] = window ? 0 : -1;           // value 0 times a finite slot
-            }
-        }
-    }
-    el.levels = *std::max_element(blevels.begin(), blevels.end());
-    el.K = window ? K : 0;
-    el.W = W;
-    el.WE = WE;
-    el.threads = threads;
-    el.rows = n;
-    el.blocks = B;
-    upload(el.lptr, lptr.data(), lptr.size(), s);
-    upload(el.row, bl.rows.data(), bl.rows.size(), s);
-    upload(el.dep, dep.data(), dep.size(), s);
-    DevBuf<i64> d_src;
-    upload(d_src, src.data(), src.size(), s);
-    el.val.alloc(src.size()); el.val32.alloc(src.size());
-    hipLaunchKernelGGL(k_pack_ell, dim3(grid_stride_blocks(i64(src.size()))), dim3(256), 0, s, i64(src.size()), d_src.p,
-                       F, el.val.p, el.val32.p);
-    el.dinv.alloc(size_t(n)); el.dinv32.alloc(size_t(n)); el.scale.alloc(size_t(n)); el.scale32.alloc(size_t(n));
-    hipLaunchKernelGGL(k_pack_rows, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, el.row.p, d_diag, F, scale, el.dinv.p,
-                       el.dinv32.p, el.scale.p, el.scale32.p);
-    NLF_HIP(hipGetLastError());
-    std::vector<SweepBlock> bd(static_cast<size_t>(B));
-    for (int b = 0; b < B; ++b)
-        bd[size_t(b)] = SweepBlock{blevels[size_t(b)], window ? bK[size_t(b)] : 0, i32(seg[size_t(b)]), 0};
-    upload(el.bdesc, bd.data(), bd.size(), s);
-    NLF_HIP(hipStreamSynchronize(s));
-    return true;
-}
-
-template<class X>
-const X* ell_scale(const nlf_precond_s::Ell& e);
-template<> const double* ell_scale<double>(const nlf_precond_s::Ell& e) { return e.scale.p; }
-template<> const float* ell_scale<float>(const nlf_precond_s::Ell& e) { return e.scale32.p; }
-
-// LDS bytes of the dependency window, and whether the prefetching kernel takes the sweep (it needs
-// the window and the level offsets in LDS and at most SWEEP_CT_LARGE compute lanes).
-static size_t ell_window_bytes(const nlf_precond_s::Ell& e, size_t xsize) {
-    return (size_t(std::max(e.K * e.W, 1)) * xsize + 15) & ~size_t(15);
-}
-static bool ell_prefetching(const nlf_precond_s::Ell& e, size_t xsize) {
-    return e.K != 0 && ell_window_bytes(e, xsize) + size_t(e.levels + 1) * sizeof(i32) <= SWEEP_LDS_BYTES &&
-           e.threads <= SWEEP_CT_LARGE;
-}
-
-template<class X>
-void ell_sweep(const nlf_precond_s::Ell& e, const X* rhs, X* lvl, X* out, X* out2, const X* scale2, const CGState* st,
-               hipStream_t s) {
-    // LDS: the dependency window, then the level offsets; the prefetching kernel needs both there
-    const size_t win = ell_window_bytes(e, sizeof(X));
-    const size_t offs = size_t(e.levels + 1) * sizeof(i32);
-    const EllSweep<X> a = e.template get<X>();
-    const SweepBlock* blk = e.blocks > 1 ? e.bdesc.p : nullptr;
-    const dim3 g(unsigned(e.blocks));
-    if (e.levels == 0) return;
-    if (!ell_prefetching(e, sizeof(X))) {
-        const size_t lds = e.K ? win : 16;
-        const dim3 b(unsigned(e.threads));
-        switch (e.WE) {
-            case 4: hipLaunchKernelGGL((k_ic_sweep_generic<X, 4>), g, b, lds, s, a, blk, rhs, out, out2, scale2, st); break;
-            case 8: hipLaunchKernelGGL((k_ic_sweep_generic<X, 8>), g, b, lds, s, a, blk, rhs, out, out2, scale2, st); break;
-            case 16: hipLaunchKernelGGL((k_ic_sweep_generic<X, 16>), g, b, lds, s, a, blk, rhs, out, out2, scale2, st); break;
-            default: hipLaunchKernelGGL((k_ic_sweep_generic<X, 32>), g, b, lds, s, a, blk, rhs, out, out2, scale2, st); break;
-        }
-        return;
-    }
-    const size_t lds = win + offs;
-    if (e.threads <= SWEEP_CT_SMALL) {
-        constexpr int CT = SWEEP_CT_SMALL, SW = SWEEP_SW_SMALL;
-        const dim3 b(unsigned(e.threads + 64 * SW));
-        switch (e.WE) {
-            case 4: hipLaunchKernelGGL((k_ic_sweep<X, 4, CT, SW>), g, b, lds, s, a, blk, rhs, lvl, st); break;
-            case 8: hipLaunchKernelGGL((k_ic_sweep<X, 8, CT, SW>), g, b, lds, s, a, blk, rhs, lvl, st); break;
-            case 16: hipLaunchKernelGGL((k_ic_sweep<X, 16, CT, SW>), g, b, lds, s, a, blk, rhs, lvl, st); break;
-            default: hipLaunchKernelGGL((k_ic_sweep<X, 32, CT, SW>), g, b, lds, s, a, blk, rhs, lvl, st); break;
-        }
-    } else {
-        constexpr int CT = SWEEP_CT_LARGE, SW = SWEEP_SW_LARGE;
-        const dim3 b(unsigned(e.threads + 64 * SW));
-        switch (e.WE) {
-            case 4: hipLaunchKernelGGL((k_ic_sweep<X, 4, CT, SW>), g, b, lds, s, a, blk, rhs, lvl, st); break;
-            case 8: hipLaunchKernelGGL((k_ic_sweep<X, 8, CT, SW>), g, b, lds, s, a, blk, rhs, lvl, st); break;
-            case 16: hipLaunchKernelGGL((k_ic_sweep<X, 16, CT, SW>), g, b, lds, s, a, blk, rhs, lvl, st); break;
-            default: hipLaunchKernelGGL((k_ic_sweep<X, 32, CT, SW>), g, b, lds, s, a, blk, rhs, lvl, st); break;
-        }
-    }
-    const i64 n = i64(e.rows);
-    hipLaunchKernelGGL(k_sweep_scatter<X>, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, e.row.p, (const X*)lvl,
-                       scale2, out, out2, st);
-}
-
-// z = S U^-1 U^-T S r through the ELL sweeps: gather, forward sweep, gather, backward sweep.
-template<class X>
-void ell_apply(const nlf_precond_s* P, i64 n, const X* r, X* z, X* rhs, X* lvl, X* y1, X* y2, const CGState* st,
-               hipStream_t s) {
-    const unsigned g = grid_stride_blocks(n);
-    hipLaunchKernelGGL(k_sweep_gather<X>, dim3(g), dim3(256), 0, s, n, P->efw.row.p, ell_scale<X>(P->efw), r, rhs, y1, st);
-    ell_sweep<X>(P->efw, rhs, lvl, y1, (X*)nullptr, (const X*)nullptr, st, s);
-    hipLaunchKernelGGL(k_sweep_gather<X>, dim3(g), dim3(256), 0, s, n, P->ebw.row.p, (const X*)nullptr, y1, rhs, y2, st);
-    ell_sweep<X>(P->ebw, rhs, lvl, y2, z, ell_scale<X>(P->ebw), st, s);
-}
-
-// Applies the preconditioner z = M^-1 r on the stream (FP64 or FP32 vectors).
-template<class X>
-void precond_apply(const nlf_precond_s* P, i64 n, const X* r, X* z, const CGState* st, hipStream_t s);
-
-template<>
-void precond_apply<double>(const nlf_precond_s* P, i64 n, const double* r, double* z, const CGState* st, hipStream_t s) {
+// Applies the preconditioner z = M^-1 r on the stream.  With `partial`, an ILLT also writes the partial
+// sums of r.z in k_dot's blocks (`blocks` of them); returns whether it did.
+bool precond_apply(const nlf_precond_s* P, i64 n, const double* r, double* z, const CGState* st, hipStream_t s,
+                   double* partial = nullptr, unsigned blocks = 0) {
     if (P && P->kind == NLF_PRECOND_JACOBI)
         hipLaunchKernelGGL(k_scale<double>, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, P->invd.p, r, z);
-    else if (P && P->kind == NLF_PRECOND_ILLT && P->ell)
-        ell_apply<double>(P, n, r, z, P->rhs_lvl.p, P->y_lvl.p, P->y1.p, P->y2.p, st, s);
-    else if (P && P->kind == NLF_PRECOND_ILLT) {
+    else if (P && P->kind == NLF_PRECOND_ILLT && P->chunked) {
+        launch_sweep(P->sw_fw, r, P->fw_lvl.p, P->ticket.p, st, s);
+        launch_sweep(P->sw_bw, P->fw_lvl.p, P->bw_lvl.p, P->ticket.p + 1, st, s);
+        hipLaunchKernelGGL(k_sweep_finish, dim3(partial ? blocks : grid_stride_blocks(n)), dim3(SPMV_THREADS), 0, s, n,
+                           P->sw_bw.pos.p, P->scale.p, P->fw_lvl.p, P->bw_lvl.p, P->ticket.p, r, z, partial, st);
+        return partial != nullptr;
+    } else if (P && P->kind == NLF_PRECOND_ILLT) {
         const size_t lds = size_t(std::max(P->fw.K * P->fw.W, P->bw.K * P->bw.W)) * sizeof(double);
-        hipLaunchKernelGGL((k_ic_solve<double>), dim3(1), dim3(P->solve_threads), lds, s, P->fw.f64(), P->bw.f64(), r,
-                           P->work.p, z, st);
+        hipLaunchKernelGGL(k_ic_solve, dim3(1), dim3(P->solve_threads), lds, s, P->fw.args(), P->bw.args(), r, P->work.p, z, st);
     } else
         NLF_HIP(hipMemcpyAsync(z, r, size_t(n) * sizeof(double), hipMemcpyDeviceToDevice, s));
-}
-
-template<>
-void precond_apply<float>(const nlf_precond_s* P, i64 n, const float* r, float* z, const CGState* st, hipStream_t s) {
-    if (P && P->kind == NLF_PRECOND_JACOBI)
-        hipLaunchKernelGGL(k_scale<float>, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, P->invd32.p, r, z);
-    else if (P && P->kind == NLF_PRECOND_ILLT && P->ell)
-        ell_apply<float>(P, n, r, z, P->rhs_lvl32.p, P->y_lvl32.p, P->y1_32.p, P->y2_32.p, st, s);
-    else if (P && P->kind == NLF_PRECOND_ILLT) {
-        const size_t lds = size_t(std::max(P->fw.K * P->fw.W, P->bw.K * P->bw.W)) * sizeof(float);
-        hipLaunchKernelGGL((k_ic_solve<float>), dim3(1), dim3(P->solve_threads), lds, s, P->fw.f32(), P->bw.f32(), r,
-                           P->work32.p, z, st);
-    } else
-        NLF_HIP(hipMemcpyAsync(z, r, size_t(n) * sizeof(float), hipMemcpyDeviceToDevice, s));
+    return false;
 }
 
 // Lanes per row: the smallest power of two (4..64) giving each lane at most 16 nonzeros for the
@@ -1694,7 +1120,7 @@ struct CG {
                            r, part1, part2);
         const int nb_res = int(spmv_blocks(64, n));
         NLF_HIP(hipMemcpyAsync(pbb, part2, size_t(nb_res) * sizeof(double), hipMemcpyDeviceToDevice, s));
-        precond_apply<X>(P, n, r, p, nullptr, s);
+        precond_apply(P, n, r, p, nullptr, s);
         hipLaunchKernelGGL(k_dot<X>, dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, r, p, part1, (const CGState*)nullptr);
         // pad partial arrays: k_init_state sums vblocks of r.z and nb_res of b.b (cleared by a kernel,
         // not a memset, so that the sequence may be captured)
@@ -1741,7 +1167,7 @@ struct CG {
         // r = M^-1-preconditioned restart data from the FP64 residual: r32 = r64, z = M r32, rz = r32.z
         auto load_residual = [&](bool first) {
             hipLaunchKernelGGL((k_convert<double, X>), dim3(vblocks), dim3(256), 0, s, n, r64.p, r);
-            precond_apply<X>(P, n, r, z, nullptr, s);
+            precond_apply(P, n, r, z, nullptr, s);
             if (first) NLF_HIP(hipMemcpyAsync(p, z, size_t(n) * sizeof(X), hipMemcpyDeviceToDevice, s));
             hipLaunchKernelGGL(k_dot<X>, dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, r, z, part1,
                                (const CGState*)nullptr);
@@ -1812,9 +1238,9 @@ struct CG {
             hipLaunchKernelGGL((k_update_xr<X, false, false>), dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, x, r, p, z,
                                (X*)nullptr, (const X*)nullptr, part2, st);
             if (sample) timer.start(1, s);
-            precond_apply<X>(P, n, r, z, st, s);
+            const bool dotted = precond_apply(P, n, r, z, st, s, part2, vblocks);
             if (sample) timer.stop(1, s);
-            hipLaunchKernelGGL(k_dot<X>, dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, r, z, part2, st);
+            if (!dotted) hipLaunchKernelGGL(k_dot<X>, dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, r, z, part2, st);
         }
         hipLaunchKernelGGL(k_beta, dim3(1), dim3(1024), 0, s, part2, int(vblocks), st);
         hipLaunchKernelGGL(k_update_p<X>, dim3(vblocks), dim3(256), 0, s, n, p, z, st);
@@ -1991,14 +1417,13 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
             level_sets(outer, cols, diag, fr, fp, br, bp);
             P->fw_levels = int(fp.size()) - 1;
             P->bw_levels = int(bp.size()) - 1;
-            // a block-diagonal matrix (a batch of independent instances) factors and sweeps block by
-            // block, the blocks side by side: one workgroup each instead of one for all
+            // a block-diagonal matrix (a batch of independent instances) factors block by block, the
+            // blocks side by side: one workgroup each instead of one for all
             const std::vector<i64> bounds = independent_blocks(outer, cols, std::max<i64>(1024, n / 2048));
             P->blocks = int(bounds.size()) - 1;
-            BlockLevels bfw, bbw;
+            BlockLevels bfw;
             if (P->blocks > 1) {
                 bfw = block_levels(fr, fp, bounds);
-                bbw = block_levels(br, bp, bounds);
                 std::vector<SweepBlock> bd(static_cast<size_t>(P->blocks));
                 for (int b = 0; b < P->blocks; ++b)
                     bd[size_t(b)] = SweepBlock{bfw.levels[size_t(b)], 0, i32(bfw.seg[size_t(b)]), 0};
@@ -2012,13 +1437,9 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
             upload(P->outer, outer.data(), outer.size(), s);
             upload(P->diag, diag.data(), diag.size(), s);
             upload(P->cols, cols.data(), cols.size(), s);
-            upload(P->bw_rows, br.data(), br.size(), s);
-            upload(P->bw_ptr, bp.data(), bp.size(), s);
             P->tpos.alloc(cols.size());
             hipLaunchKernelGGL(k_transpose_pos, dim3(blocks_for(n, 4)), dim3(256), 0, s, n, P->outer.p, P->cols.p, P->tpos.p);
             P->scale.alloc(size_t(n));
-            P->work.alloc(size_t(n));
-            P->work32.alloc(size_t(n));
             P->F.alloc(cols.size());
             DevBuf<float> scale32{size_t(n)};
             hipLaunchKernelGGL(k_scale_from_diag, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, P->diag.p, a->val.p,
@@ -2038,23 +1459,25 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
                 if (!f) { P->ok = true; P->shift = shift; break; }
                 shift = shift == 0.0 ? 1e-3 : 2 * shift;
             }
-            P->ell = P->blocks > 1 &&
-                     build_ell_blocks(outer, cols, diag, bfw, true, P->F.p, P->scale.p, P->diag.p, P->efw, s) &&
-                     build_ell_blocks(outer, cols, diag, bbw, false, P->F.p, P->scale.p, P->diag.p, P->ebw, s);
-            if (!P->ell)
-                P->ell = build_ell(outer, cols, diag, fr, fp, true, P->F.p, P->scale.p, P->diag.p, P->efw, s) &&
-                         build_ell(outer, cols, diag, br, bp, false, P->F.p, P->scale.p, P->diag.p, P->ebw, s);
-            // the packed sweeps (one workgroup, any level width) where the ELL layout does not apply
-            if (!P->ell) {
+            SweepPlan pf, pb;
+            P->chunked = plan_sweep(outer, cols, diag, fr, fp, bounds, true, pf) &&
+                         plan_sweep(outer, cols, diag, br, bp, bounds, false, pb);
+            if (P->chunked) {
+                upload_sweep(pf, true, P->outer.p, P->diag.p, P->F.p, P->scale.p, nullptr, P->sw_fw, s);
+                upload_sweep(pb, false, P->outer.p, P->diag.p, P->F.p, P->scale.p, P->sw_fw.pos.p, P->sw_bw, s);
+                P->fw_lvl.alloc(size_t(n));
+                P->bw_lvl.alloc(size_t(n));
+                P->ticket.alloc(2);
+                hipLaunchKernelGGL(k_sweep_empty, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, P->fw_lvl.p, P->bw_lvl.p,
+                                   P->ticket.p);
+                NLF_HIP(hipGetLastError());
+            } else {
+                // rows with more dependencies than the chunked sweeps take
                 build_sweep(outer, cols, diag, fr, fp, true, P->F.p, P->scale.p, P->diag.p, P->fw, s);
                 build_sweep(outer, cols, diag, br, bp, false, P->F.p, P->scale.p, P->diag.p, P->bw, s);
                 const int widest = std::max(P->fw.W, P->bw.W);
                 P->solve_threads = std::min(LEVEL_THREADS, std::max(64, (widest + 63) / 64 * 64));
-            }
-            if (P->ell) {
-                P->rhs_lvl.alloc(size_t(n)); P->y_lvl.alloc(size_t(n)); P->y1.alloc(size_t(n)); P->y2.alloc(size_t(n));
-                P->rhs_lvl32.alloc(size_t(n)); P->y_lvl32.alloc(size_t(n)); P->y1_32.alloc(size_t(n));
-                P->y2_32.alloc(size_t(n));
+                P->work.alloc(size_t(n));
             }
         } else {
             throw Error(NLF_ERR_UNSUPPORTED, "use nlf_learned_precond_create for the learned preconditioner");
@@ -2087,13 +1510,13 @@ int nlf_precond_sweep_info(nlf_precond p, int32_t out[8]) {
     if (!p || !out) return NLF_ERR_ARGUMENT;
     for (int i = 0; i < 8; ++i) out[i] = 0;
     if (p->kind != NLF_PRECOND_ILLT) return NLF_ERR_ARGUMENT;
-    const nlf_precond_s::Ell* e[2] = {&p->efw, &p->ebw};
     for (int k = 0; k < 2; ++k) {
-        if (p->ell) {
-            out[4 * k] = e[k]->levels;
-            out[4 * k + 1] = e[k]->threads;
-            out[4 * k + 2] = e[k]->K;
-            out[4 * k + 3] = nlf::ell_prefetching(*e[k], sizeof(double)) ? 2 : 1;
+        if (p->chunked) {
+            const Sweep& w = k ? p->sw_bw : p->sw_fw;
+            out[4 * k] = w.levels;
+            out[4 * k + 1] = w.width;
+            out[4 * k + 2] = SWEEP_K;
+            out[4 * k + 3] = 2;
         } else {
             const auto& w = k ? p->bw : p->fw;
             out[4 * k] = w.levels;
@@ -2120,7 +1543,7 @@ int nlf_precond_apply(nlf_precond p, const double* r, double* z) {
             LearnedGraph& g = *learned_of(p);
             learned_apply<double>(g, g.w.p, r, z, p->ctx->stream);
         } else {
-            precond_apply<double>(p, p->rows, r, z, nullptr, p->ctx->stream);
+            precond_apply(p, p->rows, r, z, nullptr, p->ctx->stream);
         }
         NLF_HIP(hipGetLastError());
     });
