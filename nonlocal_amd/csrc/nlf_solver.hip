@@ -615,13 +615,8 @@ struct nlf_precond_s {
     nlf::DevBuf<double> invd;
     nlf::DevBuf<float> invd32;
     // ILLT
-    nlf::DevBuf<nlf::i64> outer, diag, tpos;
-    nlf::DevBuf<nlf::i32> cols, fw_rows, fw_ptr;
     int fw_levels = 0, bw_levels = 0;
-    // independent diagonal blocks (more than one: fw_rows / fw_ptr hold each block's levels in turn,
-    // and the factorisation runs a workgroup per block)
-    int blocks = 1;
-    nlf::DevBuf<nlf::SweepBlock> fw_blocks;
+    int blocks = 1;                      // independent diagonal blocks
     nlf::DevBuf<double> F, scale;
     // the chunked sweeps with their value buffers (by record) and tickets
     bool chunked = false;
@@ -647,9 +642,6 @@ struct nlf_precond_s {
 
 namespace nlf {
 
-static LevelArgs fw_args(const nlf_precond_s* P) {
-    return LevelArgs{P->rows, P->fw_levels, P->outer.p, P->cols.p, P->diag.p, P->tpos.p, P->fw_rows.p, P->fw_ptr.p};
-}
 // Level sets of the lower (forward) and upper (backward) dependency DAGs of a symmetric pattern.
 static void level_sets(const std::vector<i64>& outer, const std::vector<i32>& cols, const std::vector<i64>& diag,
                        std::vector<i32>& fr, std::vector<i32>& fp, std::vector<i32>& br, std::vector<i32>& bp) {
@@ -1417,64 +1409,82 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
             level_sets(outer, cols, diag, fr, fp, br, bp);
             P->fw_levels = int(fp.size()) - 1;
             P->bw_levels = int(bp.size()) - 1;
-            // a block-diagonal matrix (a batch of independent instances) factors block by block, the
-            // blocks side by side: one workgroup each instead of one for all
+            // independent row blocks (a batch's instances) end a chunk, or get a workgroup of their own
             const std::vector<i64> bounds = independent_blocks(outer, cols, std::max<i64>(1024, n / 2048));
             P->blocks = int(bounds.size()) - 1;
-            BlockLevels bfw;
-            if (P->blocks > 1) {
-                bfw = block_levels(fr, fp, bounds);
-                std::vector<SweepBlock> bd(static_cast<size_t>(P->blocks));
-                for (int b = 0; b < P->blocks; ++b)
-                    bd[size_t(b)] = SweepBlock{bfw.levels[size_t(b)], 0, i32(bfw.seg[size_t(b)]), 0};
-                upload(P->fw_blocks, bd.data(), bd.size(), s);
-                upload(P->fw_rows, bfw.rows.data(), bfw.rows.size(), s);
-                upload(P->fw_ptr, bfw.ptr.data(), bfw.ptr.size(), s);
-            } else {
-                upload(P->fw_rows, fr.data(), fr.size(), s);
-                upload(P->fw_ptr, fp.data(), fp.size(), s);
-            }
-            upload(P->outer, outer.data(), outer.size(), s);
-            upload(P->diag, diag.data(), diag.size(), s);
-            upload(P->cols, cols.data(), cols.size(), s);
-            P->tpos.alloc(cols.size());
-            hipLaunchKernelGGL(k_transpose_pos, dim3(blocks_for(n, 4)), dim3(256), 0, s, n, P->outer.p, P->cols.p, P->tpos.p);
+            const i64 *d_outer = a->outer.p, *d_diag = a->diag.p;
+            const i32* d_cols = a->cols.p;
+            DevBuf<i64> tpos{cols.size()};
+            hipLaunchKernelGGL(k_transpose_pos, dim3(blocks_for(n, 4)), dim3(256), 0, s, n, d_outer, d_cols, tpos.p);
             P->scale.alloc(size_t(n));
             P->F.alloc(cols.size());
             DevBuf<float> scale32{size_t(n)};
-            hipLaunchKernelGGL(k_scale_from_diag, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, P->diag.p, a->val.p,
+            hipLaunchKernelGGL(k_scale_from_diag, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, d_diag, a->val.p,
                                P->scale.p, scale32.p);
             DevBuf<int> fail{1};
-            double shift = 0.0;
-            P->ok = false;
-            for (int attempt = 0; attempt < 40; ++attempt) {
-                NLF_HIP(hipMemsetAsync(fail.p, 0, sizeof(int), s));
-                hipLaunchKernelGGL(k_ic_init, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, P->outer.p, P->cols.p, P->diag.p,
-                                   a->val.p, P->scale.p, shift, P->F.p);
-                hipLaunchKernelGGL(k_ic_factor, dim3(unsigned(P->blocks)), dim3(LEVEL_THREADS), 0, s, fw_args(P.get()),
-                                   P->blocks > 1 ? P->fw_blocks.p : nullptr, P->F.p, fail.p);
-                NLF_HIP(hipGetLastError());
-                int f = 0;
-                download(&f, fail.p, 1, s);
-                if (!f) { P->ok = true; P->shift = shift; break; }
-                shift = shift == 0.0 ? 1e-3 : 2 * shift;
-            }
+            // factorisation with growing shift until no pivot fails
+            auto factor = [&](auto&& attempt_with) {
+                double shift = 0.0;
+                P->ok = false;
+                for (int attempt = 0; attempt < 40; ++attempt) {
+                    attempt_with(shift);
+                    NLF_HIP(hipGetLastError());
+                    int f = 0;
+                    download(&f, fail.p, 1, s);
+                    if (!f) { P->ok = true; P->shift = shift; break; }
+                    shift = shift == 0.0 ? 1e-3 : 2 * shift;
+                }
+            };
             SweepPlan pf, pb;
-            P->chunked = plan_sweep(outer, cols, diag, fr, fp, bounds, true, pf) &&
+            P->chunked = cols.size() < (size_t(1) << 31) && plan_sweep(outer, cols, diag, fr, fp, bounds, true, pf) &&
                          plan_sweep(outer, cols, diag, br, bp, bounds, false, pb);
             if (P->chunked) {
-                upload_sweep(pf, true, P->outer.p, P->diag.p, P->F.p, P->scale.p, nullptr, P->sw_fw, s);
-                upload_sweep(pb, false, P->outer.p, P->diag.p, P->F.p, P->scale.p, P->sw_fw.pos.p, P->sw_bw, s);
+                upload_plan(pf, P->sw_fw, s);
+                upload_plan(pb, P->sw_bw, s);
+                P->ticket.alloc(2);
+                {
+                    DevBuf<i32> list;
+                    ic_lists(P->sw_fw, n, d_outer, d_cols, d_diag, list, s);
+                    factor([&](double shift) {
+                        launch_ic(P->sw_fw, P->ticket.p, d_outer, d_cols, d_diag, tpos.p, list.p, a->val.p, P->scale.p, shift,
+                                  i64(cols.size()), P->F.p, fail.p, s);
+                    });
+                }
+                pack_sweep(pf, true, d_outer, d_diag, P->F.p, P->scale.p, nullptr, P->sw_fw, s);
+                pack_sweep(pb, false, d_outer, d_diag, P->F.p, P->scale.p, P->sw_fw.pos.p, P->sw_bw, s);
                 P->fw_lvl.alloc(size_t(n));
                 P->bw_lvl.alloc(size_t(n));
-                P->ticket.alloc(2);
                 hipLaunchKernelGGL(k_sweep_empty, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, P->fw_lvl.p, P->bw_lvl.p,
                                    P->ticket.p);
                 NLF_HIP(hipGetLastError());
             } else {
                 // rows with more dependencies than the chunked sweeps take
-                build_sweep(outer, cols, diag, fr, fp, true, P->F.p, P->scale.p, P->diag.p, P->fw, s);
-                build_sweep(outer, cols, diag, br, bp, false, P->F.p, P->scale.p, P->diag.p, P->bw, s);
+                DevBuf<i32> lrows, lptr;
+                DevBuf<SweepBlock> blk;
+                LevelArgs la{n, P->fw_levels, d_outer, d_cols, d_diag, tpos.p, nullptr, nullptr};
+                BlockLevels bl;
+                std::vector<SweepBlock> bd;
+                if (P->blocks > 1) {
+                    bl = block_levels(fr, fp, bounds);
+                    for (int b = 0; b < P->blocks; ++b) bd.push_back(SweepBlock{bl.levels[size_t(b)], 0, i32(bl.seg[size_t(b)]), 0});
+                    upload(blk, bd.data(), bd.size(), s);
+                    upload(lrows, bl.rows.data(), bl.rows.size(), s);
+                    upload(lptr, bl.ptr.data(), bl.ptr.size(), s);
+                } else {
+                    upload(lrows, fr.data(), fr.size(), s);
+                    upload(lptr, fp.data(), fp.size(), s);
+                }
+                la.lrows = lrows.p;
+                la.lptr = lptr.p;
+                factor([&](double shift) {
+                    NLF_HIP(hipMemsetAsync(fail.p, 0, sizeof(int), s));
+                    hipLaunchKernelGGL(k_ic_init, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, d_outer, d_cols, d_diag, a->val.p,
+                                       P->scale.p, shift, P->F.p);
+                    hipLaunchKernelGGL(k_ic_factor, dim3(unsigned(P->blocks)), dim3(LEVEL_THREADS), 0, s, la,
+                                       P->blocks > 1 ? (const SweepBlock*)blk.p : nullptr, P->F.p, fail.p);
+                });
+                build_sweep(outer, cols, diag, fr, fp, true, P->F.p, P->scale.p, d_diag, P->fw, s);
+                build_sweep(outer, cols, diag, br, bp, false, P->F.p, P->scale.p, d_diag, P->bw, s);
                 const int widest = std::max(P->fw.W, P->bw.W);
                 P->solve_threads = std::min(LEVEL_THREADS, std::max(64, (widest + 63) / 64 * 64));
                 P->work.alloc(size_t(n));

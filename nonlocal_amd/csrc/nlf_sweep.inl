@@ -475,20 +475,157 @@ static bool plan_sweep(const std::vector<i64>& outer, const std::vector<i32>& co
     return true;
 }
 
+// ---- factorisation --------------------------------------------------------------------------------------
+// IC(0) over the forward sweep's chunks and steps.  A row takes GL lanes, one per entry: lane l holds entry l
+// below the diagonal and computes entry l above it.  What bounds it is the chain of levels again, here with
+// a memory round trip per level: with one workgroup and one thread per row, a row's entries and merges were
+// serial loads (30 us per level at 200 x 200 Q8).  No barrier: like the sweeps, a value is its own flag and
+// is read again until it is there, each wave going through the steps by itself.  Whole set-up of the
+// preconditioner, host analysis included, before and after: 200 x 200 Q8 57 -> 14.5 ms, 220 x 220 plane
+// stress 58 -> 12.6 ms, 500 x 500 Q4 30 -> 15 ms, 1000 x 1000 Q4 152 -> 109 ms, 40 x 40 Q4 1.4 -> 0.6 ms.
+//
+// Entry m of lane l's list: the position in row j (the column of entry l above the diagonal) of column
+// cols[outer[k] + m], -1 where row j lacks it.
+template<int M> constexpr int ic_lanes() { return M <= 4 ? 4 : M <= 8 ? 8 : M <= 16 ? 16 : 32; }
+// rows a workgroup takes at a time: a whole step, or what 256 registers a lane allow
+template<int M> constexpr int ic_rows() { return M <= 12 ? 64 : M <= 16 ? 32 : 16; }
+
+__global__ void k_ic_lists(i64 n, int M, int GL, const i32* __restrict__ row, const i64* __restrict__ outer,
+                           const i32* __restrict__ cols, const i64* __restrict__ diag, i32* __restrict__ list) {
+    for (i64 t = i64(blockIdx.x) * blockDim.x + threadIdx.x; t < n * M * GL; t += i64(gridDim.x) * blockDim.x) {
+        const i64 rec = t / (M * GL), k = row[rec], b = outer[k], dk = diag[k];
+        const int m = int(t / GL % M), l = int(t % GL);
+        i32 at = -1;
+        if (b + m < dk && dk + 1 + l < outer[k + 1]) {
+            const i32 i = cols[b + m], j = cols[dk + 1 + l];
+            i64 lo = outer[j], hi = diag[j];
+            while (lo < hi) {
+                const i64 mid = (lo + hi) >> 1;
+                if (cols[mid] < i) lo = mid + 1; else hi = mid;
+            }
+            if (lo < diag[j] && cols[lo] == i) at = i32(lo);
+        }
+        list[t] = at;
+    }
+}
+
+__device__ __forceinline__ double ic_load(const double* F, i64 p) {
+    return __hip_atomic_load(F + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void ic_store(double* F, i64 p, double v) {
+    if (__double2hiint(v) == SWEEP_EMPTY_HI) v = __hiloint2double(SWEEP_NAN_HI, 0);
+    __hip_atomic_store(F + p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template<int M>
+__global__ __launch_bounds__(ic_lanes<M>() * ic_rows<M>()) void k_ic_chunks(SweepArgs s, i32* ticket, const i32* __restrict__ row,
+                                                   const i64* __restrict__ outer, const i32* __restrict__ cols,
+                                                   const i64* __restrict__ diag, const i64* __restrict__ tpos,
+                                                   const i32* __restrict__ list, const double* __restrict__ a,
+                                                   const double* __restrict__ scale, double shift, double* F, int* fail) {
+    constexpr int GL = ic_lanes<M>(), G = ic_rows<M>();
+    __shared__ i32 sh_c;
+    if (threadIdx.x == 0) sh_c = atomicAdd(ticket, 1);
+    __syncthreads();
+    const i32 c = __builtin_amdgcn_readfirstlane(sh_c);
+    if (c < 0 || c >= s.chunks) return;
+    const SweepChunk ch = s.chunk[c];
+    const i32* __restrict__ sp = s.sptr + ch.step0;
+    const int g = threadIdx.x / GL, l = threadIdx.x % GL;
+    // what does not depend on the factor, one step ahead of its use
+    struct Row {
+        i64 b, dk;
+        int nl, nu;
+        i32 at[M];
+        i64 tp;
+        double av, ad;
+    };
+    const int slots = ch.steps * (64 / G);
+    auto fetch = [&](int t) {
+        Row r;
+        const int st = t / (64 / G), rec = sp[st] + t % (64 / G) * G + g;
+        const bool on = rec < sp[st + 1];
+        const i64 k = row[on ? rec : sp[st]], e = outer[k + 1];
+        r.b = outer[k];
+        r.dk = diag[k];
+        r.nl = on ? int(r.dk - r.b) : -1;
+        r.nu = on ? int(e - r.dk - 1) : 0;
+        const bool up = l < r.nu;
+        const i64 p = up ? r.dk + 1 + l : r.dk;
+#pragma unroll
+        for (int m = 0; m < M; ++m) r.at[m] = up ? list[(i64(rec) * M + m) * GL + l] : -1;
+        r.tp = tpos[p];
+        r.av = scale[k] * a[p] * scale[cols[p]];
+        r.ad = scale[k] * a[r.dk] * scale[k] + shift;
+        return r;
+    };
+    Row next = fetch(0);
+    for (int t = 0; t < slots; ++t) {
+        const Row r = next;
+        if (t + 1 < slots) next = fetch(t + 1);
+        // the entries below the diagonal and the other rows' entries, until all are there
+        double low = 0.0, fj[M];
+        bool got = !(l < r.nl);
+#pragma unroll
+        for (int m = 0; m < M; ++m) fj[m] = 0.0;
+        u32 want = 0;
+#pragma unroll
+        for (int m = 0; m < M; ++m) want |= r.at[m] >= 0 ? 1u << m : 0u;
+        for (int spin = 0;; ++spin) {
+            if (!got) low = ic_load(F, r.b + l);
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (want >> m & 1) fj[m] = ic_load(F, r.at[m]);
+            const bool give_up = spin >= SWEEP_SPIN;
+            if (!got && (__double2hiint(low) != SWEEP_EMPTY_HI || give_up)) got = true;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if ((want >> m & 1) && (__double2hiint(fj[m]) != SWEEP_EMPTY_HI || give_up)) want &= ~(1u << m);
+            if (!__ballot(!got || want)) break;
+        }
+        double d = r.ad, v = r.av;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const double x = __shfl(low, m, GL);
+            if (m < r.nl) d -= x * x;
+            if (r.at[m] >= 0) v -= x * fj[m];
+        }
+        if (r.nl >= 0) {
+            if (!(d > 0.0) || !isfinite(d)) {
+                if (l == 0) *fail = 1;
+                d = 1.0;
+            }
+            const double ukk = sqrt(d);
+            if (l == 0) ic_store(F, r.dk, ukk);
+            if (l < r.nu) {
+                v /= ukk;
+                ic_store(F, r.dk + 1 + l, v);
+                if (r.tp != r.dk + 1 + l) ic_store(F, r.tp, v);
+            }
+        }
+    }
+}
+
+// F emptied, the ticket and the failure flag cleared
+__global__ void k_ic_empty(i64 nnz, double* __restrict__ F, i32* __restrict__ ticket, int* __restrict__ fail) {
+    const double empty = __longlong_as_double(static_cast<long long>(SWEEP_EMPTY));
+    for (i64 i = i64(blockIdx.x) * blockDim.x + threadIdx.x; i < nnz; i += i64(gridDim.x) * blockDim.x) F[i] = empty;
+    if (blockIdx.x == 0 && threadIdx.x == 0) { *ticket = 0; *fail = 0; }
+}
+
 // One sweep on the device.
 struct Sweep {
     int chunks = 0, WE = 4, levels = 0, width = 64;
     DevBuf<SweepChunk> chunk;
-    DevBuf<i32> sptr, eptr, esrc, rsrc, pos;
+    DevBuf<i32> sptr, eptr, esrc, rsrc, pos, row;
     DevBuf<double> rcoef;
     DevBuf<unsigned char> rec;
     i64 plane = 0;
     SweepArgs args() const { return {chunks, chunk.p, sptr.p, eptr.p, esrc.p, rsrc.p, rcoef.p, rec.p, plane}; }
 };
 
-static void upload_sweep(const SweepPlan& P, bool forward, const i64* d_outer, const i64* d_diag, const double* F,
-                         const double* scale, const i32* fw_pos, Sweep& sw, hipStream_t s) {
-    const i64 n = i64(P.row.size());
+// The plan without the factor's values.
+static void upload_plan(const SweepPlan& P, Sweep& sw, hipStream_t s) {
     sw.chunks = int(P.chunk.size());
     sw.WE = P.WE;
     sw.levels = P.levels;
@@ -499,17 +636,50 @@ static void upload_sweep(const SweepPlan& P, bool forward, const i64* d_outer, c
     const i32 none = 0;
     upload(sw.esrc, P.esrc.empty() ? &none : P.esrc.data(), std::max<size_t>(P.esrc.size(), 1), s);
     upload(sw.pos, P.pos.data(), P.pos.size(), s);
-    DevBuf<i32> row, dep;
-    upload(row, P.row.data(), P.row.size(), s);
+    upload(sw.row, P.row.data(), P.row.size(), s);
+    NLF_HIP(hipStreamSynchronize(s));                   // `none`
+}
+
+// The records, from the factor.
+static void pack_sweep(const SweepPlan& P, bool forward, const i64* d_outer, const i64* d_diag, const double* F,
+                       const double* scale, const i32* fw_pos, Sweep& sw, hipStream_t s) {
+    const i64 n = i64(P.row.size());
+    DevBuf<i32> dep;
     upload(dep, P.dep.data(), P.dep.size(), s);
     sw.plane = 16 * (n + 64);
     sw.rec.alloc(size_t(12 * P.WE) * size_t(n + 64));
     sw.rcoef.alloc(size_t(n + 64));
     sw.rsrc.alloc(size_t(n + 64));
-    hipLaunchKernelGGL(k_sweep_pack, dim3(grid_stride_blocks((n + 64) * P.WE)), dim3(256), 0, s, n, P.WE, int(forward), row.p, d_outer,
-                       d_diag, F, scale, fw_pos, dep.p, sw.rec.p, sw.rcoef.p, sw.rsrc.p);
+    hipLaunchKernelGGL(k_sweep_pack, dim3(grid_stride_blocks((n + 64) * P.WE)), dim3(256), 0, s, n, P.WE, int(forward), sw.row.p,
+                       d_outer, d_diag, F, scale, fw_pos, dep.p, sw.rec.p, sw.rcoef.p, sw.rsrc.p);
     NLF_HIP(hipGetLastError());
-    NLF_HIP(hipStreamSynchronize(s));                   // the plan's host arrays and `row` are released
+    NLF_HIP(hipStreamSynchronize(s));                   // the plan's host arrays are released
+}
+
+// The lists of k_ic_chunks (by record); 32-bit positions.
+static void ic_lists(const Sweep& w, i64 n, const i64* outer, const i32* cols, const i64* diag, DevBuf<i32>& list, hipStream_t s) {
+    const int GL = w.WE <= 4 ? 4 : w.WE <= 8 ? 8 : w.WE <= 16 ? 16 : 32;
+    list.alloc(size_t(n) * size_t(w.WE) * size_t(GL));
+    hipLaunchKernelGGL(k_ic_lists, dim3(grid_stride_blocks(n * w.WE * GL)), dim3(256), 0, s, n, w.WE, GL, w.row.p, outer, cols,
+                       diag, list.p);
+}
+
+static void launch_ic(const Sweep& w, i32* ticket, const i64* outer, const i32* cols, const i64* diag, const i64* tpos,
+                      const i32* list, const double* a, const double* scale, double shift, i64 nnz, double* F, int* fail,
+                      hipStream_t s) {
+    hipLaunchKernelGGL(k_ic_empty, dim3(grid_stride_blocks(nnz)), dim3(256), 0, s, nnz, F, ticket, fail);
+#define NLF_IC_CASE(W)                                                                                                   \
+    hipLaunchKernelGGL((k_ic_chunks<W>), dim3(unsigned(w.chunks)), dim3(unsigned(ic_lanes<W>() * ic_rows<W>())), 0, s,         \
+                       w.args(), ticket, w.row.p, outer, cols, diag, tpos, list, a, scale, shift, F, fail)
+    switch (w.WE) {
+        case 4: NLF_IC_CASE(4); break;
+        case 8: NLF_IC_CASE(8); break;
+        case 12: NLF_IC_CASE(12); break;
+        case 16: NLF_IC_CASE(16); break;
+        case 24: NLF_IC_CASE(24); break;
+        default: NLF_IC_CASE(32); break;
+    }
+#undef NLF_IC_CASE
 }
 
 static void launch_sweep(const Sweep& w, const double* src, double* lvl, i32* ticket, const CGState* st, hipStream_t s) {

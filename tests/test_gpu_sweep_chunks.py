@@ -2,12 +2,15 @@
 that every sweep layout is held to: chunk edges (64 rows of nodes), one chunk longer than the LDS
 window, node numbers in random order (dependencies from everywhere, most of them read through memory),
 rows with up to 32 dependencies, and one row with more (the packed sweep)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 from nonlocal_amd import _abi as A
 from nonlocal_amd import api, configs, meshgen
+from nonlocal_amd._lib import load
 from oracle import oracle as O
 from tests import helpers as H
 
@@ -92,3 +95,28 @@ def test_sweep_matches_oracle(gpu_ctx, name, build, kernel):
     bad[int(np.flatnonzero(inner)[0])] = np.nan
     assert np.isnan(Pg.solve(torch.from_numpy(bad).to(gpu_ctx.device)).cpu().numpy()).any()
     assert np.array_equal(z, Pg.solve(torch.from_numpy(r).to(gpu_ctx.device)).cpu().numpy())
+
+
+def test_shifted_factorisation(gpu_ctx):
+    """Couplings enlarged until the unshifted IC(0) meets a non-positive pivot: the retries find the oracle's
+    shift, the factor is emptied in between, and the apply matches."""
+    problem = grid(70, 66)
+    om, KL, f, xD, inner = H.oracle_assembly(problem, part=A.NLF_PART_LOCAL)
+    g = api.mesh_2d(problem.mesh, gpu_ctx)
+    K = api._assemble(g, 0, problem.models, problem.materials, inner, part=A.NLF_PART_LOCAL)
+    c = KL.export(0)
+    rows = np.repeat(np.arange(len(c.outer) - 1), np.diff(c.outer))
+    add = np.where(rows != c.inner, 0.6 * c.val, 0.0)
+    KL.set_values(c.val + add)
+    rc = np.ascontiguousarray(np.stack([rows, c.inner], axis=1), dtype=np.int64)
+    gpu_ctx.check(load().nlf_matrix_add_pairs(K.h, len(add), rc.ctypes.data_as(C.POINTER(C.c_int64)),
+                                              np.ascontiguousarray(add).ctypes.data_as(C.POINTER(C.c_double))))
+    P, Pg = O.OraclePrecond(A.NLF_PRECOND_ILLT, KL), api.preconditioner(K, A.NLF_PRECOND_ILLT)
+    ok, shift = P.ok()
+    assert ok and shift > 0.0
+    assert Pg.info()["ok"] and Pg.info()["shift"] == shift
+    r = np.random.default_rng(4).standard_normal(f.size)
+    z = Pg.solve(torch.from_numpy(r).to(gpu_ctx.device)).cpu().numpy()
+    print(f"[sweep] shift {shift}, rel err {H.rel_l2(z, P.apply(r)):.2e}", flush=True)
+    # the shifted factor is ill conditioned: an error of 1e-16 in the pivots grows by 1 / shift and more
+    assert H.rel_l2(z, P.apply(r)) <= 1e-10
