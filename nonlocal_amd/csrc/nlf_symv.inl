@@ -8,11 +8,11 @@
 //   * values column-major over U_s: sval[(kptr[s] + k) * 64 + lane] is row 64 s + lane's entry at
 //     offset U_s[k], 0 where the row has none (the padding of rows with other patterns);
 //   * meta[kptr[s] + k] = {U_s[k], window index of lane 0's transposed target, or -1 for the diagonal}.
-// The wave accumulates a_ij x_j of its rows in registers and the transposed products a_ij x_i in a
-// wave-private LDS window.  The window holds one strip per band (a run of consecutive offsets
-// u_b .. u_b + w_b - 1 of U_s): the targets 64 s + u_b + [0, 64 + w_b - 1).  One wave owns the window
-// and its LDS accesses execute in program order, so no atomics and no barriers are needed and the
-// sums run in a fixed order.  The window is then written out (part[pbase[s] + i]).  A second kernel
+// A wave accumulates a_ij x_j of the rows in registers and the transposed products a_ij x_i in an LDS
+// window.  The window holds one strip per band (a run of consecutive offsets u_b .. u_b + w_b - 1 of
+// U_s): the targets 64 s + u_b + [0, 64 + w_b - 1).  One wave owns a strip and its LDS accesses execute
+// in program order, so no atomics are needed and the sums run in a fixed order.  The window is then
+// written out (part[pbase[s] + i]).  A second kernel
 // adds, per target row, the strips that cover it in (slice, band) order to the row's direct sum.
 // The result is bitwise reproducible; it differs from the full-storage kernels' in summation order.
 //
@@ -31,32 +31,35 @@ struct SymBand {                         // a run of consecutive offsets of a sl
     int pad_;
 };
 
-#ifndef NLF_SYMV_WAVES
-#define NLF_SYMV_WAVES 4
-#endif
-#ifndef NLF_SYMV_UNROLL
-#define NLF_SYMV_UNROLL 8
-#endif
-constexpr int SYMV_WAVES = NLF_SYMV_WAVES;    // slices per block of the product kernel
-constexpr int SYMV_UNROLL = NLF_SYMV_UNROLL;  // entries each lane has in flight
+constexpr int SYMV_WAVES = 4;            // waves of a slice
+constexpr int SYMV_UNROLL = 8;           // entries each lane has in flight
 
+// Where waves 1 .. 3 of a slice begin among its slots: at starts of bands, so that no two waves add to one strip.
+struct SymCut {
+    int at[SYMV_WAVES - 1];
+};
+
+// Four waves share a slice, each taking whole bands (about a quarter of the slots); their direct sums are
+// added in wave order.  With a wave per slice and a window per wave the windows' LDS held a compute unit to
+// 16 waves, and a small matrix had few waves with long chains.  Product, before and after: 40 x 40
+// (26 slices) 23 -> 9.7 us, 150 x 150 with 8 elements' reach 47 -> 20, 220 x 220 plane stress 83 -> 60,
+// 1000 x 1000 composite 527 -> 508.
 template<bool STOP>
-__global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, i64 ns, int wmax, const i64* __restrict__ kptr,
-                                                                 const int2* __restrict__ meta, const double* __restrict__ sval,
+__global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, i64 ns, const i64* __restrict__ kptr,
+                                                                 const SymCut* __restrict__ cut, const int2* __restrict__ meta,
+                                                                 const double* __restrict__ sval,
                                                                  const i64* __restrict__ pbase, const double* __restrict__ x,
                                                                  double* __restrict__ direct, double* __restrict__ part,
                                                                  const CGState* __restrict__ st) {
-    extern __shared__ double win[];
+    extern __shared__ double W[];
+    __shared__ double sum[SYMV_WAVES - 1][64];
     if (STOP && st->done) return;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-    const i64 s = i64(blockIdx.x) * SYMV_WAVES + w;
-    if (s >= ns) return;
-    double* W = win + size_t(w) * size_t(wmax);
-    const i64 k0 = kptr[s], k1 = kptr[s + 1];
-    const i64 pb = pbase[s];
+    const i64 s = blockIdx.x;
+    const i64 kb = kptr[s], pb = pbase[s];
     const int wl = int(pbase[s + 1] - pb);
-    for (int i = lane; i < wl; i += 64) W[i] = 0.0;
+    const i64 k0 = w ? kb + cut[s].at[w - 1] : kb, k1 = w < SYMV_WAVES - 1 ? kb + cut[s].at[w] : kptr[s + 1];
     const i64 r = s * 64 + lane;
     const i64 rc = r < rows ? r : rows - 1;
     const double xr = r < rows ? x[r] : 0.0;
@@ -75,7 +78,9 @@ __global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, i64 n
             if (!in) { m[t].y = -1; a[t] = 0.0; }
         }
     };
-    load(k0, mc, ac);
+    if (k0 < k1) load(k0, mc, ac);
+    for (int i = threadIdx.x; i < wl; i += 64 * SYMV_WAVES) W[i] = 0.0;
+    __syncthreads();
     for (i64 k = k0; k < k1; k += SYMV_UNROLL) {
         double xc[SYMV_UNROLL];
 #pragma unroll
@@ -95,8 +100,14 @@ __global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, i64 n
             for (int t = 0; t < SYMV_UNROLL; ++t) { mc[t] = mn[t]; ac[t] = an[t]; }
         }
     }
-    if (r < rows) direct[r] = acc;
-    for (int i = lane; i < wl; i += 64) part[pb + i] = W[i];
+    if (w) sum[w - 1][lane] = acc;
+    __syncthreads();
+    if (w == 0 && r < rows) {
+#pragma unroll
+        for (int t = 0; t < SYMV_WAVES - 1; ++t) acc += sum[t][lane];
+        direct[r] = acc;
+    }
+    for (int i = threadIdx.x; i < wl; i += 64 * SYMV_WAVES) part[pb + i] = W[i];
 }
 
 // y_t = direct_t + the strips covering t in (slice, band) order; DOT: partial[block] = sum x_t y_t.
@@ -115,9 +126,16 @@ __global__ __launch_bounds__(256) void k_symv_reduce(i64 rows, i64 ns, const i64
         const i64 t = tau * 64 + lane;
         double acc = t < rows ? direct[t] : 0.0;
         const i64 e1 = rptr[tau + 1];
-        for (i64 e = rptr[tau]; e < e1; ++e) {
-            const SymEntry q = ent[e];
-            if (lane >= q.lo && lane < q.hi) acc += part[q.base + lane];
+        // eight strips' loads in flight; the sums stay in order
+        for (i64 e = rptr[tau]; e < e1; e += 8) {
+            double v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const SymEntry q = ent[e + k < e1 ? e + k : e1 - 1];
+                v[k] = e + k < e1 && lane >= q.lo && lane < q.hi ? part[q.base + lane] : 0.0;
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc += v[k];
         }
         if (t < rows) {
             y[t] = acc;
@@ -239,7 +257,7 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* 
                                                            const double* __restrict__ val, int words,
                                                            const i64* __restrict__ kptr, const i64* __restrict__ bptr,
                                                            int2* __restrict__ meta, SymBand* __restrict__ band,
-                                                           double* __restrict__ sval) {
+                                                           SymCut* __restrict__ cut, double* __restrict__ sval) {
     extern __shared__ unsigned bm[];          // words bitmap, words rank prefixes, words band prefixes
     unsigned* pre = bm + words;
     unsigned* bpre = pre + words;
@@ -280,6 +298,14 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* 
     for (int b = threadIdx.x; b < nbands; b += SYMB_THREADS) {
         const int next = b + 1 < nbands ? start_rank[b + 1] : total;
         band[bb + b] = SymBand{start_u[b], 63 * b + start_rank[b], next - start_rank[b], 0};
+    }
+    // the product's waves begin at the starts of bands next to the quarters of the slots
+    if (threadIdx.x < SYMV_WAVES - 1) {
+        const int target = int(i64(total) * (int(threadIdx.x) + 1) / SYMV_WAVES);
+        int best = total;
+        for (int b = 0; b < nbands; ++b)
+            if (abs(start_rank[b] - target) < abs(best - target)) best = start_rank[b];
+        cut[s].at[threadIdx.x] = best;
     }
     // values: the slice's slots SYMF_CHUNK at a time, each chunk assembled in an LDS tile (slot-major,
     // 64 rows a slot, zero where a row lacks the offset) and then stored whole, so that every store
@@ -380,6 +406,7 @@ struct nlf_symv_s {
     nlf::i64 version = -1;               // the matrix value version it was built from
     nlf::DevBuf<nlf::i64> kptr, pbase, rptr;
     nlf::DevBuf<int2> meta;
+    nlf::DevBuf<nlf::SymCut> cut;        // where the product's waves begin in each slice
     nlf::DevBuf<double> sval, part, direct;
     nlf::DevBuf<nlf::SymEntry> ent;
 };
@@ -444,6 +471,7 @@ bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
     sv->part_size = pbv[ns];
     DevBuf<i64> bptr;
     upload(bptr, bp.data(), bp.size(), s);
+    sv->cut.alloc(size_t(ns));
     sv->meta.alloc(size_t(std::max<i64>(slots, 1)));
     sv->sval.alloc(size_t(std::max<i64>(slots, 1)) * 64);
     sv->part.alloc(size_t(std::max<i64>(pbv[ns], 1)));
@@ -451,7 +479,7 @@ bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
     DevBuf<SymBand> band{size_t(std::max<i64>(bp[ns], 1))};
     hipLaunchKernelGGL(k_sym_fill, dim3(unsigned(ns)), dim3(SYMB_THREADS), symf_lds_bytes(words), s, rows,
                        a->outer.p, a->cols.p, a->diag.p, a->val.p, words, sv->kptr.p, bptr.p, sv->meta.p, band.p,
-                       sv->sval.p);
+                       sv->cut.p, sv->sval.p);
     NLF_HIP(hipGetLastError());
     // strips per target slice, in (slice, band) order
     const i64 nbands = bp[ns];
@@ -484,13 +512,13 @@ template<bool DOT>
 void launch_symv(const nlf_matrix_s* a, const double* x, double* y, double* partial, const CGState* st, hipStream_t s,
                  unsigned blocks) {
     const nlf_symv_s& v = *a->symv;
-    const unsigned b1 = unsigned((v.ns + SYMV_WAVES - 1) / SYMV_WAVES);
-    const size_t lds = size_t(SYMV_WAVES) * size_t(v.wmax) * sizeof(double);
+    const unsigned b1 = unsigned(v.ns);
+    const size_t lds = size_t(v.wmax) * sizeof(double);
     if (st)
-        hipLaunchKernelGGL(k_symv_slices<true>, dim3(b1), dim3(64 * SYMV_WAVES), lds, s, a->rows, v.ns, v.wmax, v.kptr.p,
+        hipLaunchKernelGGL(k_symv_slices<true>, dim3(b1), dim3(64 * SYMV_WAVES), lds, s, a->rows, v.ns, v.kptr.p, v.cut.p,
                            v.meta.p, v.sval.p, v.pbase.p, x, v.direct.p, v.part.p, st);
     else
-        hipLaunchKernelGGL(k_symv_slices<false>, dim3(b1), dim3(64 * SYMV_WAVES), lds, s, a->rows, v.ns, v.wmax, v.kptr.p,
+        hipLaunchKernelGGL(k_symv_slices<false>, dim3(b1), dim3(64 * SYMV_WAVES), lds, s, a->rows, v.ns, v.kptr.p, v.cut.p,
                            v.meta.p, v.sval.p, v.pbase.p, x, v.direct.p, v.part.p, st);
     const unsigned b2 = std::max(1u, blocks);
     if (st)
