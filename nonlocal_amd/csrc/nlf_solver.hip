@@ -1444,9 +1444,10 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
                 P->ticket.alloc(2);
                 {
                     DevBuf<i32> list;
-                    ic_lists(P->sw_fw, n, d_outer, d_cols, d_diag, list, s);
+                    const int W = std::max(P->sw_fw.WE, P->sw_bw.WE);
+                    ic_lists(P->sw_fw, W, n, d_outer, d_cols, d_diag, list, s);
                     factor([&](double shift) {
-                        launch_ic(P->sw_fw, P->ticket.p, d_outer, d_cols, d_diag, tpos.p, list.p, a->val.p, P->scale.p, shift,
+                        launch_ic(P->sw_fw, W, P->ticket.p, d_outer, d_cols, d_diag, tpos.p, list.p, a->val.p, P->scale.p, shift,
                                   i64(cols.size()), P->F.p, fail.p, s);
                     });
                 }

@@ -40,7 +40,7 @@ constexpr i64 SWEEP_CHUNK_ROWS = 1 << 23;   // most rows of a chunk (32-bit byte
 constexpr int SWEEP_CTL = 16, SWEEP_IDLE = 64, SWEEP_SP = 320, SWEEP_WIN = 832, SWEEP_RHS = SWEEP_WIN + SWEEP_K * 512, SWEEP_XV = SWEEP_RHS + SWEEP_R * 512,
               SWEEP_LDS = SWEEP_XV + SWEEP_EXT * 8;
 constexpr int SWEEP_ALL = 1 << 30;       // a helper wave has staged every step
-constexpr int SWEEP_SPIN = 1 << 24;      // reads of a missing value before it is taken as NaN (seconds)
+constexpr int SWEEP_SPIN = 1 << 21;      // reads of a missing value before it is taken as NaN (seconds)
 constexpr unsigned long long SWEEP_EMPTY = 0xfff8dead0badc0deull;
 constexpr int SWEEP_EMPTY_HI = int(SWEEP_EMPTY >> 32), SWEEP_NAN_HI = 0x7ff80000;
 
@@ -657,21 +657,23 @@ static void pack_sweep(const SweepPlan& P, bool forward, const i64* d_outer, con
 }
 
 // The lists of k_ic_chunks (by record); 32-bit positions.
-static void ic_lists(const Sweep& w, i64 n, const i64* outer, const i32* cols, const i64* diag, DevBuf<i32>& list, hipStream_t s) {
-    const int GL = w.WE <= 4 ? 4 : w.WE <= 8 ? 8 : w.WE <= 16 ? 16 : 32;
-    list.alloc(size_t(n) * size_t(w.WE) * size_t(GL));
-    hipLaunchKernelGGL(k_ic_lists, dim3(grid_stride_blocks(n * w.WE * GL)), dim3(256), 0, s, n, w.WE, GL, w.row.p, outer, cols,
+// W: the width class of the rows' entries on either side of the diagonal, whichever has more (a lane computes an
+// entry above it, and the lists run over those below).
+static void ic_lists(const Sweep& w, int W, i64 n, const i64* outer, const i32* cols, const i64* diag, DevBuf<i32>& list, hipStream_t s) {
+    const int GL = W <= 4 ? 4 : W <= 8 ? 8 : W <= 16 ? 16 : 32;
+    list.alloc(size_t(n) * size_t(W) * size_t(GL));
+    hipLaunchKernelGGL(k_ic_lists, dim3(grid_stride_blocks(n * W * GL)), dim3(256), 0, s, n, W, GL, w.row.p, outer, cols,
                        diag, list.p);
 }
 
-static void launch_ic(const Sweep& w, i32* ticket, const i64* outer, const i32* cols, const i64* diag, const i64* tpos,
+static void launch_ic(const Sweep& w, int W, i32* ticket, const i64* outer, const i32* cols, const i64* diag, const i64* tpos,
                       const i32* list, const double* a, const double* scale, double shift, i64 nnz, double* F, int* fail,
                       hipStream_t s) {
     hipLaunchKernelGGL(k_ic_empty, dim3(grid_stride_blocks(nnz)), dim3(256), 0, s, nnz, F, ticket, fail);
-#define NLF_IC_CASE(W)                                                                                                   \
-    hipLaunchKernelGGL((k_ic_chunks<W>), dim3(unsigned(w.chunks)), dim3(unsigned(ic_lanes<W>() * ic_rows<W>())), 0, s,         \
+#define NLF_IC_CASE(C)                                                                                                   \
+    hipLaunchKernelGGL((k_ic_chunks<C>), dim3(unsigned(w.chunks)), dim3(unsigned(ic_lanes<C>() * ic_rows<C>())), 0, s,         \
                        w.args(), ticket, w.row.p, outer, cols, diag, tpos, list, a, scale, shift, F, fail)
-    switch (w.WE) {
+    switch (W) {
         case 4: NLF_IC_CASE(4); break;
         case 8: NLF_IC_CASE(8); break;
         case 12: NLF_IC_CASE(12); break;

@@ -1,7 +1,8 @@
 """The chunked ILLT sweeps where their plan can go wrong, against the oracle's IC(0) apply at the 1e-12
 that every sweep layout is held to: chunk edges (64 rows of nodes), one chunk longer than the LDS
 window, node numbers in random order (dependencies from everywhere, most of them read through memory),
-rows with up to 32 dependencies, and one row with more (the packed sweep)."""
+rows with up to 32 entries on one side of the diagonal and few on the other, and one row with more (the
+packed sweep)."""
 import ctypes as C
 
 import numpy as np
@@ -45,14 +46,17 @@ def grid(nx, ny, seed=None):
     return _problem(_mesh(xy, elems, edges))
 
 
-def fan(m):
-    """m quads around one node of 2 m neighbours, numbered last; the first two outer nodes are fixed."""
+def fan(m, hub_first=False):
+    """m quads around one node of 2 m neighbours, numbered last or first; two outer nodes are fixed."""
     t = np.linspace(0.0, 2.0 * np.pi, 2 * m, endpoint=False)
     r = np.where(np.arange(2 * m) % 2, 1.0, 0.9)
     xy = np.concatenate([np.stack([r * np.cos(t), r * np.sin(t)], axis=1), [[0.0, 0.0]]])
     k = 2 * np.arange(m)
     elems = np.stack([np.full(m, 2 * m), k, k + 1, (k + 2) % (2 * m)], axis=1)
-    return _problem(_mesh(xy, elems, [[0, 1]]))
+    edges = np.array([[0, 1]])
+    if hub_first:
+        xy, elems, edges = np.roll(xy, 1, axis=0), (elems + 1) % (2 * m + 1), edges + 1
+    return _problem(_mesh(xy, elems, edges))
 
 
 def elastic_q8(n):
@@ -71,6 +75,8 @@ CASES = [
     ("q8_elastic", lambda: elastic_q8(15), 2),
     ("fan_32", lambda: fan(17), 2),
     ("fan_34", lambda: fan(18), 0),
+    ("fan_6_hub_first", lambda: fan(4, hub_first=True), 2),
+    ("fan_32_hub_first", lambda: fan(17, hub_first=True), 2),
 ]
 
 
