@@ -34,7 +34,7 @@ constexpr int SPMV_PAIRS_IN_FLIGHT = 4;  // nonzero pairs each lane of the pair 
 constexpr int LEVEL_THREADS = 1024;
 
 struct CGState {
-    double rz, pq, alpha, beta, bnorm, res, tol;
+    double rz, rz_prev, pq, alpha, beta, bnorm, res, tol;
     int done, indefinite;                // indefinite: p'Ap < 0 is not a breakdown (bordered Neumann systems)
     i64 it, max_it;
     int breakdown, pad2;
@@ -239,30 +239,51 @@ __global__ void k_sum_partials(const double* __restrict__ partial, int n, double
     if (threadIdx.x == 0) *out = s;
 }
 
-// alpha = rz / (p . A p)
-__global__ void k_alpha(const double* __restrict__ partial, int n, CGState* __restrict__ st) {
-    __shared__ double sh[1024 / 64];
-    if (st->done) return;
+// The sum of n partials in every thread (the same in every block: all add in one order).
+__device__ __forceinline__ double sum_partials(const double* __restrict__ partial, int n, double* sh) {
     double s = 0.0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) s += partial[i];
     s = block_sum<double>(s, sh);
-    if (threadIdx.x == 0) {
-        st->pq = s;
-        st->alpha = st->rz / s;
-        const bool bad_curvature = st->indefinite ? s == 0.0 : !(s > 0.0);
-        if (bad_curvature || !isfinite(st->alpha)) { st->breakdown = 1; st->done = 1; }
-    }
+    if (threadIdx.x == 0) sh[0] = s;
+    __syncthreads();
+    s = sh[0];
+    __syncthreads();
+    return s;
 }
 
-// x += alpha p; r -= alpha q; z = M r (identity / Jacobi, or left for a separate apply); partial rz.
+// st->done as one thread reads it: the first block may set it while this one starts
+__device__ __forceinline__ bool stopped(const CGState* st) {
+    __shared__ int done;
+    if (threadIdx.x == 0) done = st->done;
+    __syncthreads();
+    return done != 0;
+}
+
+// alpha = rz / (p . A p); x += alpha p; r -= alpha q; z = M r (identity / Jacobi, or left for a separate
+// apply); partial rz.  Every block sums the partials of p . A p itself, which costs a small system less than
+// a launch for it does (40 x 40 nodes: a solve of 47
+// iterations 4.86 -> 4.53 ms with k_update_p's); the first one
+// keeps the state, of which the others read nothing that it writes but the stop, which all find alike.
 template<class X, bool JACOBI, bool DOT>
 __global__ __launch_bounds__(SPMV_THREADS) void k_update_xr(i64 n, X* __restrict__ x, X* __restrict__ r, const X* __restrict__ p,
                                                             const X* __restrict__ q, X* __restrict__ z,
-                                                            const X* __restrict__ invd, double* __restrict__ partial,
-                                                            const CGState* __restrict__ st) {
+                                                            const X* __restrict__ invd, const double* __restrict__ ppq, int npq,
+                                                            double* __restrict__ partial, CGState* st) {
     __shared__ double sh[SPMV_THREADS / 64];
-    if (st->done) return;
-    const X a = X(st->alpha);
+    if (stopped(st)) return;
+    const double pq = sum_partials(ppq, npq, sh), rz = st->rz, alpha = rz / pq;
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    if (first) {
+        st->pq = pq;
+        st->alpha = alpha;
+        st->rz_prev = rz;
+    }
+    const bool bad_curvature = st->indefinite ? pq == 0.0 : !(pq > 0.0);
+    if (bad_curvature || !isfinite(alpha)) {
+        if (first) { st->breakdown = 1; st->done = 1; }
+        return;
+    }
+    const X a = X(alpha);
     double d = 0.0;
     for (i64 i = i64(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += i64(gridDim.x) * blockDim.x) {
         x[i] += a * p[i];
@@ -292,27 +313,23 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_dot(i64 n, const X* __restrict
     if (threadIdx.x == 0) partial[blockIdx.x] = d;
 }
 
-// mu = rz_new / rz; residual = sqrt(rz)/||b||; stop test of the reference.
-__global__ void k_beta(const double* __restrict__ partial, int n, CGState* __restrict__ st) {
-    __shared__ double sh[1024 / 64];
-    if (st->done) return;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) s += partial[i];
-    s = block_sum<double>(s, sh);
-    if (threadIdx.x == 0) {
-        st->beta = s / st->rz;
-        st->rz = s;
+// mu = rz_new / rz; p = z + mu p; residual = sqrt(rz)/||b||; stop test of the reference.  The partials of
+// r.z are summed as in k_update_xr; a direction left half updated by the stop is not used again.
+template<class X>
+__global__ __launch_bounds__(SPMV_THREADS) void k_update_p(i64 n, X* __restrict__ p, const X* __restrict__ z,
+                                                           const double* __restrict__ prz, int nrz, CGState* st) {
+    __shared__ double sh[SPMV_THREADS / 64];
+    if (stopped(st)) return;
+    const double rz = sum_partials(prz, nrz, sh), beta = rz / st->rz_prev;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->beta = beta;
+        st->rz = rz;
         st->it += 1;
-        st->res = sqrt(fabs(s)) / st->bnorm;
+        st->res = sqrt(fabs(rz)) / st->bnorm;
         if (!isfinite(st->res)) { st->breakdown = 1; st->done = 1; }
         if (st->res <= st->tol || st->it >= st->max_it) st->done = 1;
     }
-}
-
-template<class X>
-__global__ void k_update_p(i64 n, X* __restrict__ p, const X* __restrict__ z, const CGState* __restrict__ st) {
-    if (st->done) return;
-    const X b = X(st->beta);
+    const X b = X(beta);
     for (i64 i = i64(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += i64(gridDim.x) * blockDim.x) p[i] = z[i] + b * p[i];
 }
 
@@ -1046,6 +1063,11 @@ void residual64(const nlf_matrix_s* a, const double* x, const double* b, double*
 }
 
 
+// Blocks of CG's vector kernels and of the symmetric product's reduction: every block of the next kernel sums
+// their partials.
+constexpr unsigned CG_BLOCKS = 1024;
+constexpr i64 SYMV_REDUCE_BLOCKS = 2048;
+
 // Preconditioned CG on device vectors (conjugate_gradient::solve).  Vectors of type X, matrix values V.
 // The work memory (CGWork) is allocated by the object, or given by the caller (no allocation then;
 // `timed` = false also records no HIP events).
@@ -1091,7 +1113,7 @@ struct CG {
         sums = reinterpret_cast<double*>(take(2 * sizeof(double)));
         st = reinterpret_cast<CGState*>(take(sizeof(CGState)));
         sblocks = spmv_blocks(lpr, n);
-        vblocks = grid_stride_blocks(n);
+        vblocks = std::min(grid_stride_blocks(n), CG_BLOCKS);
     }
 
     bool jacobi() const { return P && P->kind == NLF_PRECOND_JACOBI; }
@@ -1103,13 +1125,21 @@ struct CG {
         sblocks = spmv_blocks(lpr, n);
     }
 
+    // FP64 products from the symmetric storage (symv_prepare done): any number of partials
+    void set_symmetric(const nlf_matrix_s* a) {
+        sym = a;
+        sblocks = unsigned(std::min<i64>((a->symv->ns + 3) / 4, SYMV_REDUCE_BLOCKS));
+    }
+
     const X* invd() const;
 
     // x: initial guess in, solution out; b: right-hand side.  Returns iterations, sets residual.
     i64 solve(const X* b, X* x, double tol, i64 max_it, double* residual, int* breakdown, int check_every = 8) {
         // r = b - A x ; z = M r ; rz = r.z ; bnorm
-        hipLaunchKernelGGL((k_residual<V, X>), dim3(spmv_blocks(64, n)), dim3(SPMV_THREADS), 0, s, n, outer, cols, val, x, b,
-                           r, part1, part2);
+        if (sym) residual64(sym, x, b, r, part1, part2, spmv_blocks(64, n), s);
+        else
+            hipLaunchKernelGGL((k_residual<V, X>), dim3(spmv_blocks(64, n)), dim3(SPMV_THREADS), 0, s, n, outer, cols, val, x, b,
+                               r, part1, part2);
         const int nb_res = int(spmv_blocks(64, n));
         NLF_HIP(hipMemcpyAsync(pbb, part2, size_t(nb_res) * sizeof(double), hipMemcpyDeviceToDevice, s));
         precond_apply(P, n, r, p, nullptr, s);
@@ -1206,7 +1236,7 @@ struct CG {
     }
 
     void iteration(X* x, bool sample = false) {
-        // z = A p ; alpha = rz / p.z
+        // z = A p with the partials of p.z
         if (sample) timer.start(0, s);
         bool done_sym = false;
         if constexpr (std::is_same_v<V, double> && std::is_same_v<X, double>) {
@@ -1217,25 +1247,23 @@ struct CG {
         }
         if (!done_sym) launch_spmv<V, X, double, true>(lpr, n, outer, cs, val, p, z, part1, st, s, false, lo);
         if (sample) timer.stop(0, s);
-        hipLaunchKernelGGL(k_alpha, dim3(1), dim3(1024), 0, s, part1, int(sblocks), st);
         if (!P || P->kind == NLF_PRECOND_IDENTITY || jacobi()) {
             // x += a p ; r -= a z ; z = M r ; partial r.z  (fused)
             if (jacobi())
                 hipLaunchKernelGGL((k_update_xr<X, true, true>), dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, x, r, p, z,
-                                   z, invd(), part2, st);
+                                   z, invd(), part1, int(sblocks), part2, st);
             else
                 hipLaunchKernelGGL((k_update_xr<X, false, true>), dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, x, r, p,
-                                   z, z, (const X*)nullptr, part2, st);
+                                   z, z, (const X*)nullptr, part1, int(sblocks), part2, st);
         } else {
             hipLaunchKernelGGL((k_update_xr<X, false, false>), dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, x, r, p, z,
-                               (X*)nullptr, (const X*)nullptr, part2, st);
+                               (X*)nullptr, (const X*)nullptr, part1, int(sblocks), part2, st);
             if (sample) timer.start(1, s);
             const bool dotted = precond_apply(P, n, r, z, st, s, part2, vblocks);
             if (sample) timer.stop(1, s);
             if (!dotted) hipLaunchKernelGGL(k_dot<X>, dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, r, z, part2, st);
         }
-        hipLaunchKernelGGL(k_beta, dim3(1), dim3(1024), 0, s, part2, int(vblocks), st);
-        hipLaunchKernelGGL(k_update_p<X>, dim3(vblocks), dim3(256), 0, s, n, p, z, st);
+        hipLaunchKernelGGL(k_update_p<X>, dim3(vblocks), dim3(SPMV_THREADS), 0, s, n, p, z, part2, int(vblocks), st);
     }
 };
 
@@ -1661,9 +1689,9 @@ int nlf_cg_solve(nlf_matrix a, nlf_precond p, const double* b, double* x, double
         };
         if (mode == NLF_MODE_FP64) {
             CG<double, double> cg(s, n, a->nnz_full, a->outer.p, a->cols.p, a->val.p, p);
-            cg.set_cols(a);
             cg.indefinite = a->neumann;
-            if (symv_prepare(a, s)) cg.sym = a;
+            if (symv_prepare(a, s)) cg.set_symmetric(a);
+            else cg.set_cols(a);
             out.iterations = cg.solve(b, x, tol, max_it, &out.residual, &breakdown);
             timings(cg.timer, sizeof(double), sizeof(double));
         } else {
@@ -1675,9 +1703,9 @@ int nlf_cg_solve(nlf_matrix a, nlf_precond p, const double* b, double* x, double
             // and need several times the iterations, while FP32 storage costs none; the FP64 true
             // residual with the FP64 matrix replaces the recursive one at every reliable update.
             CG<float, double> cg(s, n, a->nnz_full, a->outer.p, a->cols.p, a->val32.p, p);
-            cg.set_cols(a);
             cg.indefinite = a->neumann;
             if (mode == NLF_MODE_SPLIT) cg.lo = a->val_lo.p;
+            cg.set_cols(a);
             out.iterations = cg.solve_reliable(a->outer.p, a->cols.p, a->val.p, b, x, tol, max_it, 0.1,
                                                &out.true_residual, &out.outer_iterations, &breakdown);
             out.residual = out.true_residual;
