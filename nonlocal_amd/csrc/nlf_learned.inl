@@ -1521,9 +1521,10 @@ i64 fcg(hipStream_t s, nlf_matrix A, const V* val, nlf_precond M, const double* 
         double* true_res, i64* updates, int window, KernelTimer& timer, const int16_t* lo = nullptr) {
     const i64 n = A->rows;
     LearnedGraph& g = *learned_of(M);
-    // FP64 values: the products read the upper triangle once (the symmetric storage), when it applies
-    bool sym = false;
-    if constexpr (std::is_same_v<V, double>) sym = !lo && symv_prepare(A, s);
+    // the products read the upper triangle once (the symmetric storage), when it applies
+    const bool sym = symv_prepare(A, s);
+    const SymValues which = std::is_same_v<V, double> ? SYM_FP64 : lo ? SYM_SPLIT : SYM_FP32;
+    if (sym && which != SYM_FP64) symv_fill_low(A, which, s);
     // the lane count (and with it the partial-sum grid) the full-storage layout would take; the symmetric
     // storage applies only where every offset is below 2^15, as the 16-bit one does, so it is known
     // without building that layout
@@ -1542,7 +1543,7 @@ i64 fcg(hipStream_t s, nlf_matrix A, const V* val, nlf_precond M, const double* 
     };
     auto spmv_pq = [&](bool sample) {             // q = A p, partial p.q into pb; partial p.r into pa
         if (sample) timer.start(0, s);
-        if (sym) launch_symv<true>(A, p.p, q.p, pb.p, nullptr, s, sb);
+        if (sym) launch_symv<true>(A, p.p, q.p, pb.p, nullptr, s, sb, which);
         else launch_spmv<V, double, double, true>(lpr, n, A->outer.p, spmv_cols(A), val, p.p, q.p, pb.p, nullptr, s, false, lo);
         if (sample) timer.stop(0, s);
         hipLaunchKernelGGL(k_dot<double>, dim3(sb), dim3(SPMV_THREADS), 0, s, n, p.p, r.p, pa.p, (const CGState*)nullptr);

@@ -1089,7 +1089,7 @@ struct CG {
     unsigned sblocks, vblocks;
     bool timed = true;
     bool indefinite = false;            // a bordered (Neumann) system: negative curvature allowed
-    const nlf_matrix_s* sym = nullptr;  // FP64 products from the symmetric storage (symv_prepare done)
+    const nlf_matrix_s* sym = nullptr;  // products from the symmetric storage (symv_prepare done)
     KernelTimer timer;
 
     CG(hipStream_t s_, i64 n_, i64 nnz, const i64* o, const i32* c, const V* v, const nlf_precond_s* P_,
@@ -1125,7 +1125,7 @@ struct CG {
         sblocks = spmv_blocks(lpr, n);
     }
 
-    // FP64 products from the symmetric storage (symv_prepare done): any number of partials
+    // products from the symmetric storage (symv_prepare done): any number of partials
     void set_symmetric(const nlf_matrix_s* a) {
         sym = a;
         sblocks = unsigned(std::min<i64>((a->symv->ns + 3) / 4, SYMV_REDUCE_BLOCKS));
@@ -1179,7 +1179,8 @@ struct CG {
         DevBuf<double> r64{size_t(n)};
         DevBuf<X> xh{size_t(n)};
         auto true_residual = [&]() {
-            residual64(n, o64, cs, v64, lpr, x, b, r64.p, part1, part2, rb, s);
+            if (sym) residual64(sym, x, b, r64.p, part1, part2, rb, s);
+            else residual64(n, o64, cs, v64, lpr, x, b, r64.p, part1, part2, rb, s);
             hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, part1, int(rb), sums);
             hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, part2, int(rb), sums + 1);
             double h[2];
@@ -1238,14 +1239,8 @@ struct CG {
     void iteration(X* x, bool sample = false) {
         // z = A p with the partials of p.z
         if (sample) timer.start(0, s);
-        bool done_sym = false;
-        if constexpr (std::is_same_v<V, double> && std::is_same_v<X, double>) {
-            if (sym) {
-                launch_symv<true>(sym, p, z, part1, st, s, sblocks);
-                done_sym = true;
-            }
-        }
-        if (!done_sym) launch_spmv<V, X, double, true>(lpr, n, outer, cs, val, p, z, part1, st, s, false, lo);
+        if (sym) launch_symv<true>(sym, p, z, part1, st, s, sblocks, std::is_same_v<V, double> ? SYM_FP64 : lo ? SYM_SPLIT : SYM_FP32);
+        else launch_spmv<V, X, double, true>(lpr, n, outer, cs, val, p, z, part1, st, s, false, lo);
         if (sample) timer.stop(0, s);
         if (!P || P->kind == NLF_PRECOND_IDENTITY || jacobi()) {
             // x += a p ; r -= a z ; z = M r ; partial r.z  (fused)
@@ -1283,10 +1278,10 @@ namespace nlf {
 // HBM bytes one SpMV streams: values, column source, row pointers, x once and y.
 i64 spmv_stream_bytes(const nlf_matrix_s* a, size_t sv, size_t sx) {
     const i64 n = a->rows;
-    if (a->symv && sv == sizeof(double) && a->symv->version == a->val_version) {
+    if (a->symv && a->ctx->spmv_symmetric && a->symv->version == a->val_version) {
         // slice values, the strips written and read, the direct sums written and read, x once and y
         const nlf_symv_s& v = *a->symv;
-        return v.slots * 64 * i64(sizeof(double)) + 2 * v.part_size * i64(sizeof(double)) + n * i64(4 * sizeof(double));
+        return v.slots * 64 * i64(sv) + 2 * v.part_size * i64(sizeof(double)) + n * i64(4 * sizeof(double));
     }
     ensure_spmv_storage(a);
     i64 cols = a->nnz_full * i64(a->off16.p ? sizeof(int16_t) : sizeof(i32));
@@ -1705,7 +1700,12 @@ int nlf_cg_solve(nlf_matrix a, nlf_precond p, const double* b, double* x, double
             CG<float, double> cg(s, n, a->nnz_full, a->outer.p, a->cols.p, a->val32.p, p);
             cg.indefinite = a->neumann;
             if (mode == NLF_MODE_SPLIT) cg.lo = a->val_lo.p;
-            cg.set_cols(a);
+            if (symv_prepare(a, s)) {
+                symv_fill_low(a, cg.lo ? SYM_SPLIT : SYM_FP32, s);
+                cg.set_symmetric(a);
+            } else {
+                cg.set_cols(a);
+            }
             out.iterations = cg.solve_reliable(a->outer.p, a->cols.p, a->val.p, b, x, tol, max_it, 0.1,
                                                &out.true_residual, &out.outer_iterations, &breakdown);
             out.residual = out.true_residual;

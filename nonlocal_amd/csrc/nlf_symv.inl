@@ -39,15 +39,30 @@ struct SymCut {
     int at[SYMV_WAVES - 1];
 };
 
+// The instances (of a batch) whose rows a slice holds, and which of them are done; inst null: no batch.
+struct SymSkip {
+    const int2* inst;                    // first and last instance of each slice
+    const int* done;                     // done[i * stride]
+    int stride;
+    __device__ __forceinline__ bool all_done(i64 s) const {
+        if (!inst) return false;
+        const int2 r = inst[s];
+        for (int i = r.x; i <= r.y; ++i)
+            if (!done[i64(i) * stride]) return false;
+        return true;
+    }
+};
+
 // Four waves share a slice, each taking whole bands (about a quarter of the slots); their direct sums are
 // added in wave order.  With a wave per slice and a window per wave the windows' LDS held a compute unit to
 // 16 waves, and a small matrix had few waves with long chains.  Product, before and after: 40 x 40
 // (26 slices) 23 -> 9.7 us, 150 x 150 with 8 elements' reach 47 -> 20, 220 x 220 plane stress 83 -> 60,
 // 1000 x 1000 composite 527 -> 508.
-template<bool STOP>
-__global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, i64 ns, const i64* __restrict__ kptr,
+// V = float (SPLIT: with the 16-bit remainders lo): the reduced values of the mixed solves, FP64 sums.
+template<bool STOP, class V, bool SPLIT>
+__global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, SymSkip skip, const i64* __restrict__ kptr,
                                                                  const SymCut* __restrict__ cut, const int2* __restrict__ meta,
-                                                                 const double* __restrict__ sval,
+                                                                 const V* __restrict__ sval, const int16_t* __restrict__ lo,
                                                                  const i64* __restrict__ pbase, const double* __restrict__ x,
                                                                  double* __restrict__ direct, double* __restrict__ part,
                                                                  const CGState* __restrict__ st) {
@@ -57,6 +72,7 @@ __global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, i64 n
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
     const i64 s = blockIdx.x;
+    if (skip.all_done(s)) return;
     const i64 kb = kptr[s], pb = pbase[s];
     const int wl = int(pbase[s + 1] - pb);
     const i64 k0 = w ? kb + cut[s].at[w - 1] : kb, k1 = w < SYMV_WAVES - 1 ? kb + cut[s].at[w] : kptr[s + 1];
@@ -74,7 +90,9 @@ __global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, i64 n
             const bool in = kk + t < k1;
             const i64 q = in ? kk + t : k1 - 1;
             m[t] = meta[q];
-            a[t] = __builtin_nontemporal_load(sval + q * 64 + lane);
+            const V v = __builtin_nontemporal_load(sval + q * 64 + lane);
+            if constexpr (SPLIT) a[t] = split_value(v, __builtin_nontemporal_load(lo + q * 64 + lane));
+            else a[t] = double(v);
             if (!in) { m[t].y = -1; a[t] = 0.0; }
         }
     };
@@ -112,7 +130,7 @@ __global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, i64 n
 
 // y_t = direct_t + the strips covering t in (slice, band) order; DOT: partial[block] = sum x_t y_t.
 template<bool DOT, bool STOP>
-__global__ __launch_bounds__(256) void k_symv_reduce(i64 rows, i64 ns, const i64* __restrict__ rptr,
+__global__ __launch_bounds__(256) void k_symv_reduce(i64 rows, i64 ns, SymSkip skip, const i64* __restrict__ rptr,
                                                      const SymEntry* __restrict__ ent, const double* __restrict__ direct,
                                                      const double* __restrict__ part, const double* __restrict__ x,
                                                      double* __restrict__ y, double* __restrict__ partial,
@@ -123,6 +141,7 @@ __global__ __launch_bounds__(256) void k_symv_reduce(i64 rows, i64 ns, const i64
     const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
     double d = 0.0;
     for (i64 tau = i64(blockIdx.x) * 4 + w; tau < ns; tau += i64(gridDim.x) * 4) {
+        if (skip.all_done(tau)) continue;
         const i64 t = tau * 64 + lane;
         double acc = t < rows ? direct[t] : 0.0;
         const i64 e1 = rptr[tau + 1];
@@ -239,7 +258,8 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_count(i64 rows, const i64*
     }
 }
 
-// meta, bands and the values of slice s (sval zeroed beforehand).  With rank(u) the position of u in
+// meta, bands and the values of slice s; with meta null, only the values (of another type: the FP32 values, or
+// the remainders of the split ones).  With rank(u) the position of u in
 // U_s and band(u) the number of run starts <= u less one, the window index of u is 63 band + rank:
 // the strips before band b take sum_{b' < b} (64 + w_b' - 1) = 63 b + rank(u_b) entries, and ranks
 // run on consecutively inside a band.
@@ -252,12 +272,13 @@ __host__ __device__ constexpr size_t symf_lds_bytes(int words) {
     return symf_tile_offset(words) * sizeof(unsigned) + size_t(SYMF_CHUNK) * 64 * sizeof(double);
 }
 
+template<class V>
 __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* __restrict__ outer,
                                                            const i32* __restrict__ cols, const i64* __restrict__ diag,
-                                                           const double* __restrict__ val, int words,
+                                                           const V* __restrict__ val, int words,
                                                            const i64* __restrict__ kptr, const i64* __restrict__ bptr,
                                                            int2* __restrict__ meta, SymBand* __restrict__ band,
-                                                           SymCut* __restrict__ cut, double* __restrict__ sval) {
+                                                           SymCut* __restrict__ cut, V* __restrict__ sval) {
     extern __shared__ unsigned bm[];          // words bitmap, words rank prefixes, words band prefixes
     unsigned* pre = bm + words;
     unsigned* bpre = pre + words;
@@ -265,7 +286,7 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* 
     __shared__ int start_rank[256], start_u[256];
     const i64 s = blockIdx.x;
     sym_bitmap(rows, s, outer, cols, diag, words, bm);
-    const i64 kb = kptr[s], bb = bptr[s];
+    const i64 kb = kptr[s], bb = meta ? bptr[s] : 0;
     // prefixes over the words: thread t takes the contiguous run [t cw, t cw + cw)
     const int cw = (words + SYMB_THREADS - 1) / SYMB_THREADS;
     const int w0 = min(words, int(threadIdx.x) * cw), w1 = min(words, w0 + cw);
@@ -280,7 +301,7 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* 
         st += __popc(run_starts(bm, i));
     }
     __syncthreads();
-    for (int i = w0; i < w1; ++i) {
+    for (int i = w0; meta && i < w1; ++i) {
         unsigned v = bm[i];
         const unsigned starts = run_starts(bm, i);
         while (v) {
@@ -295,12 +316,12 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* 
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < nbands; b += SYMB_THREADS) {
+    for (int b = threadIdx.x; meta && b < nbands; b += SYMB_THREADS) {
         const int next = b + 1 < nbands ? start_rank[b + 1] : total;
         band[bb + b] = SymBand{start_u[b], 63 * b + start_rank[b], next - start_rank[b], 0};
     }
     // the product's waves begin at the starts of bands next to the quarters of the slots
-    if (threadIdx.x < SYMV_WAVES - 1) {
+    if (meta && threadIdx.x < SYMV_WAVES - 1) {
         const int target = int(i64(total) * (int(threadIdx.x) + 1) / SYMV_WAVES);
         int best = total;
         for (int b = 0; b < nbands; ++b)
@@ -312,7 +333,7 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* 
     // is coalesced and the padding needs no clearing pass of its own.  A row's upper entries are in
     // ascending offset, so in ascending slot rank: the entries of one chunk are the next run of the
     // row, which wave w (rows w, w + 4, ...) reads 64 at a time from the row's cursor.
-    double (*tile)[64] = reinterpret_cast<double (*)[64]>(bm + symf_tile_offset(words));
+    V (*tile)[64] = reinterpret_cast<V (*)[64]>(bm + symf_tile_offset(words));
     __shared__ i64 cursor[64];
     const int lane = threadIdx.x & 63, wv = int(threadIdx.x >> 6);
     if (threadIdx.x < 64) {
@@ -320,7 +341,7 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* 
         cursor[threadIdx.x] = r < rows ? diag[r] : 0;
     }
     for (int k0 = 0; k0 < total; k0 += SYMF_CHUNK) {
-        for (int e = threadIdx.x; e < SYMF_CHUNK * 64; e += SYMB_THREADS) tile[e >> 6][e & 63] = 0.0;
+        for (int e = threadIdx.x; e < SYMF_CHUNK * 64; e += SYMB_THREADS) tile[e >> 6][e & 63] = V(0);
         __syncthreads();
         for (int j = wv; j < 64; j += SYMB_THREADS / 64) {
             const i64 r = s * 64 + j;
@@ -330,7 +351,7 @@ __global__ __launch_bounds__(SYMB_THREADS) void k_sym_fill(i64 rows, const i64* 
             for (;;) {
                 const i64 p = p0 + lane;
                 int rank = 0x7fffffff;                         // past the row's end: in no chunk
-                double v = 0.0;
+                V v = V(0);
                 if (p < e) {
                     const int u = int(cols[p] - r);
                     rank = int(pre[u >> 5] + __popc(bm[u >> 5] & ((1u << (u & 31)) - 1u)));
@@ -401,6 +422,7 @@ __global__ void k_sym_entries(i64 n, i64 ns, const unsigned long long* __restric
 struct nlf_symv_s {
     nlf::i64 ns = 0;                     // slices of 64 rows
     int wmax = 0;                        // longest window (doubles)
+    int words = 0;                       // bitmap words of the widest offset
     nlf::i64 slots = 0;                  // sum of |U_s| (values = 64 slots)
     nlf::i64 part_size = 0;              // doubles of the strips
     nlf::i64 version = -1;               // the matrix value version it was built from
@@ -408,6 +430,8 @@ struct nlf_symv_s {
     nlf::DevBuf<int2> meta;
     nlf::DevBuf<nlf::SymCut> cut;        // where the product's waves begin in each slice
     nlf::DevBuf<double> sval, part, direct;
+    nlf::DevBuf<float> sval32;           // the reduced values of the mixed solve that filled them last
+    nlf::DevBuf<int16_t> slo;
     nlf::DevBuf<nlf::SymEntry> ent;
 };
 
@@ -418,9 +442,14 @@ void symv_release(nlf_matrix_s* a) {
     a->symv = nullptr;
 }
 
+// Longest window of a slice (doubles, 56 KB of the 64 KB of LDS that a launch may ask for): a reach of about
+// 30 elements on a structured mesh.  256 x 256 nodes with 25.6 elements' reach: 270 us from the full storage,
+// 163 us here (windows of 4600 doubles, four workgroups to a compute unit).
+constexpr i64 SYMV_WINDOW = 7168;
+
 // Builds (or rebuilds, when the values changed) the symmetric SpMV storage of a FP64 matrix.  Returns
 // false, with nothing kept, where it does not apply: offsets of 2^15 or more, more than 255 bands in a
-// slice, a window over 2048 doubles, or padding that leaves less than a quarter of the traffic saved.
+// slice, a window over SYMV_WINDOW doubles, or padding that leaves less than a quarter of the traffic saved.
 bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
     if (!a->ctx->spmv_symmetric || a->rows <= 0 || !a->val.p || a->nnz_full <= 0) return false;
     if (a->symv && a->symv->version == a->val_version && !a->values_exposed) return true;
@@ -454,10 +483,11 @@ bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
     const i64 upper_offdiag = a->nnz_upper - rows;
     // bytes: 8 per slot of 64 values and the strips twice, against 8 per full-storage value
     const double sym_bytes = double(slots) * 64.0 * 8.0 + 2.0 * 8.0 * double(std::accumulate(hW.begin(), hW.end(), i64(0)));
-    if (maxb > 255 || maxw > 2048 || sym_bytes > 0.75 * 8.0 * double(a->nnz_full) || upper_offdiag <= 0) return refuse();
+    if (maxb > 255 || maxw > SYMV_WINDOW || sym_bytes > 0.75 * 8.0 * double(a->nnz_full) || upper_offdiag <= 0) return refuse();
     auto sv = std::make_unique<nlf_symv_s>();
     sv->ns = ns;
     sv->wmax = int(maxw);
+    sv->words = words;
     sv->slots = slots;
     sv->part_size = 0;
     std::vector<i64> kp(ns + 1, 0), pbv(ns + 1, 0), bp(ns + 1, 0);
@@ -477,7 +507,7 @@ bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
     sv->part.alloc(size_t(std::max<i64>(pbv[ns], 1)));
     sv->direct.alloc(size_t(rows));
     DevBuf<SymBand> band{size_t(std::max<i64>(bp[ns], 1))};
-    hipLaunchKernelGGL(k_sym_fill, dim3(unsigned(ns)), dim3(SYMB_THREADS), symf_lds_bytes(words), s, rows,
+    hipLaunchKernelGGL(k_sym_fill<double>, dim3(unsigned(ns)), dim3(SYMB_THREADS), symf_lds_bytes(words), s, rows,
                        a->outer.p, a->cols.p, a->diag.p, a->val.p, words, sv->kptr.p, bptr.p, sv->meta.p, band.p,
                        sv->cut.p, sv->sval.p);
     NLF_HIP(hipGetLastError());
@@ -506,26 +536,52 @@ bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
     return true;
 }
 
+// The values a product reads: the FP64 ones, the FP32 ones or the split ones (symv_fill_low first).
+enum SymValues { SYM_FP64, SYM_FP32, SYM_SPLIT };
+
+// Fills the slices' reduced values from val32 (and val_lo); symv_prepare first.  Each mixed solve fills them
+// anew (one pass over the upper triangle), so they never lag behind the matrix's.
+void symv_fill_low(nlf_matrix_s* a, SymValues which, hipStream_t s) {
+    nlf_symv_s& v = *a->symv;
+    const size_t n = size_t(std::max<i64>(v.slots, 1)) * 64;
+    auto fill = [&](auto* from, auto* to) {
+        using V = std::remove_pointer_t<decltype(to)>;
+        hipLaunchKernelGGL(k_sym_fill<V>, dim3(unsigned(v.ns)), dim3(SYMB_THREADS), symf_lds_bytes(v.words), s, a->rows,
+                           a->outer.p, a->cols.p, a->diag.p, (const V*)from, v.words, v.kptr.p, (const i64*)nullptr,
+                           (int2*)nullptr, (SymBand*)nullptr, (SymCut*)nullptr, to);
+    };
+    if (v.sval32.n < n) v.sval32.alloc(n);
+    fill(a->val32.p, v.sval32.p);
+    if (which == SYM_SPLIT) {
+        if (v.slo.n < n) v.slo.alloc(n);
+        fill(a->val_lo.p, v.slo.p);
+    }
+    NLF_HIP(hipGetLastError());
+}
+
 // y = A x from the symmetric storage (symv_prepare first); DOT: partial[0 .. blocks) of x.y, the
 // reduction running on `blocks` blocks (any count: the caller's partial count).
 template<bool DOT>
 void launch_symv(const nlf_matrix_s* a, const double* x, double* y, double* partial, const CGState* st, hipStream_t s,
-                 unsigned blocks) {
+                 unsigned blocks, SymValues which = SYM_FP64, SymSkip skip = SymSkip{nullptr, nullptr, 0}) {
     const nlf_symv_s& v = *a->symv;
-    const unsigned b1 = unsigned(v.ns);
     const size_t lds = size_t(v.wmax) * sizeof(double);
-    if (st)
-        hipLaunchKernelGGL(k_symv_slices<true>, dim3(b1), dim3(64 * SYMV_WAVES), lds, s, a->rows, v.ns, v.kptr.p, v.cut.p,
-                           v.meta.p, v.sval.p, v.pbase.p, x, v.direct.p, v.part.p, st);
-    else
-        hipLaunchKernelGGL(k_symv_slices<false>, dim3(b1), dim3(64 * SYMV_WAVES), lds, s, a->rows, v.ns, v.kptr.p, v.cut.p,
-                           v.meta.p, v.sval.p, v.pbase.p, x, v.direct.p, v.part.p, st);
+    auto slices = [&](auto kernel, auto* values) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(v.ns)), dim3(64 * SYMV_WAVES), lds, s, a->rows, skip, (const i64*)v.kptr.p,
+                           (const SymCut*)v.cut.p, (const int2*)v.meta.p, values, (const int16_t*)v.slo.p,
+                           (const i64*)v.pbase.p, x, v.direct.p, v.part.p, st);
+    };
+    const double* v64 = v.sval.p;
+    const float* v32 = v.sval32.p;
+    if (which == SYM_FP64) st ? slices(k_symv_slices<true, double, false>, v64) : slices(k_symv_slices<false, double, false>, v64);
+    else if (which == SYM_FP32) st ? slices(k_symv_slices<true, float, false>, v32) : slices(k_symv_slices<false, float, false>, v32);
+    else st ? slices(k_symv_slices<true, float, true>, v32) : slices(k_symv_slices<false, float, true>, v32);
     const unsigned b2 = std::max(1u, blocks);
     if (st)
-        hipLaunchKernelGGL((k_symv_reduce<DOT, true>), dim3(b2), dim3(256), 0, s, a->rows, v.ns, v.rptr.p, v.ent.p,
+        hipLaunchKernelGGL((k_symv_reduce<DOT, true>), dim3(b2), dim3(256), 0, s, a->rows, v.ns, skip, v.rptr.p, v.ent.p,
                            v.direct.p, v.part.p, x, y, partial, st);
     else
-        hipLaunchKernelGGL((k_symv_reduce<DOT, false>), dim3(b2), dim3(256), 0, s, a->rows, v.ns, v.rptr.p, v.ent.p,
+        hipLaunchKernelGGL((k_symv_reduce<DOT, false>), dim3(b2), dim3(256), 0, s, a->rows, v.ns, skip, v.rptr.p, v.ent.p,
                            v.direct.p, v.part.p, x, y, partial, st);
 }
 
