@@ -1458,19 +1458,32 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
                     shift = shift == 0.0 ? 1e-3 : 2 * shift;
                 }
             };
-            SweepPlan pf, pb;
-            P->chunked = cols.size() < (size_t(1) << 31) && plan_sweep(outer, cols, diag, fr, fp, bounds, true, pf) &&
-                         plan_sweep(outer, cols, diag, br, bp, bounds, false, pb);
+            SweepPlan pf, pb, pi;                        // forward, backward; the factorisation's where rows merge
+            std::vector<uint8_t> mf, mb;
+            std::vector<i32> mrows, mptr;
+            auto plan = [&](bool forward, std::vector<uint8_t>& merged, SweepPlan& q) {
+                if (merged_levels(outer, cols, diag, forward, merged, mrows, mptr))
+                    return plan_sweep(outer, cols, diag, mrows, mptr, bounds, forward, merged, false, q);
+                merged.clear();
+                return plan_sweep(outer, cols, diag, forward ? fr : br, forward ? fp : bp, bounds, forward, merged, false, q);
+            };
+            P->chunked = cols.size() < (size_t(1) << 31) && plan(true, mf, pf) && plan(false, mb, pb);
             if (P->chunked) {
                 upload_plan(pf, P->sw_fw, s);
                 upload_plan(pb, P->sw_bw, s);
                 P->ticket.alloc(2);
                 {
+                    Sweep own;                           // a merged pair's rows are factored one after the other
+                    if (!mf.empty()) {
+                        plan_sweep(outer, cols, diag, fr, fp, bounds, true, {}, true, pi);
+                        upload_plan(pi, own, s);
+                    }
+                    const Sweep& sw = mf.empty() ? P->sw_fw : own;
                     DevBuf<i32> list;
                     const int W = std::max(P->sw_fw.WE, P->sw_bw.WE);
-                    ic_lists(P->sw_fw, W, n, d_outer, d_cols, d_diag, list, s);
+                    ic_lists(sw, W, n, d_outer, d_cols, d_diag, list, s);
                     factor([&](double shift) {
-                        launch_ic(P->sw_fw, W, P->ticket.p, d_outer, d_cols, d_diag, tpos.p, list.p, a->val.p, P->scale.p, shift,
+                        launch_ic(sw, W, P->ticket.p, d_outer, d_cols, d_diag, tpos.p, list.p, a->val.p, P->scale.p, shift,
                                   i64(cols.size()), P->F.p, fail.p, s);
                     });
                 }

@@ -7,7 +7,8 @@
 // levels: with one workgroup for all rows a level cost a barrier among ten waves and all record traffic
 // went through one compute unit; a chunk's level is one wave's work with no barrier.  One apply (both
 // sweeps, one workgroup against chunks): 500 x 500 Q4 nodes 1.14 -> 0.34 ms, 1000 x 1000 2.41 -> 0.71 ms,
-// 220 x 220 plane stress 3.07 -> 0.50 ms, 200 x 200 Q8 3.77 -> 0.62 ms, 40 x 40 Q4 67 -> 33 us.
+// 220 x 220 plane stress 3.07 -> 0.50 ms, 200 x 200 Q8 3.77 -> 0.62 ms, 40 x 40 Q4 67 -> 33 us
+// (before rows were merged, see merged_levels).
 //
 // A workgroup is four waves, one per SIMD, that talk through LDS counters:
 //   compute  holds the next records (factor values, dependency addresses) in a register ring and has no
@@ -329,13 +330,15 @@ __global__ void k_sweep_empty(i64 n, double* __restrict__ fw, double* __restrict
     if (blockIdx.x == 0 && threadIdx.x < 2) ticket[threadIdx.x] = 0;
 }
 
-// The records' values from the factor: entry j of a record is its row's j-th entry below (forward) or
-// above (backward) the diagonal over the diagonal; the right-hand side's factor is s_k / U_kk and the
-// row (forward) or 1 / U_kk and the row's record in the forward sweep (backward).
+// The records' values from the factor.  Entry j of a record is its row's j-th entry below (forward) or above
+// (backward) the diagonal over the diagonal; of a row merged with the one before it in the sweep (see
+// merged_levels) it is the entry at src[2 t] less m times that row's at src[2 t + 1] (-1: none), m the
+// coefficient between the two, and m itself for src[2 t + 1] = -2.  The right-hand side's factor is s_k / U_kk
+// and the row (forward) or 1 / U_kk and the row's record in the forward sweep (backward).
 __global__ void k_sweep_pack(i64 n, int WE, int forward, const i32* __restrict__ row, const i64* __restrict__ outer,
                              const i64* __restrict__ diag, const double* __restrict__ F, const double* __restrict__ scale,
-                             const i32* __restrict__ fw_pos, const i32* __restrict__ dep, unsigned char* __restrict__ out,
-                             double* __restrict__ rcoef, i32* __restrict__ rsrc) {
+                             const i32* __restrict__ fw_pos, const i32* __restrict__ dep, const i32* __restrict__ src,
+                             unsigned char* __restrict__ out, double* __restrict__ rcoef, i32* __restrict__ rsrc) {
     for (i64 t = i64(blockIdx.x) * blockDim.x + threadIdx.x; t < (n + 64) * WE; t += i64(gridDim.x) * blockDim.x) {
         const i64 rec = t / WE;
         const int j = int(t - rec * WE);
@@ -347,9 +350,20 @@ __global__ void k_sweep_pack(i64 n, int WE, int forward, const i32* __restrict__
             if (j == 0) { rcoef[rec] = 0.0; rsrc[rec] = 0; }
             continue;
         }
-        const i64 k = row[rec], dk = diag[k], p = (forward ? outer[k] : dk + 1) + j, e = forward ? dk : outer[k + 1];
+        const i64 k = row[rec], dk = diag[k];
         const double inv = 1.0 / F[dk];
-        *v = p < e ? F[p] * inv : 0.0;
+        if (src) {
+            const i32 pk = src[2 * t], pa = src[2 * t + 1];
+            double x = pk >= 0 ? F[pk] * inv : 0.0;
+            if (pa != -1) {
+                const double m = F[forward ? dk - 1 : dk + 1] * inv;
+                x = pa < 0 ? m : x - m * (F[pa] / F[diag[forward ? k - 1 : k + 1]]);
+            }
+            *v = x;
+        } else {
+            const i64 p = (forward ? outer[k] : dk + 1) + j, e = forward ? dk : outer[k + 1];
+            *v = p < e ? F[p] * inv : 0.0;
+        }
         *d = dep[t];
         if (j == 0) {
             rcoef[rec] = forward ? scale[k] * inv : inv;
@@ -365,30 +379,105 @@ struct SweepPlan {
     std::vector<i32> sptr, eptr, esrc;
     std::vector<i32> row, pos;           // row of each record, record of each row
     std::vector<i32> dep;
+    std::vector<i32> src;                // with merged rows: two factor positions per entry (k_sweep_pack)
 };
+
+static int sweep_width(i64 entries) { return entries <= 4 ? 4 : entries <= 8 ? 8 : entries <= 12 ? 12 : entries <= 16 ? 16 : entries <= 24 ? 24 : 32; }
+
+// Levels with rows merged in pairs: row k takes the place of its dependency a on the row right before it in the
+// sweep, y_a = b_a - sum c_ad y_d, into its own sum, so that both are solved at once: b_k - m b_a and the
+// coefficients c_kd - m c_ad over the union of the two rows' dependencies (and m for b_a).  A pair is merged
+// where that union still fits the entries a record has anyway, so a step costs the same and there are fewer:
+// plane stress 2 levels a node less one (1320 -> 660 at 220 x 220), Q8 1600 -> 1000 at 200 x 200; never on Q4
+// heat rows, whose unions have 6 entries.  One apply: plane stress 500 -> 280 us, Q8 617 -> 484 us.
+// False where too few pairs merge to matter.
+static bool merged_levels(const std::vector<i64>& outer, const std::vector<i32>& cols, const std::vector<i64>& diag,
+                          bool forward, std::vector<uint8_t>& merged, std::vector<i32>& lrows, std::vector<i32>& lptr) {
+    const i64 n = i64(diag.size());
+    auto begin = [&](i64 k) { return forward ? outer[k] : diag[k] + 1; };
+    auto end = [&](i64 k) { return forward ? diag[k] : outer[k + 1]; };
+    i64 widest = 0;
+    for (i64 k = 0; k < n; ++k) widest = std::max(widest, end(k) - begin(k));
+    if (widest > SWEEP_MAX_WE) return false;
+    const int cap = sweep_width(widest);
+    // whether row k's entries with those of the row before it fit a record (a itself among them: the entry of b_a)
+    auto fits = [&](i64 k) {
+        const i64 a = forward ? k - 1 : k + 1;
+        const i64 b = begin(k), e = end(k);
+        if (e == b || i64(cols[size_t(forward ? e - 1 : b)]) != a) return false;
+        i64 p = b, q = begin(a), count = 0;
+        const i64 ea = end(a);
+        while (p < e || q < ea) {
+            const i32 cp = p < e ? cols[size_t(p)] : INT32_MAX, cq = q < ea ? cols[size_t(q)] : INT32_MAX;
+            p += cp <= cq;
+            q += cq <= cp;
+            ++count;
+        }
+        return count <= cap;
+    };
+    // a look at some rows first: of those that fit, every second one is merged
+    const i64 every = std::max<i64>(1, n / 1024);
+    i64 seen = 0, fit = 0;
+    for (i64 k = every / 2; k < n; k += every, ++seen) fit += fits(k);
+    if (8 * fit < seen) return false;
+    merged.assign(size_t(n), 0);
+    std::vector<i32> lev(static_cast<size_t>(n));
+    i32 levels = 0;
+    i64 pairs = 0;
+    for (i64 o = 0; o < n; ++o) {
+        const i64 k = forward ? o : n - 1 - o, a = forward ? k - 1 : k + 1;
+        const i64 b = begin(k), e = end(k);
+        const bool linked = e > b && i64(cols[size_t(forward ? e - 1 : b)]) == a;
+        const bool join = linked && !merged[size_t(a)] && fits(k);
+        i32 l = linked ? lev[size_t(a)] + (join ? 0 : 1) : 0;
+        for (i64 p = b; p < e; ++p)
+            if (i64(cols[size_t(p)]) != a) l = std::max(l, lev[size_t(cols[size_t(p)])] + 1);
+        if (join) {
+            merged[size_t(k)] = 1;
+            ++pairs;
+            lev[size_t(a)] = l;                              // nothing but k depends on a yet
+        }
+        lev[size_t(k)] = l;
+        levels = std::max(levels, l + 1);
+    }
+    if (8 * pairs < n) return false;
+    lptr.assign(size_t(levels) + 1, 0);
+    for (i64 k = 0; k < n; ++k) lptr[size_t(lev[size_t(k)]) + 1]++;
+    for (i32 l = 0; l < levels; ++l) lptr[size_t(l) + 1] += lptr[size_t(l)];
+    lrows.resize(size_t(n));
+    std::vector<i32> at(lptr.begin(), lptr.end() - 1);
+    for (i64 o = 0; o < n; ++o) {
+        const i64 k = forward ? o : n - 1 - o;
+        lrows[size_t(at[size_t(lev[size_t(k)])]++)] = i32(k);
+    }
+    return true;
+}
 
 // Chunks, steps and dependencies of one sweep; false when a row has more than SWEEP_MAX_WE dependencies.
 // lrows / lptr: the rows by level, in sweep order within a level.  bounds: independent row blocks, whose
-// boundaries end a chunk.
+// boundaries end a chunk.  merged: rows merged with the one before them in the sweep (merged_levels; empty:
+// none), kept in one step with it.  steps_only: no dependencies (for the factorisation).
 //
 // A chunk grows while its steps stay few more than its levels: each level of the chunk then fits the
 // wave, so a longer chunk would only lengthen the chain and a shorter one would add a hand-over between
 // workgroups (about 2.5 us).  On a grid of n x n nodes in row order that is 64 rows of nodes.
 static bool plan_sweep(const std::vector<i64>& outer, const std::vector<i32>& cols, const std::vector<i64>& diag,
                        const std::vector<i32>& lrows, const std::vector<i32>& lptr, const std::vector<i64>& bounds,
-                       bool forward, SweepPlan& P) {
+                       bool forward, const std::vector<uint8_t>& merged, bool steps_only, SweepPlan& P) {
     const i64 n = i64(diag.size());
     i64 widest = 0;
     for (i64 k = 0; k < n; ++k) widest = std::max(widest, forward ? diag[k] - outer[k] : outer[k + 1] - diag[k] - 1);
     if (widest > SWEEP_MAX_WE) return false;
-    P.WE = widest <= 4 ? 4 : widest <= 8 ? 8 : widest <= 12 ? 12 : widest <= 16 ? 16 : widest <= 24 ? 24 : 32;
+    P.WE = sweep_width(widest);
+    auto is_merged = [&](i64 k) { return !merged.empty() && merged[size_t(k)]; };
     // levels wider than the cap (often level 0, the first-kind rows) are split: their records are independent
     std::vector<i32> lev(static_cast<size_t>(n));
     int levels = 0;
     i64 w = 1;
     for (size_t L = 0; L + 1 < lptr.size(); ++L)
-        for (i32 t = lptr[L]; t < lptr[L + 1]; t += SWEEP_LEVEL_CAP, ++levels) {
-            const i32 e = std::min(t + SWEEP_LEVEL_CAP, lptr[L + 1]);
+        for (i32 t = lptr[L], e; t < lptr[L + 1]; t = e, ++levels) {
+            e = std::min(t + SWEEP_LEVEL_CAP, lptr[L + 1]);
+            if (e < lptr[L + 1] && is_merged(lrows[size_t(e)])) --e;           // not between a pair
             w = std::max<i64>(w, e - t);
             for (i32 i = t; i < e; ++i) lev[size_t(lrows[size_t(i)])] = levels;
         }
@@ -405,7 +494,7 @@ static bool plan_sweep(const std::vector<i64>& outer, const std::vector<i32>& co
             const i64 k = forward ? o : n - 1 - o;
             const bool edge = b + 1 < bounds.size() && k == (forward ? bounds[b] : bounds[bounds.size() - 1 - b] - 1);
             if (edge) ++b;
-            if (c < 0 || edge || steps - distinct > std::max<i64>(4, distinct / 64) || o - first.back() >= SWEEP_CHUNK_ROWS) {
+            if (c < 0 || edge || (!is_merged(k) && (steps - distinct > std::max<i64>(4, distinct / 64) || o - first.back() >= SWEEP_CHUNK_ROWS))) {
                 ++c;
                 first.push_back(o);
                 steps = distinct = 0;
@@ -429,7 +518,8 @@ static bool plan_sweep(const std::vector<i64>& outer, const std::vector<i32>& co
             P.pos[size_t(k)] = i32(rec);
         }
     }
-    P.dep.assign(size_t(P.WE) * size_t(n), 0);
+    if (!steps_only) P.dep.assign(size_t(P.WE) * size_t(n), 0);
+    if (!merged.empty()) P.src.assign(2 * size_t(P.WE) * size_t(n), -1);
     P.chunk.resize(size_t(C));
     std::vector<i32> step_of(static_cast<size_t>(n)), lane_of(static_cast<size_t>(n));
     std::vector<i32> x_chunk(static_cast<size_t>(n), -1), x_idx(static_cast<size_t>(n), 0);     // last external slot of a row
@@ -442,7 +532,12 @@ static bool plan_sweep(const std::vector<i64>& outer, const std::vector<i32>& co
         for (i64 rec = first[size_t(c)]; rec < first[size_t(c) + 1]; ++rec) {
             const i32 k = P.row[size_t(rec)];
             const i64 pb = forward ? outer[k] : diag[k] + 1, pe = forward ? diag[k] : outer[k + 1];
-            if (lev[size_t(k)] != level || lane == 64 || in_step + int(pe - pb) > SWEEP_EXT_STEP) {
+            // a pair's records lie side by side: the later one reads the earlier one's right-hand side
+            const bool joined = is_merged(k);
+            const bool pair = rec + 1 < first[size_t(c) + 1] && is_merged(P.row[size_t(rec) + 1]) && !joined &&
+                              P.row[size_t(rec) + 1] == (forward ? k + 1 : k - 1);
+            if (!joined && (lev[size_t(k)] != level || lane + int(pair) >= 64 ||
+                            in_step + (pair ? 2 : 1) * P.WE > SWEEP_EXT_STEP)) {
                 ++step;
                 lane = in_step = 0;
                 level = lev[size_t(k)];
@@ -452,12 +547,12 @@ static bool plan_sweep(const std::vector<i64>& outer, const std::vector<i32>& co
             }
             step_of[size_t(k)] = step;
             lane_of[size_t(k)] = lane++;
+            if (steps_only) continue;
             i32* dep = &P.dep[size_t(P.WE) * size_t(rec)];
-            for (i64 p = pb; p < pe; ++p) {
-                const i32 i = cols[size_t(p)];
+            auto depend = [&](i32 i) {
                 if (chunk_of[size_t(i)] == c && step - step_of[size_t(i)] <= SWEEP_K) {
                     *dep++ = SWEEP_WIN + ((step_of[size_t(i)] % SWEEP_K) * 64 + lane_of[size_t(i)]) * 8;
-                    continue;
+                    return;
                 }
                 if (x_chunk[size_t(i)] != c || ext_begin - x_idx[size_t(i)] > SWEEP_EXT_REUSE) {
                     x_chunk[size_t(i)] = c;
@@ -466,6 +561,30 @@ static bool plan_sweep(const std::vector<i64>& outer, const std::vector<i32>& co
                     ++in_step;
                 }
                 *dep++ = SWEEP_XV + (x_idx[size_t(i)] % SWEEP_EXT) * 8;
+            };
+            if (merged.empty()) {
+                for (i64 p = pb; p < pe; ++p) depend(cols[size_t(p)]);
+                continue;
+            }
+            i32* src = &P.src[2 * size_t(P.WE) * size_t(rec)];
+            const i32 a = forward ? k - 1 : k + 1;
+            i64 p = pb, q = joined ? (forward ? outer[a] : diag[a] + 1) : 0;
+            const i64 qe = joined ? (forward ? diag[a] : outer[a + 1]) : 0;
+            while (p < pe || q < qe) {
+                const i32 cp = p < pe ? cols[size_t(p)] : INT32_MAX, cq = q < qe ? cols[size_t(q)] : INT32_MAX;
+                const i32 i = std::min(cp, cq);
+                if (joined && i == a) {
+                    src[0] = i32(p);
+                    src[1] = -2;
+                    *dep++ = SWEEP_RHS + ((step % SWEEP_R) * 64 + lane_of[size_t(a)]) * 8;
+                } else {
+                    src[0] = cp == i ? i32(p) : -1;
+                    src[1] = cq == i ? i32(q) : -1;
+                    depend(i);
+                }
+                src += 2;
+                p += cp == i;
+                q += cq == i;
             }
         }
         P.sptr.push_back(i32(first[size_t(c) + 1]));
@@ -644,14 +763,15 @@ static void upload_plan(const SweepPlan& P, Sweep& sw, hipStream_t s) {
 static void pack_sweep(const SweepPlan& P, bool forward, const i64* d_outer, const i64* d_diag, const double* F,
                        const double* scale, const i32* fw_pos, Sweep& sw, hipStream_t s) {
     const i64 n = i64(P.row.size());
-    DevBuf<i32> dep;
+    DevBuf<i32> dep, src;
     upload(dep, P.dep.data(), P.dep.size(), s);
+    if (!P.src.empty()) upload(src, P.src.data(), P.src.size(), s);
     sw.plane = 16 * (n + 64);
     sw.rec.alloc(size_t(12 * P.WE) * size_t(n + 64));
     sw.rcoef.alloc(size_t(n + 64));
     sw.rsrc.alloc(size_t(n + 64));
     hipLaunchKernelGGL(k_sweep_pack, dim3(grid_stride_blocks((n + 64) * P.WE)), dim3(256), 0, s, n, P.WE, int(forward), sw.row.p,
-                       d_outer, d_diag, F, scale, fw_pos, dep.p, sw.rec.p, sw.rcoef.p, sw.rsrc.p);
+                       d_outer, d_diag, F, scale, fw_pos, dep.p, src.p, sw.rec.p, sw.rcoef.p, sw.rsrc.p);
     NLF_HIP(hipGetLastError());
     NLF_HIP(hipStreamSynchronize(s));                   // the plan's host arrays are released
 }
