@@ -764,6 +764,109 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     }
 }
 
+// Thermal Q8 pair blocks with V_MFMA_F64_16X16X4 (measured on gfx950: lane l holds A[l % 16][l / 16],
+// B[l / 16][l % 16] and D[l / 16 + 4 r][l % 16] in register r).  With the 9 quadrature points padded to 12
+// (zero weights) and column n = 8 c + i for gradient component c of node i:
+//   V[qn][n] = sum_ql Phi[ql][qn] HL[ql][n]   three products; A lane: one influence value, B: fixed per eL
+//   T[n][n'] = sum_qn V[qn][n] HN[qn][n']     three products; D of the first is A of the second as it lies
+//   K[i][j]  = T[i][j] + T[8 + i][8 + j]      (C is in HN), one exchange between lanes 8 apart
+// A pair's influence values are evaluated once, not by each of eL's 8 nodes, and the operands are whole rows:
+// the node-centric contraction gathered 1.3 KB per node, element and neighbour, lane by lane.  Assembly of
+// 200 x 200 Q8, 10 elements' reach: 62.3 ms there, 3.4 ms here and 10.0 ms in the node kernel that adds the blocks.
+constexpr int PAIR8_ROWS = 12, PAIR8_H = PAIR8_ROWS * 16;      // doubles of an element's HL or HN
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+__global__ void k_pair8_prep(i64 E, const double* __restrict__ D, FeTables t, const i32* __restrict__ group_of,
+                             const GroupParams* __restrict__ groups, double* __restrict__ HL, double* __restrict__ HN) {
+    const i64 x = i64(blockIdx.x) * blockDim.x + threadIdx.x;      // (e, q, i)
+    if (x >= E * PAIR8_ROWS * 8) return;
+    const i64 e = x / (PAIR8_ROWS * 8);
+    const int q = int(x / 8 % PAIR8_ROWS), i = int(x % 8);
+    double lx = 0.0, ly = 0.0, nx = 0.0, ny = 0.0;
+    if (q < 9) {
+        const GroupParams g = groups[group_of[e]];
+        lx = t.w[q] * D[2 * ((e * 8 + i) * 9 + q)];
+        ly = t.w[q] * D[2 * ((e * 8 + i) * 9 + q) + 1];
+        if (g.ckind == NLF_CONDUCTIVITY_ISOTROPIC) { nx = g.c[0] * lx; ny = g.c[0] * ly; }
+        else if (g.ckind == NLF_CONDUCTIVITY_ORTHOTROPIC) { nx = g.c[0] * lx; ny = g.c[1] * ly; }
+        else { nx = g.c[0] * lx + g.c[2] * ly; ny = g.c[2] * lx + g.c[1] * ly; }
+    }
+    const i64 at = e * PAIR8_H + q * 16 + i;
+    HL[at] = lx;
+    HL[at + 8] = ly;
+    HN[at] = nx;
+    HN[at + 8] = ny;
+}
+
+template<int POLY>
+__global__ __launch_bounds__(256) void k_pairs8_mfma(PairArgs<double> a) {
+    constexpr int SETS = 2;                                       // pairs whose loads and products overlap
+    const int l = threadIdx.x & 63;
+    const int col = l & 15, h = l >> 4;
+    const i64 waves = i64(gridDim.x) * (blockDim.x >> 6);
+    for (i64 li = i64(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6); li < a.count; li += waves) {
+        const i64 eL = a.list ? a.list[li] : li;
+        const i64 slot = a.eoff[eL];
+        const GroupParams gp = a.groups[a.group_of[eL]];          // one group per wave
+        if (!gp.nonlocal) continue;
+        double hl[3], xlx[3], xly[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int ql = 4 * k + h, qc = ql < 9 ? ql : 8;       // the padding's weights are zero
+            hl[k] = a.HL[eL * PAIR8_H + ql * 16 + col];
+            xlx[k] = a.xq[2 * (eL * 9 + qc)];
+            xly[k] = a.xq[2 * (eL * 9 + qc) + 1];
+        }
+        const int qn = col < 9 ? col : 8;
+        const i64 nb_b = a.nb_off[eL], cnt = a.nb_off[eL + 1] - nb_b;
+        const i32 emin = a.el_min[eL];
+        const double s = 1.0 - gp.p1;
+        double* const out = a.pairs + i64(h + (col < 8 ? 0 : 4)) * a.plane + slot * 8 + (col & 7);
+        i32 id_next = l < cnt ? a.nb_ids[nb_b + l] : 0;
+        for (i64 b64 = 0; b64 < cnt; b64 += 64) {
+            const i32 id = id_next;
+            // the pair reaches the upper triangle of some row of eL, or a Dirichlet column
+            const bool nd = b64 + l < cnt && (a.el_max[id] >= emin || a.el_dir[id]);
+            if (b64 + 64 + l < cnt) id_next = a.nb_ids[nb_b + b64 + 64 + l];
+            unsigned long long todo = __ballot(nd);
+            while (todo) {
+                int pos[SETS];
+                double xnx[SETS], xny[SETS], hn[SETS][3];
+#pragma unroll
+                for (int u = 0; u < SETS; ++u) {
+                    pos[u] = todo ? int(__builtin_ctzll(todo)) : -1;
+                    if (todo) todo &= todo - 1;
+                    const i64 eNL = __builtin_amdgcn_readlane(id, pos[u] < 0 ? pos[0] : pos[u]);
+                    xnx[u] = a.xq[2 * (eNL * 9 + qn)];
+                    xny[u] = a.xq[2 * (eNL * 9 + qn) + 1];
+#pragma unroll
+                    for (int r = 0; r < 3; ++r) hn[u][r] = a.HN[eNL * PAIR8_H + (4 * r + h) * 16 + col];
+                }
+                f64x4 v[SETS], t[SETS];
+#pragma unroll
+                for (int u = 0; u < SETS; ++u) v[u] = t[u] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+#pragma unroll
+                    for (int u = 0; u < SETS; ++u)
+                        v[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(influence_poly<POLY>(gp.inf, xlx[k], xly[k], xnx[u], xny[u]), hl[k],
+                                                                    v[u], 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 3; ++r)
+#pragma unroll
+                    for (int u = 0; u < SETS; ++u) t[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[u][r], hn[u][r], t[u], 0, 0, 0);
+#pragma unroll
+                for (int u = 0; u < SETS; ++u) {
+                    // columns 0-7 keep rows h of component 0 and take those of component 1; columns 8-15 the rows h + 4
+                    const double other = __shfl_xor(col < 8 ? t[u][1] : t[u][2], 8);
+                    const double k = (col < 8 ? t[u][0] : t[u][3]) + other;
+                    if (pos[u] >= 0) out[(b64 + pos[u]) * 8] = s * k;
+                }
+            }
+        }
+    }
+}
+
 // FP32 pair blocks with V_MFMA_F32_4X4X1_16B_F32: sixteen independent rank-1 4x4 updates per
 // wave; lane l = 4 b + c belongs to block b and (measured on gfx950) holds A_b[c][0], B_b[0][c]
 // and D_b[i][c] in accumulator register i.  One wave handles one element eL and sixteen
@@ -953,7 +1056,7 @@ __global__ __launch_bounds__(THREADS) void k_assemble(AssemblyArgs a) {
                 if (!active[u]) continue;
                 const i64 t = base + u * i64(blockDim.x) + threadIdx.x;
                 if (from_pairs) {
-                    const T* pr = pairs + i64(iL) * a.plane + (eoff + t) * 4;
+                    const T* pr = pairs + i64(iL) * a.plane + (eoff + t) * NN;
                     for (int j = 0; j < NN; ++j) v[u][j][0] = pr[j];
                 }
                 if constexpr (NN % 4 == 0) {
@@ -1389,12 +1492,12 @@ void launch_assemble_kernel(const AssemblyArgs& a, bool injective, size_t lds, d
     }
 }
 
-// The pair-block variant runs when the arguments carry pair blocks (thermal Q4).
+// The pair-block variant runs when the arguments carry pair blocks (thermal Q4, and Q8 in FP64).
 template<int DOF, int NN, int NQ, class T>
 void launch_assemble(const AssemblyArgs& a, bool injective, size_t lds, i64 count, hipStream_t s, int threads = ASM_THREADS) {
     if (count <= 0) return;
     const dim3 g(static_cast<unsigned>(count));
-    if constexpr (DOF == 1 && NN == 4 && NQ == 4) {
+    if constexpr (DOF == 1 && (NN == 4 || sizeof(T) == sizeof(double))) {
         if (sizeof(T) == sizeof(double) ? a.pairs != nullptr : a.pairs32 != nullptr) {
             launch_assemble_kernel<DOF, NN, NQ, T, true>(a, injective, lds, g, s, threads);
             return;
@@ -1694,7 +1797,7 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
     aa.rounds = m->max_degree;
     const bool injective = m->injective;
     const bool node_only = m->ctx->assembly_pairs == 0;
-    const bool use_pairs = mat->physics == 0 && m->nn == 4 && any_nonlocal && !only_local && !node_only;
+    const bool use_pairs = mat->physics == 0 && (m->nn == 4 || F64) && any_nonlocal && !only_local && !node_only;
     // local-only matrices whose rows fit a wave: one wave per node
     unsigned long long max_upper = 0, max_bound = 0;
     if (!any_nonlocal || only_local) {
@@ -1714,14 +1817,15 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
         else if (mat->physics == 1 && m->nn == 4) hipLaunchKernelGGL((k_assemble_local<2, 4, 4, T>), dim3(nb), dim3(256), 0, s, aa);
         else hipLaunchKernelGGL((k_assemble_local<2, 8, 9, T>), dim3(nb), dim3(256), 0, s, aa);
     } else if (use_pairs) {
-        // thermal Q4 nonlocal blocks through the MFMA pair kernel.  When every element's blocks (16
+        // thermal nonlocal blocks through the MFMA pair kernels.  When every element's blocks (nn * nn
         // values per neighbour pair) fit the budget -- 8 GiB, or NLF_OPT_PAIR_BUDGET_MIB -- one pass
         // lists every element once with its blocks at its neighbour-list offset; otherwise node chunk
         // by node chunk (plan_pairs): the buffer is bounded whatever the mesh size, and elements
         // shared by two chunks are contracted once in each.  The chunks run back to back on the
         // stream (each chunk's offsets are written after the previous chunk's kernels, in stream order).
         const i64 E = m->E, N = m->N;
-        const i64 per_pair = 16 * i64(sizeof(T));
+        const int nn = m->nn;                          // values of a pair block: nn * nn
+        const i64 per_pair = nn * nn * i64(sizeof(T));
         PairPlan own;
         if (!plan || plan->per_pair != per_pair) {
             std::vector<i64> nb_off(size_t(E + 1));
@@ -1747,11 +1851,17 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
             d_order.alloc(plan->order_val.size());
             sort_pairs_u64(k_in.p, k_out.p, v_in.p, d_order.p, i64(plan->order_val.size()), s);
         }
-        DevBuf<T> HL{size_t(E) * 32}, HN{size_t(E) * 32}, pairs;
-        Weights4 w4{};
-        for (int q = 0; q < 4; ++q) w4.w[q] = m->fe.w[q];
-        hipLaunchKernelGGL(k_pair_prep<T>, dim3(blocks_for(E * 16, 256)), dim3(256), 0, s, E, m->D.p, w4, m->group_of.p,
-                           d_groups.p, HL.p, HN.p);
+        const size_t per_element = nn == 4 ? 32 : PAIR8_H;
+        DevBuf<T> HL{size_t(E) * per_element}, HN{size_t(E) * per_element}, pairs;
+        if (nn == 4) {
+            Weights4 w4{};
+            for (int q = 0; q < 4; ++q) w4.w[q] = m->fe.w[q];
+            hipLaunchKernelGGL(k_pair_prep<T>, dim3(blocks_for(E * 16, 256)), dim3(256), 0, s, E, m->D.p, w4, m->group_of.p,
+                               d_groups.p, HL.p, HN.p);
+        } else if constexpr (F64) {
+            hipLaunchKernelGGL(k_pair8_prep, dim3(blocks_for(E * PAIR8_ROWS * 8, 256)), dim3(256), 0, s, E, m->D.p, m->fe,
+                               m->group_of.p, d_groups.p, HL.p, HN.p);
+        }
         PairArgs<T> pr{};
         pr.nb_off = m->nb_off.p; pr.nb_ids = m->nb_ids.p; pr.group_of = m->group_of.p;
         pr.groups = d_groups.p; pr.xq = m->xq.p; pr.HL = HL.p; pr.HN = HN.p; pr.el_min = el_min.p;
@@ -1761,7 +1871,11 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
             const unsigned pb = unsigned(std::min<i64>((count + 3) / 4, 16384));
             pr.count = count;
             if constexpr (F64) {
-                if (poly == 1) hipLaunchKernelGGL(k_pairs_mfma<1>, dim3(pb), dim3(256), 0, s, pr);
+                if (nn == 8) {
+                    if (poly == 1) hipLaunchKernelGGL(k_pairs8_mfma<1>, dim3(pb), dim3(256), 0, s, pr);
+                    else if (poly == 2) hipLaunchKernelGGL(k_pairs8_mfma<2>, dim3(pb), dim3(256), 0, s, pr);
+                    else hipLaunchKernelGGL(k_pairs8_mfma<0>, dim3(pb), dim3(256), 0, s, pr);
+                } else if (poly == 1) hipLaunchKernelGGL(k_pairs_mfma<1>, dim3(pb), dim3(256), 0, s, pr);
                 else if (poly == 2) hipLaunchKernelGGL(k_pairs_mfma<2>, dim3(pb), dim3(256), 0, s, pr);
                 else hipLaunchKernelGGL(k_pairs_mfma<0>, dim3(pb), dim3(256), 0, s, pr);
             } else {
@@ -1776,21 +1890,22 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
             if (all_pairs > 0) {
                 hipLaunchKernelGGL(k_padded_slots, dim3(blocks_for(E, 256)), dim3(256), 0, s, E, m->nb_off.p, d_eoff.p);
                 exclusive_scan_i64(d_eoff.p, E, s);
-                pairs.alloc(size_t(all_pairs) * 16);
-                pr.list = d_order.p; pr.eoff = d_eoff.p; pr.pairs = pairs.p; pr.plane = all_pairs * 4;
+                pairs.alloc(size_t(all_pairs) * size_t(nn * nn));
+                pr.list = d_order.p; pr.eoff = d_eoff.p; pr.pairs = pairs.p; pr.plane = all_pairs * nn;
                 contract(E);
                 if constexpr (F64) ca.pairs = pairs.p; else ca.pairs32 = pairs.p;
-                ca.plane = all_pairs * 4;
+                ca.plane = all_pairs * nn;
                 ca.eoff = d_eoff.p;
             }
-            launch_assemble<1, 4, 4, T>(ca, injective, lds, N, s, m->ctx->assembly_threads);
+            if (nn == 4) launch_assemble<1, 4, 4, T>(ca, injective, lds, N, s, m->ctx->assembly_threads);
+            else launch_assemble<1, 8, 9, T>(ca, injective, lds, N, s, m->ctx->assembly_threads);
             NLF_HIP(hipGetLastError());
         } else {
             DevBuf<i64> d_eoff{size_t(E)}, d_cofs;
             DevBuf<i32> d_list;
             upload(d_list, plan->list.data(), plan->list.size(), s);
             upload(d_cofs, plan->cofs.data(), plan->cofs.size(), s);
-            if (plan->max_total > 0) pairs.alloc(size_t(plan->max_total) * 16);
+            if (plan->max_total > 0) pairs.alloc(size_t(plan->max_total) * size_t(nn * nn));
             pr.eoff = d_eoff.p;
             for (const PairChunk& c : plan->chunks) {
                 AssemblyArgs ca = aa;
@@ -1799,13 +1914,14 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
                 if (count > 0 && c.total > 0) {
                     hipLaunchKernelGGL(k_scatter_offsets, dim3(blocks_for(count, 256)), dim3(256), 0, s, count,
                                        d_list.p + c.lbeg, d_cofs.p + c.lbeg, d_eoff.p);
-                    pr.list = d_order.p + c.lbeg; pr.pairs = pairs.p; pr.plane = c.total * 4;
+                    pr.list = d_order.p + c.lbeg; pr.pairs = pairs.p; pr.plane = c.total * nn;
                     contract(count);
                     if constexpr (F64) ca.pairs = pairs.p; else ca.pairs32 = pairs.p;
-                    ca.plane = c.total * 4;
+                    ca.plane = c.total * nn;
                     ca.eoff = d_eoff.p;
                 }
-                launch_assemble<1, 4, 4, T>(ca, injective, lds, c.n1 - c.n0, s, m->ctx->assembly_threads);
+                if (nn == 4) launch_assemble<1, 4, 4, T>(ca, injective, lds, c.n1 - c.n0, s, m->ctx->assembly_threads);
+                else launch_assemble<1, 8, 9, T>(ca, injective, lds, c.n1 - c.n0, s, m->ctx->assembly_threads);
                 NLF_HIP(hipGetLastError());
             }
             NLF_HIP(hipStreamSynchronize(s));          // before the chunk offsets and lists are released
@@ -1955,9 +2071,9 @@ int nlf_assemble_ex(nlf_mesh m, int physics, const nlf_model* models, const void
         DevBuf<int> overflow{1};
         NLF_HIP(hipMemsetAsync(overflow.p, 0, sizeof(int), s));
         pa.cnt = mat->outer.p; pa.bcnt = mat->b_outer.p; pa.overflow = overflow.p;
-        // thermal Q4 nonlocal assembly takes the MFMA pair path: its chunk plan needs the neighbour
+        // thermal nonlocal assembly takes the MFMA pair path: its chunk plan needs the neighbour
         // offsets on the host and is computed while pass 0 of the pattern runs
-        const bool pairs_path = physics == 0 && m->nn == 4 && any_nonlocal && !only_local && m->ctx->assembly_pairs != 0;
+        const bool pairs_path = physics == 0 && any_nonlocal && !only_local && m->ctx->assembly_pairs != 0;
         PairPlan plan;
         // no nonlocal group: the columns of a node are the nodes of its own elements (k_pattern_local)
         bool local_done = false;
@@ -2017,7 +2133,7 @@ int nlf_assemble_ex(nlf_mesh m, int physics, const nlf_model* models, const void
             }
             hipLaunchKernelGGL(k_pattern<0>, dim3(unsigned(m->N)), dim3(pth), lds_bitmap, s, pa);
             NLF_HIP(hipGetLastError());
-            if (pairs_path) plan = plan_pairs(m, nb_off_h, 16 * i64(sizeof(double)));
+            if (pairs_path) plan = plan_pairs(m, nb_off_h, m->nn * m->nn * i64(sizeof(double)));
             int ovf = 0;
             download(&ovf, overflow.p, 1, s);
             NLF_CHECK(!ovf, NLF_ERR_UNSUPPORTED, "column node ids of a row span more than 393k ids (renumber the mesh)");
