@@ -61,8 +61,12 @@ __device__ __forceinline__ Acc block_sum(Acc v, Acc* sh) {
 // Columns are absolute (cols) or, when off16 is given, 16-bit offsets from the row (col = r + off):
 // 10 instead of 12 bytes per FP64 nonzero.  Each lane keeps four (value, column) pairs and then
 // four x gathers in flight.
-template<class T>
-__device__ __forceinline__ T stream_load(const T* p, bool nt) { return nt ? __builtin_nontemporal_load(p) : *p; }
+// (a template: with a bool argument the two loads are merged into a plain one before it is known)
+template<bool NT, class T>
+__device__ __forceinline__ T stream_load(const T* p) {
+    if constexpr (NT) return __builtin_nontemporal_load(p);
+    else return *p;
+}
 
 // Split values: hi (FP32) + lo * 2^-16 ulp(hi), lo a 16-bit integer (40 significand bits).
 __device__ __forceinline__ double split_value(float h, int16_t l) {
@@ -71,7 +75,8 @@ __device__ __forceinline__ double split_value(float h, int16_t l) {
     return double(h) + double(l) * __longlong_as_double(static_cast<long long>(e + 857u) << 52);
 }
 
-// SPLIT (V = float): each value is split_value(val[p], lo[p]), summed in Acc.
+// SPLIT (V = float): each value is split_value(val[p], lo[p]), summed in Acc.  NT (a variant for
+// timing, per-nonzero offsets): the matrix stream is loaded non-temporally.
 template<int LPR, class V, class X, class Acc, bool DOT, bool XCD = false, int UNROLL = 4, bool NT = false,
          bool SPLIT = false>
 __global__ __launch_bounds__(SPMV_THREADS) void k_spmv(i64 rows, const i64* __restrict__ outer, const i32* __restrict__ cols,
@@ -97,7 +102,6 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv(i64 rows, const i64* __re
             // offsets of row r: off16[ob + p] (ob = 0 for per-nonzero offsets; with the row-pattern
             // dictionary ob moves p into the row's shared pattern, which stays in L2)
             const i64 ob = pstart ? pstart[r] : 0;
-            const bool nt_off = NT && !pstart;
             i64 p = b + sub;
             for (; p + (UNROLL - 1) * LPR < e; p += UNROLL * LPR) {
                 i64 c[UNROLL];
@@ -105,9 +109,9 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv(i64 rows, const i64* __re
                 int16_t vl[UNROLL];
 #pragma unroll
                 for (int t = 0; t < UNROLL; ++t) {
-                    c[t] = off16 ? r + i64(stream_load(off16 + ob + p + t * LPR, nt_off))
-                                 : i64(stream_load(cols + p + t * LPR, NT));
-                    v[t] = stream_load(val + p + t * LPR, NT);
+                    c[t] = off16 ? r + i64(stream_load<NT>(off16 + ob + p + t * LPR))
+                                 : i64(stream_load<NT>(cols + p + t * LPR));
+                    v[t] = stream_load<NT>(val + p + t * LPR);
                     if constexpr (SPLIT) vl[t] = lo[p + t * LPR];
                 }
                 X xv[UNROLL];
@@ -120,9 +124,9 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv(i64 rows, const i64* __re
                 }
             }
             for (; p < e; p += LPR) {
-                const i64 c = off16 ? r + i64(stream_load(off16 + ob + p, nt_off)) : i64(stream_load(cols + p, NT));
-                if constexpr (SPLIT) acc += Acc(split_value(stream_load(val + p, NT), lo[p])) * Acc(x[c]);
-                else acc += Acc(stream_load(val + p, NT)) * Acc(x[c]);
+                const i64 c = off16 ? r + i64(stream_load<NT>(off16 + ob + p)) : i64(stream_load<NT>(cols + p));
+                if constexpr (SPLIT) acc += Acc(split_value(stream_load<NT>(val + p), lo[p])) * Acc(x[c]);
+                else acc += Acc(stream_load<NT>(val + p)) * Acc(x[c]);
             }
         }
         for (int o = LPR / 2; o > 0; o >>= 1) acc += shfl_down_t(acc, o);   // lane sub==0 of each group holds the sum
@@ -150,7 +154,9 @@ template<> struct Pair<float> { typedef float T __attribute__((ext_vector_type(2
 // XCD: each block takes a contiguous chunk of row groups, and the blocks that the hardware deals
 // round-robin to one XCD take adjacent chunks, so each XCD's L2 holds the x window of its own
 // eighth of the rows (without it, concurrently active rows span the whole matrix on every XCD).
-template<int LPR, class V, class X, class Acc, bool DOT, bool SPLIT = false, bool XCD = false, int PF = SPMV_PAIRS_IN_FLIGHT>
+// NT: the values are loaded non-temporally (the offsets are not: a row-pattern dictionary is read again).
+template<int LPR, class V, class X, class Acc, bool DOT, bool SPLIT = false, bool XCD = false, int PF = SPMV_PAIRS_IN_FLIGHT,
+         bool NT = false>
 __global__ __launch_bounds__(SPMV_THREADS) void k_spmv2(i64 rows, const i64* __restrict__ outer,
                                                         const int16_t* __restrict__ off, const i64* __restrict__ pstart,
                                                         const V* __restrict__ val, const int16_t* __restrict__ lo,
@@ -194,7 +200,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv2(i64 rows, const i64* __r
                 int cw[PF], lw[PF];
 #pragma unroll
                 for (int u = 0; u < PF; ++u) {
-                    v[u] = *reinterpret_cast<const V2*>(val + p + 2 * LPR * u);
+                    v[u] = stream_load<NT>(reinterpret_cast<const V2*>(val + p + 2 * LPR * u));
                     cw[u] = *reinterpret_cast<const int*>(o + p + 2 * LPR * u);
                     lw[u] = lo_pair(p + 2 * LPR * u);
                 }
@@ -211,7 +217,7 @@ __global__ __launch_bounds__(SPMV_THREADS) void k_spmv2(i64 rows, const i64* __r
                 }
             }
             for (; p + 1 < e; p += 2 * LPR) {
-                const V2 v0 = *reinterpret_cast<const V2*>(val + p);
+                const V2 v0 = stream_load<NT>(reinterpret_cast<const V2*>(val + p));
                 const int c0 = *reinterpret_cast<const int*>(o + p);
                 const int l0 = lo_pair(p);
                 acc += value(v0.x, int16_t(l0 & 0xffff)) * Acc(x[r + int16_t(c0 & 0xffff)]);
@@ -859,11 +865,11 @@ unsigned spmv_blocks(int lpr, i64 rows) {
 // lo: 16-bit remainders of split values (V = float, NLF_MODE_SPLIT), else null.  With 16-bit
 // offsets (per nonzero or the dictionary) the pair kernel k_spmv2 runs unless pairs = false; xcd
 // selects its XCD-contiguous row chunks (the one-nonzero-per-load kernel's XCD numbering when
-// pairs = false).
+// pairs = false).  nt: the pair kernel's values (not split ones) bypass the caches.
 template<class V, class X, class Acc, bool DOT>
 void launch_spmv(int lpr, i64 rows, const i64* outer, SpmvCols cs, const V* val, const X* x, X* y,
                  double* partial, const CGState* st, hipStream_t s, bool xcd = false, const int16_t* lo = nullptr,
-                 bool pairs = true, int pf = SPMV_PAIRS_IN_FLIGHT) {
+                 bool pairs = true, int pf = SPMV_PAIRS_IN_FLIGHT, bool nt = false) {
     const i32* cols = cs.cols;
     const int16_t* off16 = cs.off;
     const i64* pstart = cs.pstart;
@@ -906,6 +912,10 @@ void launch_spmv(int lpr, i64 rows, const i64* outer, SpmvCols cs, const V* val,
         if (pf == 2)                                                                                               \
             hipLaunchKernelGGL((k_spmv2<L, V, X, Acc, DOT, false, false, 2>), dim3(blocks), dim3(SPMV_THREADS), 0, s, rows, \
                                outer, off16, pstart, val, static_cast<const int16_t*>(nullptr), x, y, partial, st);   \
+        else if (nt)                                                                                               \
+            hipLaunchKernelGGL((k_spmv2<L, V, X, Acc, DOT, false, false, SPMV_PAIRS_IN_FLIGHT, true>), dim3(blocks),  \
+                               dim3(SPMV_THREADS), 0, s, rows, outer, off16, pstart, val,                           \
+                               static_cast<const int16_t*>(nullptr), x, y, partial, st);                           \
         else                                                                                                       \
             hipLaunchKernelGGL((k_spmv2<L, V, X, Acc, DOT, false, false, SPMV_PAIRS_IN_FLIGHT>), dim3(blocks),        \
                                dim3(SPMV_THREADS), 0, s, rows, outer, off16, pstart, val,                           \
@@ -1068,6 +1078,12 @@ void residual64(const nlf_matrix_s* a, const double* x, const double* b, double*
 constexpr unsigned CG_BLOCKS = 1024;
 constexpr i64 SYMV_REDUCE_BLOCKS = 2048;
 
+// Above this size the full storage's values bypass the caches in a solve with sweeps: the last-level cache
+// holds 256 MB, a smaller matrix is read from it again, a larger one only drives out the factor that the
+// sweeps read next, whose loads' latency bounds them.  Q8 sheets, us per iteration without / with: 31 000
+// rows (112 MB) 259 / 271, 44 000 (204 MB) 352 / 363, 59 000 (352 MB) 550 / 447, 121 000 (1264 MB) 978 / 809.
+constexpr i64 SPMV_NT_BYTES = i64(256) << 20;
+
 // Preconditioned CG on device vectors (conjugate_gradient::solve).  Vectors of type X, matrix values V.
 // The work memory (CGWork) is allocated by the object, or given by the caller (no allocation then;
 // `timed` = false also records no HIP events).
@@ -1090,12 +1106,14 @@ struct CG {
     bool timed = true;
     bool indefinite = false;            // a bordered (Neumann) system: negative curvature allowed
     const nlf_matrix_s* sym = nullptr;  // products from the symmetric storage (symv_prepare done)
+    bool nt = false;                    // the matrix values bypass the caches (see SPMV_NT_BYTES)
     KernelTimer timer;
 
     CG(hipStream_t s_, i64 n_, i64 nnz, const i64* o, const i32* c, const V* v, const nlf_precond_s* P_,
        void* work = nullptr)
         : s(s_), n(n_), outer(o), cols(c), val(v), P(P_) {
         cs.cols = c;
+        nt = P && P->chunked && nnz * i64(sizeof(V)) > SPMV_NT_BYTES;
         lpr = pick_lpr(double(nnz) / double(std::max<i64>(n, 1)));
         if (!work) {
             own.alloc(CGWork::bytes<X>(n));
@@ -1240,7 +1258,7 @@ struct CG {
         // z = A p with the partials of p.z
         if (sample) timer.start(0, s);
         if (sym) launch_symv<true>(sym, p, z, part1, st, s, sblocks, std::is_same_v<V, double> ? SYM_FP64 : lo ? SYM_SPLIT : SYM_FP32);
-        else launch_spmv<V, X, double, true>(lpr, n, outer, cs, val, p, z, part1, st, s, false, lo);
+        else launch_spmv<V, X, double, true>(lpr, n, outer, cs, val, p, z, part1, st, s, false, lo, true, SPMV_PAIRS_IN_FLIGHT, nt);
         if (sample) timer.stop(0, s);
         if (!P || P->kind == NLF_PRECOND_IDENTITY || jacobi()) {
             // x += a p ; r -= a z ; z = M r ; partial r.z  (fused)
