@@ -479,99 +479,132 @@ __global__ __launch_bounds__(MP_THREADS) void k_lf_out_back(i64 n, const double*
 }
 
 // gradients of W_s, W_m; dL/dh_in (direct part) = W_s^T gh, dL/dm = W_m^T gh.
-__global__ __launch_bounds__(MP_THREADS) void k_lf_layer_back1(i64 n, const float* __restrict__ gh, const float* __restrict__ hin,
-                                                               const float* __restrict__ m, const float* __restrict__ wl,
-                                                               float* __restrict__ gdir, float* __restrict__ gm,
-                                                               float* __restrict__ gpart_layer) {
-    __shared__ float Ws[MP_H][MP_H + 1], Wm[MP_H][MP_H + 1];
-    __shared__ float red[MP_NODES][MP_H + 1];
-    for (int i = threadIdx.x; i < MP_H * MP_H; i += blockDim.x) {
-        Ws[i / MP_H][i % MP_H] = wl[P_WS + i];
-        Wm[i / MP_H][i % MP_H] = wl[P_WM + i];
-    }
-    __syncthreads();
+// Latency of the loads and of LDS bounds it: 16 nodes per block, the thread's weight columns in registers, a
+// node's vectors read back from LDS four values at a time, and the blocks' sums formed with 4 barriers in all.
+// 128 x 128 nodes: 12 us (28 with 8 nodes, a shuffle per broadcast value and 128 barriers).
+constexpr int BACK1_THREADS = 512, BACK1_NODES = BACK1_THREADS / MP_H;
+__global__ __launch_bounds__(BACK1_THREADS) void k_lf_layer_back1(i64 n, const float* __restrict__ gh, const float* __restrict__ hin,
+                                                                  const float* __restrict__ m, const float* __restrict__ wl,
+                                                                  float* __restrict__ gdir, float* __restrict__ gm,
+                                                                  float* __restrict__ gpart_layer) {
+    __shared__ __align__(16) float vec[3][BACK1_NODES][MP_H];
+    __shared__ float red[BACK1_THREADS / 64][MP_H * (MP_H + 1)];
     const int c = threadIdx.x % MP_H, slot = threadIdx.x / MP_H;
-    float gws[MP_H], gwm[MP_H];
+    float ws[MP_H], wm[MP_H], gws[MP_H], gwm[MP_H];
 #pragma unroll
-    for (int k = 0; k < MP_H; ++k) { gws[k] = 0.0f; gwm[k] = 0.0f; }
-    const i64 nn = (n + MP_NODES - 1) / MP_NODES * MP_NODES;
-    for (i64 u0 = i64(blockIdx.x) * MP_NODES; u0 < nn; u0 += i64(gridDim.x) * MP_NODES) {
-        const i64 u = u0 + slot;
-        const bool live = u < n;
-        float da = 0.0f, hu = 0.0f, mu = 0.0f;
-        if (live) {
+    for (int k = 0; k < MP_H; ++k) {
+        ws[k] = wl[P_WS + k * MP_H + c];
+        wm[k] = wl[P_WM + k * MP_H + c];
+        gws[k] = 0.0f;
+        gwm[k] = 0.0f;
+    }
+    float da = 0.0f, hu = 0.0f, mu = 0.0f;
+    auto load = [&](i64 u) {
+        da = hu = mu = 0.0f;
+        if (u < n) {
             da = gh[u * MP_H + c];
             hu = hin[u * MP_H + c];
             mu = m[u * MP_H + c];
         }
+    };
+    load(i64(blockIdx.x) * BACK1_NODES + slot);
+    // A node's 32 threads are half a wave, whose LDS accesses are carried out in order: no barrier here.
+    for (i64 u0 = i64(blockIdx.x) * BACK1_NODES; u0 < n; u0 += i64(gridDim.x) * BACK1_NODES) {
+        const i64 u = u0 + slot;
+        const float d = da;
+        vec[0][slot][c] = hu;
+        vec[1][slot][c] = mu;
+        vec[2][slot][c] = da;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        load(u + i64(gridDim.x) * BACK1_NODES);
         float dh = 0.0f, dm = 0.0f;
 #pragma unroll
-        for (int k = 0; k < MP_H; ++k) {
-            const float hk = __shfl(hu, k, MP_H), mk = __shfl(mu, k, MP_H), dk = __shfl(da, k, MP_H);
-            gws[k] += da * hk;                  // dW_s[c][k]
-            gwm[k] += da * mk;                  // dW_m[c][k]
-            dh += Ws[k][c] * dk;                // (W_s^T da)_c
-            dm += Wm[k][c] * dk;                // (W_m^T da)_c
+        for (int k = 0; k < MP_H; k += 4) {
+            const float4 h4 = *reinterpret_cast<const float4*>(&vec[0][slot][k]), m4 = *reinterpret_cast<const float4*>(&vec[1][slot][k]),
+                         d4 = *reinterpret_cast<const float4*>(&vec[2][slot][k]);
+            const float hk[4] = {h4.x, h4.y, h4.z, h4.w}, mk[4] = {m4.x, m4.y, m4.z, m4.w}, dk[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                gws[k + j] += d * hk[j];                  // dW_s[c][k]
+                gwm[k + j] += d * mk[j];                  // dW_m[c][k]
+                dh += ws[k + j] * dk[j];                  // (W_s^T da)_c
+                dm += wm[k + j] * dk[j];                  // (W_m^T da)_c
+            }
         }
-        if (live) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (u < n) {
             gdir[u * MP_H + c] = dh;
             gm[u * MP_H + c] = dm;
         }
     }
     float* row = gpart_layer + i64(blockIdx.x) * NPARAM;
-    for (int k = 0; k < MP_H; ++k) {
-        red[slot][c] = gws[k];
-        __syncthreads();
-        if (slot == 0) {
-            float t = 0.0f;
-            for (int q = 0; q < MP_NODES; ++q) t += red[q][c];
-            row[P_WS + c * MP_H + k] = t;
+    auto sum = [&](const float (&g)[MP_H], int first) {
+#pragma unroll
+        for (int k = 0; k < MP_H; ++k) {
+            const float t = g[k] + __shfl_xor(g[k], MP_H);           // the wave's two nodes
+            if (threadIdx.x % 64 < MP_H) red[threadIdx.x / 64][c * (MP_H + 1) + k] = t;
         }
         __syncthreads();
-        red[slot][c] = gwm[k];
-        __syncthreads();
-        if (slot == 0) {
+        for (int i = threadIdx.x; i < MP_H * MP_H; i += BACK1_THREADS) {
             float t = 0.0f;
-            for (int q = 0; q < MP_NODES; ++q) t += red[q][c];
-            row[P_WM + c * MP_H + k] = t;
+#pragma unroll
+            for (int q = 0; q < BACK1_THREADS / 64; ++q) t += red[q][i + i / MP_H];
+            row[first + i] = t;
         }
         __syncthreads();
-    }
+    };
+    sum(gws, P_WS);
+    sum(gwm, P_WM);
 }
 
 // dL/dh_in[v] = direct + sum_{u in N(v)} g_uv (.) dm_u ;  dW_e[c][f] += sum dm_u[c] h_v[c] f_uv[f]
-__global__ __launch_bounds__(MP_THREADS) void k_lf_layer_back2(i64 n, const i64* __restrict__ outer, const i32* __restrict__ cols,
-                                                               const float4* __restrict__ feat, const float* __restrict__ wl,
-                                                               const float* __restrict__ gm, const float* __restrict__ hin,
-                                                               const float* __restrict__ gdir, float* __restrict__ ghin,
-                                                               float* __restrict__ gpart_layer) {
-    __shared__ float red[MP_NODES][MP_H + 1];
+// Bound by the chain of loads of a node's row (bounds, columns, the neighbours' dm): 32 nodes per block, and a
+// row's loads in flight together, nine at a time, which is a row of a grid of quadrilaterals.
+// 128 x 128 nodes: 15 us (25 with 8 nodes per block and a neighbour at a time).
+constexpr int BACK2_THREADS = 1024, BACK2_NODES = BACK2_THREADS / MP_H, BACK2_ROW = 9;
+__global__ __launch_bounds__(BACK2_THREADS) void k_lf_layer_back2(i64 n, const i64* __restrict__ outer, const i32* __restrict__ cols,
+                                                                  const float4* __restrict__ feat, const float* __restrict__ wl,
+                                                                  const float* __restrict__ gm, const float* __restrict__ hin,
+                                                                  const float* __restrict__ gdir, float* __restrict__ ghin,
+                                                                  float* __restrict__ gpart_layer) {
+    __shared__ float red[MP_F][BACK2_NODES][MP_H + 1];
     const int c = threadIdx.x % MP_H, slot = threadIdx.x / MP_H;
     const float e0 = wl[P_WE + c * MP_F + 0], e1 = wl[P_WE + c * MP_F + 1], e2 = wl[P_WE + c * MP_F + 2],
                 e3 = wl[P_WE + c * MP_F + 3];
     float ge[MP_F] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (i64 v = i64(blockIdx.x) * MP_NODES + slot; v < n; v += i64(gridDim.x) * MP_NODES) {
+    for (i64 v = i64(blockIdx.x) * BACK2_NODES + slot; v < n; v += i64(gridDim.x) * BACK2_NODES) {
+        const i64 p0 = outer[v], p1 = outer[v + 1];
         float acc = gdir[v * MP_H + c];
         const float hv = hin[v * MP_H + c];
-        for (i64 p = outer[v]; p < outer[v + 1]; ++p) {
-            const float4 f = feat[p];
-            const float dmu = gm[i64(cols[p]) * MP_H + c];
-            acc += (e0 * f.x + e1 * f.y + e2 * f.z + e3 * f.w) * dmu;
-            const float t = dmu * hv;
-            ge[0] += t * f.x; ge[1] += t * f.y; ge[2] += t * f.z; ge[3] += t * f.w;
+        for (i64 p = p0; p < p1; p += BACK2_ROW) {
+            i32 u[BACK2_ROW];
+            float dmu[BACK2_ROW];
+#pragma unroll
+            for (int j = 0; j < BACK2_ROW; ++j) u[j] = cols[p + j < p1 ? p + j : p1 - 1];
+#pragma unroll
+            for (int j = 0; j < BACK2_ROW; ++j) dmu[j] = gm[i64(u[j]) * MP_H + c];
+#pragma unroll
+            for (int j = 0; j < BACK2_ROW; ++j) {
+                if (p + j >= p1) break;
+                const float4 f = feat[p + j];
+                acc += (e0 * f.x + e1 * f.y + e2 * f.z + e3 * f.w) * dmu[j];
+                const float t = dmu[j] * hv;
+                ge[0] += t * f.x; ge[1] += t * f.y; ge[2] += t * f.z; ge[3] += t * f.w;
+            }
         }
         ghin[v * MP_H + c] = acc;
     }
     float* row = gpart_layer + i64(blockIdx.x) * NPARAM;
-    for (int f = 0; f < MP_F; ++f) {
-        red[slot][c] = ge[f];
-        __syncthreads();
-        if (slot == 0) {
-            float t = 0.0f;
-            for (int q = 0; q < MP_NODES; ++q) t += red[q][c];
-            row[P_WE + c * MP_F + f] = t;
-        }
-        __syncthreads();
+#pragma unroll
+    for (int f = 0; f < MP_F; ++f) red[f][slot][c] = ge[f];
+    __syncthreads();
+    if (threadIdx.x < MP_H * MP_F) {
+        const int f = threadIdx.x / MP_H;
+        float t = 0.0f;
+        for (int q = 0; q < BACK2_NODES; ++q) t += red[f][q][c];
+        row[P_WE + c * MP_F + f] = t;
     }
 }
 
@@ -591,12 +624,24 @@ __global__ __launch_bounds__(MP_THREADS) void k_lf_input_back(i64 n, const float
     }
 }
 
-__global__ void k_lf_reduce(const float* __restrict__ gpart, int nb, float* __restrict__ grad) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= NPARAM) return;
+// grad[i] = the sum of the blocks' partials, in FP64.  A thread's loads follow each other, so a parameter's rows
+// are dealt to 16 threads: 7 MB of partials in 5 us (64 with a thread per parameter).
+constexpr int REDUCE_COLS = 64, REDUCE_PARTS = 16;
+__global__ __launch_bounds__(REDUCE_COLS * REDUCE_PARTS) void k_lf_reduce(const float* __restrict__ gpart, int nb,
+                                                                         float* __restrict__ grad) {
+    __shared__ double red[REDUCE_PARTS][REDUCE_COLS];
+    const int c = threadIdx.x % REDUCE_COLS, part = threadIdx.x / REDUCE_COLS, i = blockIdx.x * REDUCE_COLS + c;
     double t = 0.0;
-    for (int b = 0; b < nb; ++b) t += gpart[i64(b) * NPARAM + i];
-    grad[i] = float(t);
+    if (i < NPARAM) {
+#pragma unroll 8
+        for (int b = part; b < nb; b += REDUCE_PARTS) t += gpart[i64(b) * NPARAM + i];
+    }
+    red[part][c] = t;
+    __syncthreads();
+    if (part == 0 && i < NPARAM) {
+        for (int q = 1; q < REDUCE_PARTS; ++q) t += red[q][c];
+        grad[i] = float(t);
+    }
 }
 
 // Adam (Kingma & Ba 2015) with bias correction.
@@ -1400,14 +1445,14 @@ double learned_loss_grad(LearnedGraph& g, const float* w, nlf_matrix A, const do
     for (int l = MP_L - 1; l >= 0; --l) {
         const float* wl = w + P_LAYER0 + l * P_LAYER_SIZE;
         float* gp = g.gpart.p + P_LAYER0 + l * P_LAYER_SIZE;
-        hipLaunchKernelGGL(k_lf_layer_back1, dim3(gb), dim3(MP_THREADS), 0, s, n, gcur, g.h[l].p, g.m[l].p, wl, g.gdir.p,
+        hipLaunchKernelGGL(k_lf_layer_back1, dim3(gb), dim3(BACK1_THREADS), 0, s, n, gcur, g.h[l].p, g.m[l].p, wl, g.gdir.p,
                            g.gm.p, gp);
-        hipLaunchKernelGGL(k_lf_layer_back2, dim3(gb), dim3(MP_THREADS), 0, s, n, g.outer.p, g.cols.p, feat, wl, g.gm.p,
+        hipLaunchKernelGGL(k_lf_layer_back2, dim3(gb), dim3(BACK2_THREADS), 0, s, n, g.outer.p, g.cols.p, feat, wl, g.gm.p,
                            g.h[l].p, g.gdir.p, gnext, gp);
         std::swap(gcur, gnext);
     }
     hipLaunchKernelGGL(k_lf_input_back, dim3(gb), dim3(MP_THREADS), 0, s, n, gcur, g.x.p, g.gpart.p);
-    hipLaunchKernelGGL(k_lf_reduce, dim3((NPARAM + 255) / 256), dim3(256), 0, s, g.gpart.p, int(gb), g.grad.p);
+    hipLaunchKernelGGL(k_lf_reduce, dim3((NPARAM + REDUCE_COLS - 1) / REDUCE_COLS), dim3(REDUCE_COLS * REDUCE_PARTS), 0, s, g.gpart.p, int(gb), g.grad.p);
     NLF_HIP(hipGetLastError());
     double h[2];
     download(h, sums.p, 2, s);
