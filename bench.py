@@ -173,10 +173,9 @@ def cpu_baseline(problem, plain_iterations, check, cg_iterations):
 
 def bench_batch(args):
     """64 uneven thermal instances (Q4 sides 32-256 log-uniform, r in [0.02, 0.1], p1 in [0.2, 1],
-    lambda in [0.5, 2], seed 3): one batched assembly + lockstep mixed-precision Jacobi-PCG under a
-    captured hipGraph, against 64 sequential plain FP64 ILLT-CG solves of the same instances.  (The
-    batch's ILLT option cuts the iterations 2.7x here but its single-workgroup sweep runs the 64
-    instances' levels one after another, 22 ms per iteration: slower than Jacobi on this batch.)"""
+    lambda in [0.5, 2], seed 3): one batched assembly + lockstep mixed-precision PCG (ILLT, or Jacobi with
+    --batch-precond) under a captured hipGraph, against 64 sequential plain FP64 ILLT-CG solves of the same
+    instances."""
     print(json.dumps(batch64_record(args.tol, args.steps, args.warmup, args.batch_precond)), flush=True)
 
 

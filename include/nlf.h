@@ -158,9 +158,10 @@ int         nlf_ctx_synchronize(nlf_ctx ctx);
 #define NLF_OPT_PATTERN_THREADS  4   /* threads per node workgroup of the pattern build: 64, 128 (default), 256 */
 #define NLF_OPT_PAIR_BUDGET_MIB  5   /* MiB for the MFMA pair blocks of one assembly pass; 0 (default): 8 GiB;
                                         a mesh whose blocks do not fit is assembled in node chunks */
-#define NLF_OPT_SPMV_SYMMETRIC   6   /* 1 (default): the FP64 products of CG, flexible CG and nlf_spmv read the upper
-                                        triangle once (the reference's symmetric product), from a slice layout built
-                                        on the first solve; 0: the full (both-triangle) storage */
+#define NLF_OPT_SPMV_SYMMETRIC   6   /* 1 (default): the products of CG, flexible CG and batches (FP64, FP32 or split
+                                        values) and of nlf_spmv read the upper triangle once (the reference's
+                                        symmetric product), from a slice layout built on the first solve; 0: the
+                                        full (both-triangle) storage */
 int         nlf_ctx_set_option(nlf_ctx ctx, int option, int value);
 void*       nlf_ctx_stream(nlf_ctx ctx);
 
@@ -321,8 +322,7 @@ int nlf_precond_info(nlf_precond p, int* ok, double* shift, int* fw_levels, int*
 int nlf_precond_sweep_info(nlf_precond p, int32_t out[8]);
 /* No reference counterpart: the independent diagonal blocks an ILLT found in its matrix (contiguous
  * row ranges with no entry between them, such as a batch's instances, of at least 1024 rows each),
- * each factored by a workgroup of its own, side by side, and swept in chunks of its own; 1 for a
- * connected matrix. */
+ * factored and swept side by side in chunks of their own; 1 for a connected matrix. */
 int nlf_precond_blocks(nlf_precond p, int32_t* blocks);
 int nlf_precond_apply(nlf_precond p, const double* r_dev, double* z_dev);
 int nlf_precond_export_factor(nlf_precond p, double* values, double* scale);

@@ -408,8 +408,8 @@ class preconditioner:
         return {"forward": dict(zip(keys, out[0:4])), "backward": dict(zip(keys, out[4:8]))}
 
     def blocks(self):
-        """Independent diagonal blocks of an ILLT's matrix, each factored by a workgroup of its own
-        and swept in chunks of its own (nlf_precond_blocks)."""
+        """Independent diagonal blocks of an ILLT's matrix, factored and swept side by side in chunks
+        of their own (nlf_precond_blocks)."""
         out = C.c_int32()
         self.ctx.check(load().nlf_precond_blocks(self.h, C.byref(out)))
         return out.value

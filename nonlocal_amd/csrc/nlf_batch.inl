@@ -1,11 +1,13 @@
 // Batched solves: many independent instances stored as the diagonal blocks of one matrix (instance
 // i owns rows [row_begin[i], row_begin[i+1])), solved by lockstep preconditioned CG with
 // per-instance scalars: Jacobi, or an IC(0) (ILLT) preconditioner of the batch's local matrix, whose
-// factor is block diagonal like the matrix, so one level-scheduled sweep applies every instance's.  Compiled as part of nlf_solver.hip (shares block_sum / shfl helpers).
+// factor is block diagonal like the matrix, so one launch per sweep applies every instance's.  Compiled as
+// part of nlf_solver.hip (shares block_sum / shfl helpers).
 //
 // Every launch covers all instances: a block never straddles two instances, partial dot products
 // are written per block and summed per instance in a fixed order (bitwise reproducible), and a
-// converged instance's blocks skip their work.  The SpMV groups instances by lanes-per-row class
+// converged instance's blocks skip their work.  The product reads the symmetric slice storage
+// (nlf_symv.inl) where that applies; otherwise the SpMV groups instances by lanes-per-row class
 // (one launch per class); the class of an instance comes from its nonzeros per row and a target
 // number of nonzeros per lane, which the autotuner picks by timing the batched SpMV (and caches
 // per batch signature).  G iterations are captured once into a hipGraph and the graph is
@@ -627,7 +629,7 @@ int nlf_batch_autotune(nlf_batch b, const char* cache_path, double* chosen) {
 
 // No reference counterpart.  The preconditioner of the batch's solves: an ILLT built on the batch's local
 // matrix (block diagonal like the batch; same rows), or NULL for Jacobi of the matrix (the default).  An
-// ILLT of a block-diagonal matrix factors and sweeps every instance on a workgroup of its own.
+// ILLT of a block-diagonal matrix factors and sweeps every instance in chunks of its own.
 int nlf_batch_set_preconditioner(nlf_batch bt, nlf_precond p) {
     if (!bt) return NLF_ERR_ARGUMENT;
     return guarded(bt->ctx, [&] {

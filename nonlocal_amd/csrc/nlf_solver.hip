@@ -1,16 +1,18 @@
 // Krylov layer: CSR SpMV, CG (conjugate_gradient.hpp:48-79), Jacobi and ILLT preconditioners
 // (eigen_preconditioner.hpp:50-57), FP32-inner / FP64-refinement mixed mode.
 //
-// SpMV runs on the full (both-triangle) storage so every output row is a gather (no scatter, no
-// atomics, deterministic); LPR lanes cooperate on one row.  CG keeps its scalars on the device in a
-// state block; each iteration is 5 launches (SpMV+dot, alpha, update+precond+dot, beta, p update)
-// with no host synchronisation; the host reads the state every few iterations.
+// The products read the upper triangle from slices (nlf_symv.inl), or the full (both-triangle) storage where
+// that does not apply: every output row is a gather there (no scatter, no atomics, deterministic) and LPR
+// lanes cooperate on one row.  CG keeps its scalars on the device in a state block; an iteration is the
+// product with its dot, the update with the Jacobi preconditioner and its dot (or the two sweeps and their
+// finish) and the p update, which form alpha and beta themselves, with no host synchronisation; the host
+// reads the state every few iterations.
 //
 // ILLT: IC(0) of the local matrix, diagonal scaling s = 1/sqrt|a_ii| and shift retries (our choice:
 // Eigen::IncompleteCholesky is not vendored, so its factor is not reproduced).  Rows are grouped by
-// dependency level (computed once on the host from the pattern).  The factorisation is one persistent
-// 1024-thread workgroup per independent block with a barrier between levels; the triangular sweeps run
-// as a dataflow over chunks of rows (nlf_sweep.inl).
+// dependency level (computed once on the host from the pattern).  The factorisation and the triangular
+// sweeps run as dataflows over chunks of rows (nlf_sweep.inl); with more than 32 dependencies in a row, as one
+// 1024-thread workgroup per independent block with a barrier between levels.
 #include "nlf_internal.hpp"
 
 #include <mutex>
