@@ -9,9 +9,15 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("scale,above", [(0.6, False), (0.7, True)])
-def test_residual_on_both_sides(scale, above):
-    ctx = api.Context()
-    ctx.set_option(A.NLF_OPT_SPMV_SYMMETRIC, 0)
+def test_residual_on_both_sides(gpu_ctx, scale, above):
+    gpu_ctx.set_option(A.NLF_OPT_SPMV_SYMMETRIC, 0)
+    try:
+        _check(gpu_ctx, scale, above)
+    finally:
+        gpu_ctx.set_option(A.NLF_OPT_SPMV_SYMMETRIC, 1)
+
+
+def _check(ctx, scale, above):
     p = configs.cfg1(scale)
     g = api.mesh_2d(p.mesh, ctx)
     api.find_neighbours(g, api._radii(p.models))
