@@ -24,12 +24,11 @@
 // next).  k_sweep_finish empties both buffers after the backward sweep.  Chunks are handed out in order
 // by a ticket, so whoever waits waits for a workgroup that is already running.
 
+#include "nlf_sweep_flow.hpp"
+
 namespace nlf {
 
 constexpr int SWEEP_LEVEL_CAP = 512;     // records of a level before it is split into several
-constexpr int SWEEP_K = 48;              // steps the LDS window holds
-constexpr int SWEEP_R = 48;              // steps the right-hand side ring holds
-constexpr int SWEEP_RB = 16;             // steps the rhs wave stages at a time
 constexpr int SWEEP_EXT = 1024;          // slots of the external values' ring
 constexpr int SWEEP_EXT_STEP = 256;      // most new external values of a step
 constexpr int SWEEP_EXT_REUSE = 256;     // how far back (in values) a step may use an external value again
@@ -40,6 +39,7 @@ constexpr i64 SWEEP_CHUNK_ROWS = 1 << 23;   // most rows of a chunk (32-bit byte
 // first records of coming steps, window, right-hand sides, external values
 constexpr int SWEEP_CTL = 16, SWEEP_IDLE = 64, SWEEP_SP = 320, SWEEP_WIN = 832, SWEEP_RHS = SWEEP_WIN + SWEEP_K * 512, SWEEP_XV = SWEEP_RHS + SWEEP_R * 512,
               SWEEP_LDS = SWEEP_XV + SWEEP_EXT * 8;
+static_assert(SWEEP_SP + 4 * SWEEP_FIRST <= SWEEP_WIN, "the ring of first records lies before the window");
 constexpr int SWEEP_ALL = 1 << 30;       // a helper wave has staged every step
 constexpr int SWEEP_SPIN = 1 << 21;      // reads of a missing value before it is taken as NaN (seconds)
 constexpr unsigned long long SWEEP_EMPTY = 0xfff8dead0badc0deull;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void k_sweep(SweepArgs a, const double* __rest
             for (int u = 0; u < D; ++u) {
                 const int s = s0 + u;
                 while (s >= avail)
-                    avail = min(min(ctl_load(ctl), ctl_load(ctl + 1)), ctl_load(ctl + 3) + SWEEP_K);
+                    avail = min(min(ctl_load(ctl), ctl_load(ctl + 1)), sweep_window_end(ctl_load(ctl + 3)));
                 double x = rs[u * 64];
                 double dv[WE];
 #pragma unroll
@@ -199,10 +199,10 @@ __global__ __launch_bounds__(256) void k_sweep(SweepArgs a, const double* __rest
             for (int u = 0; u < B; ++u) w[u] = y[u] * x[u];
             gather();
             addresses(spc);
-            while (ctl_load(ctl + 2) < s0 + B - SWEEP_R || ctl_load(ctl + 3) < s0 + B - 2 * SWEEP_R) __builtin_amdgcn_s_sleep(1);
+            while (!sweep_rhs_free(s0, ctl_load(ctl + 2), ctl_load(ctl + 3))) __builtin_amdgcn_s_sleep(1);
 #pragma unroll
             for (int u = 0; u < B; ++u) rhs[((s0 + u) % SWEEP_R) * 64 + lane] = w[u];
-            if (lane <= B) reinterpret_cast<u32*>(lds + SWEEP_SP)[(s0 + lane) % (2 * SWEEP_R)] = u32(spa - rec0) * 8;
+            if (lane <= B) reinterpret_cast<u32*>(lds + SWEEP_SP)[(s0 + lane) % SWEEP_FIRST] = u32(spa - rec0) * 8;
             ctl_store(mine, s0 + B >= n ? SWEEP_ALL : s0 + B);
             spa = spb;
             spb = spc;
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(256) void k_sweep(SweepArgs a, const double* __rest
             u32 b[B + 1];
             int lo[B], hi[B];
 #pragma unroll
-            for (int k = 0; k <= B; ++k) b[k] = first[(done + min(k, m)) % (2 * SWEEP_R)];
+            for (int k = 0; k <= B; ++k) b[k] = first[(done + min(k, m)) % SWEEP_FIRST];
 #pragma unroll
             for (int k = 0; k < B; ++k) {
                 const double w = win[((done + min(k, m - 1)) % SWEEP_K) * 64 + lane];
