@@ -59,7 +59,14 @@ struct SymSkip {
 // (26 slices) 23 -> 9.7 us, 150 x 150 with 8 elements' reach 47 -> 20, 220 x 220 plane stress 83 -> 60,
 // 1000 x 1000 composite 527 -> 508.
 // V = float (SPLIT: with the 16-bit remainders lo): the reduced values of the mixed solves, FP64 sums.
-template<bool STOP, class V, bool SPLIT>
+//
+// APART: a value that is not finite reaches only the rows that have an entry for it, as with the full storage.  A
+// padded slot is not multiplied then: its x may belong to another instance of a batch, which 0 * NaN would
+// destroy.  The selects cost a product that reads from memory nothing (1000 x 1000 nodes 522 us with and without)
+// and a batch less than its runs differ by (32 instances of 32 to 256 a side, FP32 values, assembly and solve: 298
+// and 267 ms without, 301 and 263 with), but a CG on a matrix in the cache 1 to 2 % (150 x 150 nodes, ten time steps:
+// 73.0 -> 74.6 ms); a CG ends at the first such value wherever it is, so its products go without.
+template<bool STOP, class V, bool SPLIT, bool APART>
 __global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, SymSkip skip, const i64* __restrict__ kptr,
                                                                  const SymCut* __restrict__ cut, const int2* __restrict__ meta,
                                                                  const V* __restrict__ sval, const int16_t* __restrict__ lo,
@@ -110,8 +117,9 @@ __global__ __launch_bounds__(64 * SYMV_WAVES) void k_symv_slices(i64 rows, SymSk
         if (more) load(k + SYMV_UNROLL, mn, an);
 #pragma unroll
         for (int t = 0; t < SYMV_UNROLL; ++t) {
-            acc += ac[t] * xc[t];
-            if (mc[t].y >= 0) W[mc[t].y + lane] += ac[t] * xr;
+            const bool entry = !APART || ac[t] != 0.0;
+            acc += ac[t] * (entry ? xc[t] : 0.0);
+            if (mc[t].y >= 0) W[mc[t].y + lane] += ac[t] * (entry ? xr : 0.0);
         }
         if (more) {
 #pragma unroll
@@ -559,8 +567,9 @@ void symv_fill_low(nlf_matrix_s* a, SymValues which, hipStream_t s) {
     NLF_HIP(hipGetLastError());
 }
 
-// y = A x from the symmetric storage (symv_prepare first); DOT: partial[0 .. blocks) of x.y, the
-// reduction running on `blocks` blocks (any count: the caller's partial count).
+// y = A x from the symmetric storage (symv_prepare first).  DOT (a product inside CG): partial[0 .. blocks) of x.y,
+// the reduction running on `blocks` blocks (any count: the caller's partial count); passed over once st says done.
+// Otherwise the rows stay apart (see k_symv_slices) and st is not read.
 template<bool DOT>
 void launch_symv(const nlf_matrix_s* a, const double* x, double* y, double* partial, const CGState* st, hipStream_t s,
                  unsigned blocks, SymValues which = SYM_FP64, SymSkip skip = SymSkip{nullptr, nullptr, 0}) {
@@ -571,18 +580,18 @@ void launch_symv(const nlf_matrix_s* a, const double* x, double* y, double* part
                            (const SymCut*)v.cut.p, (const int2*)v.meta.p, values, (const int16_t*)v.slo.p,
                            (const i64*)v.pbase.p, x, v.direct.p, v.part.p, st);
     };
-    const double* v64 = v.sval.p;
-    const float* v32 = v.sval32.p;
-    if (which == SYM_FP64) st ? slices(k_symv_slices<true, double, false>, v64) : slices(k_symv_slices<false, double, false>, v64);
-    else if (which == SYM_FP32) st ? slices(k_symv_slices<true, float, false>, v32) : slices(k_symv_slices<false, float, false>, v32);
-    else st ? slices(k_symv_slices<true, float, true>, v32) : slices(k_symv_slices<false, float, true>, v32);
     const unsigned b2 = std::max(1u, blocks);
-    if (st)
-        hipLaunchKernelGGL((k_symv_reduce<DOT, true>), dim3(b2), dim3(256), 0, s, a->rows, v.ns, skip, v.rptr.p, v.ent.p,
+    auto product = [&](auto stop) {
+        constexpr bool STOP = decltype(stop)::value;
+        if (which == SYM_FP64) slices(k_symv_slices<STOP, double, false, !DOT>, (const double*)v.sval.p);
+        else if (which == SYM_FP32) slices(k_symv_slices<STOP, float, false, !DOT>, (const float*)v.sval32.p);
+        else slices(k_symv_slices<STOP, float, true, !DOT>, (const float*)v.sval32.p);
+        hipLaunchKernelGGL((k_symv_reduce<DOT, STOP>), dim3(b2), dim3(256), 0, s, a->rows, v.ns, skip, v.rptr.p, v.ent.p,
                            v.direct.p, v.part.p, x, y, partial, st);
-    else
-        hipLaunchKernelGGL((k_symv_reduce<DOT, false>), dim3(b2), dim3(256), 0, s, a->rows, v.ns, skip, v.rptr.p, v.ent.p,
-                           v.direct.p, v.part.p, x, y, partial, st);
+    };
+    if constexpr (DOT)
+        if (st) return product(std::true_type{});
+    product(std::false_type{});
 }
 
 }  // namespace nlf

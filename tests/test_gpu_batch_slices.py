@@ -1,0 +1,80 @@
+"""Batched solves whose products read the symmetric slice storage, where a slice of 64 rows holds rows of two
+instances and zero padding that points from one into the other."""
+import numpy as np
+import pytest
+import torch
+
+from nonlocal_amd import _abi as A
+from nonlocal_amd import api, batch, configs
+from tests.helpers import direct_solution, oracle_assembly, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+SIDES = [40, 32, 37, 33]
+BAD = 1
+BOUND = {A.NLF_MODE_FP64: 1e-10, A.NLF_MODE_MIXED: 1e-8}
+
+
+def _instances(lam=1.0):
+    """Four uneven instances, no size a multiple of 64; the second one's conductivity is given."""
+    return [configs.thermal_q4(n, 0.3 + 0.1 * k, 2.5 / n, lam if k == BAD else 1.0 + 0.2 * k, name=f"s{k}")
+            for k, n in enumerate(SIDES)]
+
+
+@pytest.fixture(scope="module")
+def references():
+    refs = []
+    for p in _instances():
+        om, K, f, xD, inner = oracle_assembly(p)
+        refs.append(direct_solution(K, f))
+    return refs
+
+
+# (no ILLT with the conductivity: one factorisation serves the batch, fails and says so)
+@pytest.mark.parametrize("precond,what", [(A.NLF_PRECOND_JACOBI, "load"), (A.NLF_PRECOND_JACOBI, "start"),
+                                          (A.NLF_PRECOND_JACOBI, "conductivity"), (A.NLF_PRECOND_ILLT, "load"),
+                                          (A.NLF_PRECOND_ILLT, "start")])
+@pytest.mark.parametrize("mode", [A.NLF_MODE_FP64, A.NLF_MODE_MIXED])
+def test_instances_stay_apart(gpu_ctx, references, precond, mode, what):
+    """One instance with a not-a-number in its load or its start value, or an infinite conductivity: the others'
+    solutions are the oracle's."""
+    print(f"[batch slices] {what} precond {precond} mode {mode}", flush=True)
+    solver = batch.BatchSolver(_instances(np.inf if what == "conductivity" else 1.0), gpu_ctx, precond=precond)
+    assert solver.K.symv_info() is not None
+    begin, end = solver.node_begin[BAD], solver.node_begin[BAD + 1]
+    x0 = torch.zeros_like(solver.b)
+    if what != "conductivity":
+        (solver.b if what == "load" else x0)[(begin + end) // 2] = float("nan")
+        (solver.b if what == "load" else x0)[[begin, end - 1]] = float("nan")
+    x, its, res, st = solver.solve(tol=1e-12, mode=mode, x0=x0)
+    for i, (xi, ref) in enumerate(zip(solver.split(x), references)):
+        if i != BAD:
+            assert res[i] <= 1e-12, f"instance {i}"
+            assert rel_l2(xi.cpu().numpy(), ref) < BOUND[mode], f"instance {i}"
+
+
+def test_product_of_a_vector_with_nan(gpu_ctx):
+    """nlf_spmv on the slices: not-a-number exactly in the rows with an entry for it, with windows of more than
+    2048 values (radius of 27 elements on a 100 x 100 mesh)."""
+    problem = configs.thermal_q4(100, 0.5, 27.3 / 100)
+    om, K, f, xD, inner = oracle_assembly(problem)
+    g = api.mesh_2d(problem.mesh, gpu_ctx)
+    api._search(g, problem.models)
+    Kg = api._assemble(g, 0, problem.models, problem.materials, inner)
+    slots, strips = Kg.symv_info()
+    print(f"[batch slices] {slots} slots, {strips} strip values in {(f.size + 63) // 64} slices", flush=True)
+    assert strips > 2048 * ((f.size + 63) // 64)
+    x = np.random.default_rng(5).standard_normal(f.size)
+    y = Kg.spmv(torch.from_numpy(x).to(gpu_ctx.device)).cpu().numpy()
+    assert rel_l2(y, K.spmv(x)) <= 1e-13
+    col = f.size // 2 + 3
+    x[col] = np.nan
+    bad = Kg.spmv(torch.from_numpy(x).to(gpu_ctx.device)).cpu().numpy()
+    c = Kg.export(0)                                           # the upper triangle
+    rows = np.repeat(np.arange(f.size), np.diff(c.outer))
+    touched = np.zeros(f.size, dtype=bool)
+    nz = c.val != 0.0
+    touched[rows[nz & (c.inner == col)]] = True
+    touched[c.inner[nz & (rows == col)]] = True
+    assert np.array_equal(np.isnan(bad), touched)
+    assert np.array_equal(bad[~touched], y[~touched])
