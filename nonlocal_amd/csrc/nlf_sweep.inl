@@ -41,7 +41,6 @@ constexpr int SWEEP_CTL = 16, SWEEP_IDLE = 64, SWEEP_SP = 320, SWEEP_WIN = 832, 
               SWEEP_LDS = SWEEP_XV + SWEEP_EXT * 8;
 static_assert(SWEEP_SP + 4 * SWEEP_FIRST <= SWEEP_WIN, "the ring of first records lies before the window");
 constexpr int SWEEP_ALL = 1 << 30;       // a helper wave has staged every step
-constexpr int SWEEP_SPIN = 1 << 21;      // reads of a missing value before it is taken as NaN (seconds)
 constexpr unsigned long long SWEEP_EMPTY = 0xfff8dead0badc0deull;
 constexpr int SWEEP_EMPTY_HI = int(SWEEP_EMPTY >> 32), SWEEP_NAN_HI = 0x7ff80000;
 
@@ -63,6 +62,7 @@ struct SweepArgs {
     // record's bytes together each load touches 64 lines, and 9 such loads took the step of 12 entries 490 cycles
     const unsigned char* rec;
     i64 plane;                           // bytes of a plane
+    i64 wait;                            // most reads of a missing value (sweep_wait_reads)
 };
 
 // Register-ring depth: the steps whose records are in flight, as many as 256 registers hold (3 per entry
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void k_sweep(SweepArgs a, const double* __rest
                 at[k] = es[min(e, total - 1)];
                 got[k] = e >= total;
             }
-            for (int spin = 0;; ++spin) {
+            for (i64 spin = 0;; ++spin) {
                 // a slot is free once no step at or after the next one uses the value it holds
                 if (limit < min(e0 + B, total)) limit = ep[min(ctl_load(ctl + 2), n)] + SWEEP_EXT - SWEEP_EXT_REUSE;
                 unsigned long long w[SWEEP_EB];
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void k_sweep(SweepArgs a, const double* __rest
 #pragma unroll
                 for (int k = 0; k < SWEEP_EB; ++k) {
                     const int e = e0 + 64 * k + lane;
-                    if (!got[k] && e < limit && (w[k] != SWEEP_EMPTY || spin >= SWEEP_SPIN)) {
+                    if (!got[k] && e < limit && (w[k] != SWEEP_EMPTY || spin >= a.wait)) {
                         xv[e % SWEEP_EXT] = __longlong_as_double(static_cast<long long>(w[k]));
                         got[k] = true;
                     }
@@ -690,12 +690,12 @@ __global__ __launch_bounds__(ic_lanes<M>() * ic_rows<M>()) void k_ic_chunks(Swee
         u32 want = 0;
 #pragma unroll
         for (int m = 0; m < M; ++m) want |= r.at[m] >= 0 ? 1u << m : 0u;
-        for (int spin = 0;; ++spin) {
+        for (i64 spin = 0;; ++spin) {
             if (!got) low = ic_load(F, r.b + l);
 #pragma unroll
             for (int m = 0; m < M; ++m)
                 if (want >> m & 1) fj[m] = ic_load(F, r.at[m]);
-            const bool give_up = spin >= SWEEP_SPIN;
+            const bool give_up = spin >= s.wait;
             if (!got && (__double2hiint(low) != SWEEP_EMPTY_HI || give_up)) got = true;
 #pragma unroll
             for (int m = 0; m < M; ++m)
@@ -739,8 +739,8 @@ struct Sweep {
     DevBuf<i32> sptr, eptr, esrc, rsrc, pos, row;
     DevBuf<double> rcoef;
     DevBuf<unsigned char> rec;
-    i64 plane = 0;
-    SweepArgs args() const { return {chunks, chunk.p, sptr.p, eptr.p, esrc.p, rsrc.p, rcoef.p, rec.p, plane}; }
+    i64 plane = 0, steps = 0;            // steps of all chunks
+    SweepArgs args() const { return {chunks, chunk.p, sptr.p, eptr.p, esrc.p, rsrc.p, rcoef.p, rec.p, plane, sweep_wait_reads(steps)}; }
 };
 
 // The plan without the factor's values.
@@ -749,6 +749,7 @@ static void upload_plan(const SweepPlan& P, Sweep& sw, hipStream_t s) {
     sw.WE = P.WE;
     sw.levels = P.levels;
     sw.width = P.width;
+    sw.steps = i64(P.sptr.size()) - sw.chunks;
     upload(sw.chunk, P.chunk.data(), P.chunk.size(), s);
     upload(sw.sptr, P.sptr.data(), P.sptr.size(), s);
     upload(sw.eptr, P.eptr.data(), P.eptr.size(), s);

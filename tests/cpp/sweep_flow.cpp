@@ -3,6 +3,8 @@
 // steps stored.  The external values' wave is taken to be done (it only delays the compute wave, which the orders
 // cover).  The counters only grow and each rule only opens with them, so a wave that acts on older counters acts
 // as it would now: a rule may be tested and acted on at one time.
+//
+// And the bound of a wait for another chunk: never shorter than all steps of the plan one after the other.
 #include <array>
 #include <cstdio>
 #include <vector>
@@ -37,6 +39,12 @@ bool holds(int e, int last, int ring) { return e <= last && last - e < ring; }
 }  // namespace
 
 int main() {
+    constexpr double READ = 0.2, STEP = 3.0, MARGIN = 4.0;     // us: the shortest read, the longest step
+    for (long long steps = 1; steps <= (1ll << 31); steps *= 2)
+        if (double(sweep_wait_reads(steps)) * READ < MARGIN * STEP * double(steps)) {
+            std::printf("a wait ends before %lld steps\n", steps);
+            return 1;
+        }
     std::vector<bool> seen(size_t(BLOCKS + 1) * 3 * (STEPS + 1) * 3 * (SWEEP_K + 1) * 4 * (BATCH + 1));
     std::vector<State> todo{State{}};
     seen[State{}.index()] = true;
