@@ -161,7 +161,11 @@ int         nlf_ctx_synchronize(nlf_ctx ctx);
 #define NLF_OPT_SPMV_SYMMETRIC   6   /* 1 (default): the products of CG, flexible CG and batches (FP64, FP32 or split
                                         values) and of nlf_spmv read the upper triangle once (the reference's
                                         symmetric product), from a slice layout built on the first solve; 0: the
-                                        full (both-triangle) storage */
+                                        full (both-triangle) storage, which is also read where there is no
+                                        memory for the slices */
+#define NLF_OPT_ALLOC_LIMIT_MIB  7   /* MiB of the largest device block the context may allocate, 0 (default): any;
+                                        a larger one fails as if the device had no memory for it (tests of what
+                                        happens then) */
 int         nlf_ctx_set_option(nlf_ctx ctx, int option, int value);
 void*       nlf_ctx_stream(nlf_ctx ctx);
 

@@ -25,6 +25,7 @@ NLF_OPT_ASSEMBLY_THREADS = 3
 NLF_OPT_PATTERN_THREADS = 4
 NLF_OPT_PAIR_BUDGET_MIB = 5
 NLF_OPT_SPMV_SYMMETRIC = 6
+NLF_OPT_ALLOC_LIMIT_MIB = 7
 
 
 class Model(C.Structure):

@@ -423,10 +423,10 @@ i64 batch_cg(nlf_batch B, const V* val, const double* b, double* x, double tol, 
     if (M) { rt.alloc(size_t(n)); zt.alloc(size_t(n)); }
     // The products read the upper triangle once where the symmetric storage applies (32 instances of 32 to 256
     // a side, FP32 values: 630 -> 297 ms for assembly and solve, 560 ms of it left with the full storage); a slice whose instances are all done is passed over.
-    const bool sym = symv_prepare(A, s);
+    DevBuf<int2> slice_inst{size_t((n + 63) / 64)};
     const SymValues which = std::is_same_v<V, double> ? SYM_FP64 : SYM_FP32;
-    if (sym && which == SYM_FP32) symv_fill_low(A, which, s);
-    DevBuf<int2> slice_inst;
+    const SymSolve slices(A, which, s);
+    const bool sym = slices.on;
     SymSkip live{nullptr, nullptr, 0};
     if (sym) {
         std::vector<int2> si(size_t(A->symv->ns));
@@ -438,7 +438,7 @@ i64 batch_cg(nlf_batch B, const V* val, const double* b, double* x, double tol, 
             while (P.row_begin_h[size_t(j) + 1] <= r1) ++j;
             si[k] = make_int2(i, j);
         }
-        upload(slice_inst, si.data(), si.size(), s);
+        NLF_HIP(hipMemcpyAsync(slice_inst.p, si.data(), si.size() * sizeof(int2), hipMemcpyHostToDevice, s));
         NLF_HIP(hipStreamSynchronize(s));              // `si`
         static_assert(sizeof(BatchState) % sizeof(int) == 0, "the done flags are read as ints");
         live = SymSkip{slice_inst.p, &st.p->done, int(sizeof(BatchState) / sizeof(int))};

@@ -25,6 +25,11 @@ struct Error : std::runtime_error {
     Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
 
+// A device block that could not be had (device_alloc): what is only there to be faster is then left out.
+struct OutOfMemory : Error {
+    explicit OutOfMemory(const std::string& m) : Error(NLF_ERR_HIP, m) {}
+};
+
 #define NLF_HIP(expr)                                                                                   \
     do {                                                                                                \
         hipError_t e_ = (expr);                                                                         \
@@ -310,6 +315,7 @@ struct nlf_ctx_s {
     int pattern_threads = 128;           // NLF_OPT_PATTERN_THREADS
     int pair_budget_mib = 0;             // NLF_OPT_PAIR_BUDGET_MIB (0: automatic)
     int spmv_symmetric = 1;              // NLF_OPT_SPMV_SYMMETRIC
+    int alloc_limit_mib = 0;             // NLF_OPT_ALLOC_LIMIT_MIB (0: none)
     // free device blocks of this context's buffers (device_alloc / device_free)
     bool alive = true;
     std::mutex blocks_mu;

@@ -1566,18 +1566,19 @@ i64 fcg(hipStream_t s, nlf_matrix A, const V* val, nlf_precond M, const double* 
         double* true_res, i64* updates, int window, KernelTimer& timer, const int16_t* lo = nullptr) {
     const i64 n = A->rows;
     LearnedGraph& g = *learned_of(M);
+    const unsigned vb = grid_stride_blocks(n), rb = spmv_blocks(64, n);       // no product has more blocks than rb
+    const size_t np = std::max<size_t>(vb, rb);
+    DevBuf<double> r{size_t(n)}, z{size_t(n)}, p{size_t(n)}, q{size_t(n)}, pa{np}, pb{np}, sums{2};
+    DevBuf<FCGState> st{1};
     // the products read the upper triangle once (the symmetric storage), when it applies
-    const bool sym = symv_prepare(A, s);
     const SymValues which = std::is_same_v<V, double> ? SYM_FP64 : lo ? SYM_SPLIT : SYM_FP32;
-    if (sym && which != SYM_FP64) symv_fill_low(A, which, s);
+    const SymSolve slices(A, which, s);
+    const bool sym = slices.on;
     // the lane count (and with it the partial-sum grid) the full-storage layout would take; the symmetric
     // storage applies only where every offset is below 2^15, as the 16-bit one does, so it is known
     // without building that layout
     const int lpr = sym ? pick_lpr(double(A->nnz_full) / double(std::max<i64>(n, 1)), true) : pick_lpr(A);
-    const unsigned sb = spmv_blocks(lpr, n), vb = grid_stride_blocks(n), rb = spmv_blocks(64, n);
-    const size_t np = std::max<size_t>(std::max<size_t>(sb, vb), rb);
-    DevBuf<double> r{size_t(n)}, z{size_t(n)}, p{size_t(n)}, q{size_t(n)}, pa{np}, pb{np}, sums{2};
-    DevBuf<FCGState> st{1};
+    const unsigned sb = spmv_blocks(lpr, n);
     auto true_residual = [&]() {
         residual64(A, x, b, r.p, pa.p, pb.p, rb, s);
         hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, pa.p, int(rb), sums.p);

@@ -240,6 +240,8 @@ void* device_alloc(size_t bytes, size_t* cap, nlf_ctx* owner) {
         return p;
     }
     const size_t want = block_bytes(bytes);
+    if (c->alloc_limit_mib && want > size_t(c->alloc_limit_mib) << 20)
+        throw OutOfMemory(std::to_string(want) + " bytes: over the context's limit of a block");
     {
         std::lock_guard<std::mutex> lock(c->blocks_mu);
         auto it = c->free_blocks.lower_bound(want);
@@ -263,7 +265,9 @@ void* device_alloc(size_t bytes, size_t* cap, nlf_ctx* owner) {
         e = hipMalloc(&p, want);
         if (e != hipSuccess) {
             (void)hipGetLastError();
-            throw Error(NLF_ERR_HIP, std::string("hipMalloc(") + std::to_string(want) + " bytes): " + hipGetErrorString(e));
+            const std::string msg = std::string("hipMalloc(") + std::to_string(want) + " bytes): " + hipGetErrorString(e);
+            if (e == hipErrorOutOfMemory) throw OutOfMemory(msg);
+            throw Error(NLF_ERR_HIP, msg);
         }
     }
     *cap = want;
@@ -365,6 +369,9 @@ int nlf_ctx_set_option(nlf_ctx ctx, int option, int value) {
         ctx->pair_budget_mib = value;
     } else if (option == NLF_OPT_SPMV_SYMMETRIC) {
         ctx->spmv_symmetric = value != 0;
+    } else if (option == NLF_OPT_ALLOC_LIMIT_MIB) {
+        if (value < 0) return NLF_ERR_ARGUMENT;
+        ctx->alloc_limit_mib = value;
     }
     else return NLF_ERR_ARGUMENT;
     return NLF_OK;

@@ -1101,6 +1101,8 @@ struct CG {
     const int16_t* lo = nullptr;        // split values: 16-bit remainders (NLF_MODE_SPLIT)
     const nlf_precond_s* P;
     DevBuf<unsigned char> own;
+    DevBuf<double> r64;                 // solve_reliable: the FP64 residual and the increment of the solution
+    DevBuf<X> xh;
     X *r = nullptr, *z = nullptr, *p = nullptr;
     double *part1 = nullptr, *part2 = nullptr, *pbb = nullptr, *prz = nullptr, *pb2 = nullptr, *sums = nullptr;
     CGState* st = nullptr;
@@ -1153,6 +1155,12 @@ struct CG {
 
     const X* invd() const;
 
+    // the memory of solve_reliable
+    void reserve_reliable() {
+        r64.alloc(size_t(n));
+        xh.alloc(size_t(n));
+    }
+
     // x: initial guess in, solution out; b: right-hand side.  Returns iterations, sets residual.
     i64 solve(const X* b, X* x, double tol, i64 max_it, double* residual, int* breakdown, int check_every = 8) {
         // r = b - A x ; z = M r ; rz = r.z ; bnorm
@@ -1191,13 +1199,11 @@ struct CG {
     // Mixed precision with reliable updates: the CG recurrences run in X (FP32) on the X matrix;
     // whenever the recursive residual has dropped by `delta` since the last update, the FP32
     // solution increment is folded into the FP64 solution, the residual is recomputed in FP64 with
-    // the FP64 matrix and replaces the recursive one; the search direction is kept, so the Krylov
-    // process is not restarted.  Stops on the FP64 true residual ||b - A x|| / ||b|| <= tol.
+    // the FP64 matrix and replaces the recursive one (reserve_reliable first); the search direction is kept, so the
+    // Krylov process is not restarted.  Stops on the FP64 true residual ||b - A x|| / ||b|| <= tol.
     i64 solve_reliable(const i64* o64, const i32* c64, const double* v64, const double* b, double* x, double tol,
                        i64 max_it, double delta, double* true_res, i64* updates, int* breakdown) {
         const unsigned rb = spmv_blocks(64, n);
-        DevBuf<double> r64{size_t(n)};
-        DevBuf<X> xh{size_t(n)};
         auto true_residual = [&]() {
             if (sym) residual64(sym, x, b, r64.p, part1, part2, rb, s);
             else residual64(n, o64, cs, v64, lpr, x, b, r64.p, part1, part2, rb, s);
@@ -1733,12 +1739,10 @@ int nlf_cg_solve(nlf_matrix a, nlf_precond p, const double* b, double* x, double
             CG<float, double> cg(s, n, a->nnz_full, a->outer.p, a->cols.p, a->val32.p, p);
             cg.indefinite = a->neumann;
             if (mode == NLF_MODE_SPLIT) cg.lo = a->val_lo.p;
-            if (symv_prepare(a, s)) {
-                symv_fill_low(a, cg.lo ? SYM_SPLIT : SYM_FP32, s);
-                cg.set_symmetric(a);
-            } else {
-                cg.set_cols(a);
-            }
+            cg.reserve_reliable();
+            const SymSolve sym(a, cg.lo ? SYM_SPLIT : SYM_FP32, s);
+            if (sym.on) cg.set_symmetric(a);
+            else cg.set_cols(a);
             out.iterations = cg.solve_reliable(a->outer.p, a->cols.p, a->val.p, b, x, tol, max_it, 0.1,
                                                &out.true_residual, &out.outer_iterations, &breakdown);
             out.residual = out.true_residual;

@@ -455,15 +455,9 @@ void symv_release(nlf_matrix_s* a) {
 // 163 us here (windows of 4600 doubles, four workgroups to a compute unit).
 constexpr i64 SYMV_WINDOW = 7168;
 
-// Builds (or rebuilds, when the values changed) the symmetric SpMV storage of a FP64 matrix.  Returns
-// false, with nothing kept, where it does not apply: offsets of 2^15 or more, more than 255 bands in a
-// slice, a window over SYMV_WINDOW doubles, or padding that leaves less than a quarter of the traffic saved.
-bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
-    if (!a->ctx->spmv_symmetric || a->rows <= 0 || !a->val.p || a->nnz_full <= 0) return false;
-    if (a->symv && a->symv->version == a->val_version && !a->values_exposed) return true;
-    if (a->symv_refused_version == a->val_version) return false;
-    symv_release(a);
-    auto refuse = [&]() { a->symv_refused_version = a->val_version; return false; };
+// The storage where it applies, in a->symv; false where it does not.
+static bool symv_build(nlf_matrix_s* a, hipStream_t s) {
+    auto refuse = [] { return false; };
     const i64 rows = a->rows, ns = (rows + 63) / 64;
     if (ns >= (i64(1) << 27)) return refuse();
     // the widest upper offset
@@ -544,12 +538,34 @@ bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
     return true;
 }
 
+// Nothing kept, and no further attempt with these values.
+static bool symv_refuse(nlf_matrix_s* a) {
+    symv_release(a);
+    a->symv_refused_version = a->val_version;
+    return false;
+}
+
+// Builds (or rebuilds, when the values changed) the symmetric SpMV storage of a FP64 matrix.  Returns
+// false, with nothing kept, where it does not apply: offsets of 2^15 or more, more than 255 bands in a
+// slice, a window over SYMV_WINDOW doubles, padding that leaves less than a quarter of the traffic saved, or no
+// memory for it.
+bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
+    if (!a->ctx->spmv_symmetric || a->rows <= 0 || !a->val.p || a->nnz_full <= 0) return false;
+    if (a->symv && a->symv->version == a->val_version && !a->values_exposed) return true;
+    if (a->symv_refused_version == a->val_version) return false;
+    symv_release(a);
+    try {
+        return symv_build(a, s) || symv_refuse(a);
+    } catch (const OutOfMemory&) {
+        return symv_refuse(a);
+    }
+}
+
 // The values a product reads: the FP64 ones, the FP32 ones or the split ones (symv_fill_low first).
 enum SymValues { SYM_FP64, SYM_FP32, SYM_SPLIT };
 
-// Fills the slices' reduced values from val32 (and val_lo); symv_prepare first.  Each mixed solve fills them
-// anew (one pass over the upper triangle), so they never lag behind the matrix's.
-void symv_fill_low(nlf_matrix_s* a, SymValues which, hipStream_t s) {
+// Fills the slices' reduced values from val32 (and val_lo); symv_prepare first.
+static void symv_fill_low(nlf_matrix_s* a, SymValues which, hipStream_t s) {
     nlf_symv_s& v = *a->symv;
     const size_t n = size_t(std::max<i64>(v.slots, 1)) * 64;
     auto fill = [&](auto* from, auto* to) {
@@ -566,6 +582,31 @@ void symv_fill_low(nlf_matrix_s* a, SymValues which, hipStream_t s) {
     }
     NLF_HIP(hipGetLastError());
 }
+
+// The slices of one solve, with the values it reads.  Reduced values are filled anew for each solve (one pass over
+// the upper triangle), so they never lag behind the matrix's, and given back at its end.  What the solve allocates
+// itself it allocates first: a solve that fits with the full storage then runs with it where the slices do not fit
+// beside.
+struct SymSolve {
+    nlf_matrix_s* a;
+    SymValues which;
+    bool on;
+    SymSolve(nlf_matrix_s* a_, SymValues w, hipStream_t s) : a(a_), which(w), on(symv_prepare(a_, s)) {
+        if (!on || which == SYM_FP64) return;
+        try {
+            symv_fill_low(a, which, s);
+        } catch (const OutOfMemory&) {
+            on = symv_refuse(a);
+        }
+    }
+    ~SymSolve() {
+        if (!on || !a->symv) return;
+        a->symv->sval32.release();
+        a->symv->slo.release();
+    }
+    SymSolve(const SymSolve&) = delete;
+    SymSolve& operator=(const SymSolve&) = delete;
+};
 
 // y = A x from the symmetric storage (symv_prepare first).  DOT (a product inside CG): partial[0 .. blocks) of x.y,
 // the reduction running on `blocks` blocks (any count: the caller's partial count); passed over once st says done.

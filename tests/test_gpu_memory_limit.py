@@ -1,0 +1,112 @@
+"""Storage that is only there to be faster is left out where there is no memory for it: the same solve as without
+it, to the bit.  NLF_OPT_ALLOC_LIMIT_MIB makes the one block fail that is to be left out."""
+import contextlib
+
+import numpy as np
+import pytest
+import torch
+
+from nonlocal_amd import _abi as A
+from nonlocal_amd import api, batch, configs, learned
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+MODES = [A.NLF_MODE_FP64, A.NLF_MODE_MIXED, A.NLF_MODE_SPLIT]
+
+
+@contextlib.contextmanager
+def option(ctx, which, value, normal):
+    ctx.set_option(which, value)
+    try:
+        yield
+    finally:
+        ctx.set_option(which, normal)
+
+
+def full_storage(ctx):
+    return option(ctx, A.NLF_OPT_SPMV_SYMMETRIC, 0, 1)
+
+
+def limit(ctx, too_large):
+    """A limit that a block of `too_large` bytes exceeds, by less than a MiB."""
+    assert too_large > 2 << 20
+    return option(ctx, A.NLF_OPT_ALLOC_LIMIT_MIB, (too_large - 1) >> 20, 0)
+
+
+def without_slices(ctx, make, solve, reduced):
+    """solve(K) with the full storage, then without memory for the slices (`reduced`: for their reduced values)."""
+    K = make()
+    with full_storage(ctx):
+        want = solve(K)
+    slots = make().symv_info()[0]
+    if reduced:
+        assert K.symv_info() is not None
+    with limit(ctx, slots * 64 * (4 if reduced else 8)):
+        got = solve(K)
+        assert K.symv_info() is None
+    assert torch.equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    return want
+
+
+@pytest.mark.parametrize("mode,reduced", [(m, False) for m in MODES] + [(m, True) for m in MODES[1:]])
+def test_cg(gpu_ctx, mode, reduced):
+    print(f"[memory limit] cg mode {mode} reduced {reduced}", flush=True)
+    problem = configs.thermal_q4(100, 0.5, 6.3 / 100)
+    om, Ko, f, xD, inner = H.oracle_assembly(problem)
+    g = api.mesh_2d(problem.mesh, gpu_ctx)
+    api._search(g, problem.models)
+    b = torch.from_numpy(f).to(gpu_ctx.device)
+
+    def make():
+        K = api._assemble(g, 0, problem.models, problem.materials, inner)
+        if mode == A.NLF_MODE_MIXED:
+            K.make_fp32()
+        if mode == A.NLF_MODE_SPLIT:
+            K.make_split()
+        return K
+
+    def solve(K):
+        cg = api.conjugate_gradient(K)
+        cg.init_preconditioner(A.NLF_PRECOND_JACOBI)
+        cg.set_tolerance(1e-12)
+        return cg.solve(b, mode=mode), cg.iterations()
+
+    x, it = without_slices(gpu_ctx, make, solve, reduced)
+    assert H.rel_l2(x.cpu().numpy(), H.direct_solution(Ko, f)) <= 1e-9
+
+
+@pytest.mark.parametrize("mode,reduced", [(A.NLF_MODE_FP64, False), (A.NLF_MODE_MIXED, False), (A.NLF_MODE_MIXED, True)])
+def test_flexible_cg(gpu_ctx, mode, reduced):
+    print(f"[memory limit] flexible cg mode {mode} reduced {reduced}", flush=True)
+
+    def make():
+        tp = learned.TrainingProblem(96, seed=1, ctx=gpu_ctx, count=3, r=5.3 / 96)
+        tp.K.make_fp32()
+        tp.K.problem = tp
+        return tp.K
+
+    def solve(K):
+        x, st = learned.fcg_solve(K, K.problem.learned, K.problem.b, tol=1e-10, max_it=20000, mode=mode)
+        assert st.true_residual <= 1e-10
+        return x, st.iterations
+
+    without_slices(gpu_ctx, make, solve, reduced)
+
+
+@pytest.mark.parametrize("mode,reduced", [(A.NLF_MODE_FP64, False), (A.NLF_MODE_MIXED, False), (A.NLF_MODE_MIXED, True)])
+def test_batch(gpu_ctx, mode, reduced):
+    print(f"[memory limit] batch mode {mode} reduced {reduced}", flush=True)
+    problems = [configs.thermal_q4(n, 0.5, 5.3 / n, name=f"m{n}") for n in (90, 70, 81)]
+
+    def make():
+        solver = batch.BatchSolver(problems, gpu_ctx)
+        solver.K.solver = solver
+        return solver.K
+
+    def solve(K):
+        x, its, res, st = K.solver.solve(tol=1e-11, mode=mode)
+        assert res.max() <= 1e-11
+        return x, its
+
+    without_slices(gpu_ctx, make, solve, reduced)
