@@ -1493,35 +1493,8 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
                 merged.clear();
                 return plan_sweep(outer, cols, diag, forward ? fr : br, forward ? fp : bp, bounds, forward, merged, false, q);
             };
-            P->chunked = cols.size() < (size_t(1) << 31) && plan(true, mf, pf) && plan(false, mb, pb);
-            if (P->chunked) {
-                upload_plan(pf, P->sw_fw, s);
-                upload_plan(pb, P->sw_bw, s);
-                P->ticket.alloc(2);
-                {
-                    Sweep own;                           // a merged pair's rows are factored one after the other
-                    if (!mf.empty()) {
-                        plan_sweep(outer, cols, diag, fr, fp, bounds, true, {}, true, pi);
-                        upload_plan(pi, own, s);
-                    }
-                    const Sweep& sw = mf.empty() ? P->sw_fw : own;
-                    DevBuf<i32> list;
-                    const int W = std::max(P->sw_fw.WE, P->sw_bw.WE);
-                    ic_lists(sw, W, n, d_outer, d_cols, d_diag, list, s);
-                    factor([&](double shift) {
-                        launch_ic(sw, W, P->ticket.p, d_outer, d_cols, d_diag, tpos.p, list.p, a->val.p, P->scale.p, shift,
-                                  i64(cols.size()), P->F.p, fail.p, s);
-                    });
-                }
-                pack_sweep(pf, true, d_outer, d_diag, P->F.p, P->scale.p, nullptr, P->sw_fw, s);
-                pack_sweep(pb, false, d_outer, d_diag, P->F.p, P->scale.p, P->sw_fw.pos.p, P->sw_bw, s);
-                P->fw_lvl.alloc(size_t(n));
-                P->bw_lvl.alloc(size_t(n));
-                hipLaunchKernelGGL(k_sweep_empty, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, P->fw_lvl.p, P->bw_lvl.p,
-                                   P->ticket.p);
-                NLF_HIP(hipGetLastError());
-            } else {
-                // rows with more dependencies than the chunked sweeps take
+            // level by level, a workgroup per independent block
+            auto factor_levels = [&] {
                 DevBuf<i32> lrows, lptr;
                 DevBuf<SweepBlock> blk;
                 LevelArgs la{n, P->fw_levels, d_outer, d_cols, d_diag, tpos.p, nullptr, nullptr};
@@ -1546,6 +1519,44 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
                     hipLaunchKernelGGL(k_ic_factor, dim3(unsigned(P->blocks)), dim3(LEVEL_THREADS), 0, s, la,
                                        P->blocks > 1 ? (const SweepBlock*)blk.p : nullptr, P->F.p, fail.p);
                 });
+            };
+            // over the chunks; false where there is no memory for its lists (up to 4 KB a row)
+            auto factor_chunks = [&] {
+                try {
+                    Sweep own;                           // a merged pair's rows are factored one after the other
+                    if (!mf.empty()) {
+                        plan_sweep(outer, cols, diag, fr, fp, bounds, true, {}, true, pi);
+                        upload_plan(pi, own, s);
+                    }
+                    const Sweep& sw = mf.empty() ? P->sw_fw : own;
+                    DevBuf<i32> list;
+                    const int W = std::max(P->sw_fw.WE, P->sw_bw.WE);
+                    ic_lists(sw, W, n, d_outer, d_cols, d_diag, list, s);
+                    factor([&](double shift) {
+                        launch_ic(sw, W, P->ticket.p, d_outer, d_cols, d_diag, tpos.p, list.p, a->val.p, P->scale.p, shift,
+                                  i64(cols.size()), P->F.p, fail.p, s);
+                    });
+                    return true;
+                } catch (const OutOfMemory&) {
+                    return false;
+                }
+            };
+            P->chunked = cols.size() < (size_t(1) << 31) && plan(true, mf, pf) && plan(false, mb, pb);
+            if (P->chunked) {
+                upload_plan(pf, P->sw_fw, s);
+                upload_plan(pb, P->sw_bw, s);
+                P->ticket.alloc(2);
+                if (!factor_chunks()) factor_levels();
+                pack_sweep(pf, true, d_outer, d_diag, P->F.p, P->scale.p, nullptr, P->sw_fw, s);
+                pack_sweep(pb, false, d_outer, d_diag, P->F.p, P->scale.p, P->sw_fw.pos.p, P->sw_bw, s);
+                P->fw_lvl.alloc(size_t(n));
+                P->bw_lvl.alloc(size_t(n));
+                hipLaunchKernelGGL(k_sweep_empty, dim3(grid_stride_blocks(n)), dim3(256), 0, s, n, P->fw_lvl.p, P->bw_lvl.p,
+                                   P->ticket.p);
+                NLF_HIP(hipGetLastError());
+            } else {
+                // rows with more dependencies than the chunked sweeps take
+                factor_levels();
                 build_sweep(outer, cols, diag, fr, fp, true, P->F.p, P->scale.p, d_diag, P->fw, s);
                 build_sweep(outer, cols, diag, br, bp, false, P->F.p, P->scale.p, d_diag, P->bw, s);
                 const int widest = std::max(P->fw.W, P->bw.W);

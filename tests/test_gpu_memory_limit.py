@@ -110,3 +110,25 @@ def test_batch(gpu_ctx, mode, reduced):
         return x, its
 
     without_slices(gpu_ctx, make, solve, reduced)
+
+
+@pytest.mark.parametrize("build", [lambda: configs.cfg1(0.2), lambda: configs.cfg2(0.2)], ids=["q8", "elastic_q4"])
+def test_factorisation(gpu_ctx, build):
+    """The incomplete factorisation without the lists that its chunks work from: the same preconditioner."""
+    problem = build()
+    print(f"[memory limit] factorisation of {problem.mesh.n_nodes} rows", flush=True)
+    om, KL, f, xD, inner = H.oracle_assembly(problem, part=A.NLF_PART_LOCAL)
+    g = api.mesh_2d(problem.mesh, gpu_ctx)
+    K = api._assemble(g, problem.physics, problem.models, problem.materials, inner, part=A.NLF_PART_LOCAL)
+    upper = KL.export(0)
+    above = np.diff(upper.outer) - 1                                    # entries beside the diagonal
+    below = np.bincount(upper.inner, minlength=f.size) - 1
+    entries = max(above.max(), below.max())
+    width, lanes = next((w, l) for w, l in [(4, 4), (8, 8), (12, 16), (16, 16), (24, 32), (32, 32)] if entries <= w)
+    r = torch.from_numpy(np.random.default_rng(2).standard_normal(f.size)).to(gpu_ctx.device)
+    P = api.preconditioner(K, A.NLF_PRECOND_ILLT)
+    z = P.solve(r).cpu().numpy()
+    with limit(gpu_ctx, f.size * width * lanes * 4):
+        Q = api.preconditioner(K, A.NLF_PRECOND_ILLT)
+    assert Q.info()["ok"] and Q.info()["shift"] == P.info()["shift"] and Q.sweep_info() == P.sweep_info()
+    assert H.rel_l2(Q.solve(r).cpu().numpy(), z) <= 1e-12            # as every layout against the oracle's
