@@ -1810,13 +1810,8 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
         max_upper = h_len[0];
         max_bound = h_len[1];
     }
-    if ((!any_nonlocal || only_local) && max_upper <= 64 && max_bound <= 64) {
-        const unsigned nb = unsigned((m->N + 3) / 4);
-        if (mat->physics != 1 && m->nn == 4) hipLaunchKernelGGL((k_assemble_local<1, 4, 4, T>), dim3(nb), dim3(256), 0, s, aa);
-        else if (mat->physics != 1 && m->nn == 8) hipLaunchKernelGGL((k_assemble_local<1, 8, 9, T>), dim3(nb), dim3(256), 0, s, aa);
-        else if (mat->physics == 1 && m->nn == 4) hipLaunchKernelGGL((k_assemble_local<2, 4, 4, T>), dim3(nb), dim3(256), 0, s, aa);
-        else hipLaunchKernelGGL((k_assemble_local<2, 8, 9, T>), dim3(nb), dim3(256), 0, s, aa);
-    } else if (use_pairs) {
+    PairPlan own;
+    auto by_pairs = [&](AssemblyArgs aa) {
         // thermal nonlocal blocks through the MFMA pair kernels.  When every element's blocks (nn * nn
         // values per neighbour pair) fit the budget -- 8 GiB, or NLF_OPT_PAIR_BUDGET_MIB -- one pass
         // lists every element once with its blocks at its neighbour-list offset; otherwise node chunk
@@ -1826,7 +1821,6 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
         const i64 E = m->E, N = m->N;
         const int nn = m->nn;                          // values of a pair block: nn * nn
         const i64 per_pair = nn * nn * i64(sizeof(T));
-        PairPlan own;
         if (!plan || plan->per_pair != per_pair) {
             std::vector<i64> nb_off(size_t(E + 1));
             download(nb_off.data(), m->nb_off.p, nb_off.size(), s);
@@ -1927,10 +1921,30 @@ void assemble_values(nlf_matrix_s* mat, hipStream_t s, const PairPlan* plan = nu
             NLF_HIP(hipStreamSynchronize(s));          // before the chunk offsets and lists are released
         }
         NLF_HIP(hipStreamSynchronize(s));              // before the pair buffer is released
-    } else if (mat->physics != 1 && m->nn == 4) launch_assemble<1, 4, 4, T>(aa, injective, lds, m->N, s, m->ctx->assembly_threads);
-    else if (mat->physics != 1 && m->nn == 8) launch_assemble<1, 8, 9, T>(aa, injective, lds, m->N, s, m->ctx->assembly_threads);
-    else if (mat->physics == 1 && m->nn == 4) launch_assemble<2, 4, 4, T>(aa, injective, lds, m->N, s, m->ctx->assembly_threads);
-    else launch_assemble<2, 8, 9, T>(aa, injective, lds, m->N, s, m->ctx->assembly_threads);
+    };
+    // the blocks only save time: without memory for them every node contracts its own entries, as it does where
+    // they are switched off (nothing has been added to the values when an allocation fails)
+    auto by_nodes = [&] {
+        if (mat->physics != 1 && m->nn == 4) launch_assemble<1, 4, 4, T>(aa, injective, lds, m->N, s, m->ctx->assembly_threads);
+        else if (mat->physics != 1 && m->nn == 8) launch_assemble<1, 8, 9, T>(aa, injective, lds, m->N, s, m->ctx->assembly_threads);
+        else if (mat->physics == 1 && m->nn == 4) launch_assemble<2, 4, 4, T>(aa, injective, lds, m->N, s, m->ctx->assembly_threads);
+        else launch_assemble<2, 8, 9, T>(aa, injective, lds, m->N, s, m->ctx->assembly_threads);
+    };
+    if ((!any_nonlocal || only_local) && max_upper <= 64 && max_bound <= 64) {
+        const unsigned nb = unsigned((m->N + 3) / 4);
+        if (mat->physics != 1 && m->nn == 4) hipLaunchKernelGGL((k_assemble_local<1, 4, 4, T>), dim3(nb), dim3(256), 0, s, aa);
+        else if (mat->physics != 1 && m->nn == 8) hipLaunchKernelGGL((k_assemble_local<1, 8, 9, T>), dim3(nb), dim3(256), 0, s, aa);
+        else if (mat->physics == 1 && m->nn == 4) hipLaunchKernelGGL((k_assemble_local<2, 4, 4, T>), dim3(nb), dim3(256), 0, s, aa);
+        else hipLaunchKernelGGL((k_assemble_local<2, 8, 9, T>), dim3(nb), dim3(256), 0, s, aa);
+    } else if (use_pairs) {
+        try {
+            by_pairs(aa);
+        } catch (const OutOfMemory&) {
+            by_nodes();
+        }
+    } else {
+        by_nodes();
+    }
     NLF_HIP(hipGetLastError());
     T* values = nullptr;
     if constexpr (F64) values = mat->val.p; else values = mat->val32.p;

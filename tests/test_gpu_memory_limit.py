@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from nonlocal_amd import _abi as A
-from nonlocal_amd import api, batch, configs, learned
+from nonlocal_amd import api, batch, configs, learned, meshgen
 from tests import helpers as H
 
 pytestmark = pytest.mark.gpu
@@ -132,3 +132,23 @@ def test_factorisation(gpu_ctx, build):
         Q = api.preconditioner(K, A.NLF_PRECOND_ILLT)
     assert Q.info()["ok"] and Q.info()["shift"] == P.info()["shift"] and Q.sweep_info() == P.sweep_info()
     assert H.rel_l2(Q.solve(r).cpu().numpy(), z) <= 1e-12            # as every layout against the oracle's
+
+
+@pytest.mark.parametrize("q8", [True, False], ids=["q8", "q4"])
+def test_assembly(gpu_ctx, q8):
+    """Nonlocal heat matrices without the element-pair blocks: the node-centric contraction's values."""
+    n = 14 if q8 else 40
+    mesh = meshgen.structured_q8(n, jitter=0.2, seed=n) if q8 else meshgen.structured_q4(n, jitter=0.2, seed=n)
+    print(f"[memory limit] assembly of {mesh.n_nodes} nodes", flush=True)
+    models, mats = [configs.bell(0.4, 4.3 / n)], [A.thermal_material()]
+    g = api.mesh_2d(mesh, gpu_ctx)
+    api.find_neighbours(g, H.radii(models))
+    inner = np.ones(mesh.n_nodes, dtype=np.uint8)
+    inner[:n] = 0
+    with option(gpu_ctx, A.NLF_OPT_ASSEMBLY_PAIRS, 0, 1):
+        want = api._assemble(g, 0, models, mats, inner)
+    with limit(gpu_ctx, int(g.neighbours()[0][-1]) * mesh.nn ** 2 * 8):
+        got = api._assemble(g, 0, models, mats, inner)
+    for part in (1, 2):
+        a, b = got.export(part), want.export(part)
+        assert np.array_equal(a.inner, b.inner) and np.array_equal(a.val, b.val)
