@@ -391,7 +391,9 @@ int nlf_fcg_solve(nlf_matrix a, nlf_precond learned, nlf_precond fallback, const
  * G iterations per captured hipGraph replay; each instance stops on its FP64 true residual. */
 int nlf_batch_create(nlf_matrix a, int count, const int64_t* row_begin, nlf_batch* out);
 int nlf_batch_destroy(nlf_batch b);
-/* picks each instance's SpMV tile (lanes per row, rows per block) by timing; cache_path may be NULL */
+/* picks each instance's SpMV tile (lanes per row, rows per block) on the full storage by timing; cache_path may be
+ * NULL.  Where the products read the symmetric slices (NLF_OPT_SPMV_SYMMETRIC) there is no tile to pick: nothing is
+ * timed or written, and chosen is the tile that stands */
 int nlf_batch_autotune(nlf_batch b, const char* cache_path, double* chosen);
 /* No reference counterpart.  ILLT (IC(0) of the batch's local matrix, block diagonal like the batch) for the
  * batch's solves, or NULL for Jacobi (the default); the handle must outlive the solves. */

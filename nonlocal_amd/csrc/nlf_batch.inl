@@ -568,7 +568,9 @@ int nlf_batch_destroy(nlf_batch b) {
 // Autotuner: times the batched SpMV for each target of nonzeros per lane (which sets every
 // instance's lanes-per-row class and rows-per-block tile) and keeps the fastest.  With a cache
 // file, a batch whose signature (instance sizes and nonzeros) is listed there reuses the stored
-// choice; a new measurement is appended.  chosen (optional) receives the target.
+// choice; a new measurement is appended.  chosen (optional) receives the target.  Where the products
+// read the symmetric slices there is nothing to choose: no layout is built, nothing measured or
+// appended, and the target stays as it is.
 int nlf_batch_autotune(nlf_batch b, const char* cache_path, double* chosen) {
     if (!b) return NLF_ERR_ARGUMENT;
     return guarded(b->ctx, [&] {
@@ -594,7 +596,9 @@ int nlf_batch_autotune(nlf_batch b, const char* cache_path, double* chosen) {
             }
         }
         const auto t0 = std::chrono::steady_clock::now();
-        if (!found) {
+        if (!found && symv_prepare(A, s)) {
+            best_t = P.target;
+        } else if (!found) {
             DevBuf<double> x{size_t(A->rows)}, y{size_t(A->rows)};
             hipLaunchKernelGGL(k_bfill, dim3(grid_stride_blocks(A->rows)), dim3(256), 0, s, A->rows, x.p, 1.0);
             hipEvent_t e0, e1;
@@ -620,7 +624,7 @@ int nlf_batch_autotune(nlf_batch b, const char* cache_path, double* chosen) {
                     std::fclose(f);
                 }
         }
-        batch_build_plan(P, A, best_t, s);
+        if (best_t != P.target) batch_build_plan(P, A, best_t, s);
         NLF_HIP(hipStreamSynchronize(s));
         b->tune_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
         if (chosen) *chosen = best_t;

@@ -53,6 +53,20 @@ def test_instances_stay_apart(gpu_ctx, references, precond, mode, what):
             assert rel_l2(xi.cpu().numpy(), ref) < BOUND[mode], f"instance {i}"
 
 
+def test_autotuner_has_nothing_to_choose(gpu_ctx, tmp_path):
+    """Where the solve reads the slices, the autotuner times and writes nothing; with them off it does."""
+    solver = batch.BatchSolver(_instances(), gpu_ctx)
+    cache = tmp_path / "tune.txt"
+    assert solver.autotune(str(cache)) == 4.0 and not cache.exists()
+    gpu_ctx.set_option(A.NLF_OPT_SPMV_SYMMETRIC, 0)
+    try:
+        chosen = solver.autotune(str(cache))
+    finally:
+        gpu_ctx.set_option(A.NLF_OPT_SPMV_SYMMETRIC, 1)
+    assert chosen in (1.0, 2.0, 4.0, 8.0, 16.0) and len(cache.read_text().split()) == 2
+    assert solver.autotune(str(cache)) == chosen                # a stored choice is taken either way
+
+
 def test_product_of_a_vector_with_nan(gpu_ctx):
     """nlf_spmv on the slices: not-a-number exactly in the rows with an entry for it, with windows of more than
     2048 values (radius of 27 elements on a 100 x 100 mesh)."""
