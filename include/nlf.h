@@ -161,8 +161,9 @@ int         nlf_ctx_synchronize(nlf_ctx ctx);
 #define NLF_OPT_SPMV_SYMMETRIC   6   /* 1 (default): the products of CG, flexible CG and batches (FP64, FP32 or split
                                         values) and of nlf_spmv read the upper triangle once (the reference's
                                         symmetric product), from a slice layout built on the first solve; 0: the
-                                        full (both-triangle) storage, which is also read where there is no
-                                        memory for the slices */
+                                        full (both-triangle) storage, which is also read where it is faster
+                                        (small systems of reduced values, small batches) and where there is
+                                        no memory for the slices */
 #define NLF_OPT_ALLOC_LIMIT_MIB  7   /* MiB of the largest device block the context may allocate, 0 (default): any;
                                         a larger one fails as if the device had no memory for it (tests of what
                                         happens then) */

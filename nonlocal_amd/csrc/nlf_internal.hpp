@@ -420,7 +420,7 @@ struct SpmvCols {
     const int16_t* off;       // offsets (col - row); with pstart: the dictionary
     const i64* pstart;
 };
-i64 spmv_stream_bytes(const nlf_matrix_s* a, size_t sv, size_t sx);   // HBM bytes of one SpMV
+i64 spmv_stream_bytes(const nlf_matrix_s* a, size_t sv, size_t sx, bool slices);   // HBM bytes of one SpMV
 
 // Aggregation coarse space for the learned preconditioner's two-level form:
 // B r = M r + P A_c^-1 P^T r, P the 0/1 map of rows to aggregates (a grid of cells over the node

@@ -1563,7 +1563,7 @@ __global__ __launch_bounds__(256) void k_graph_stats(i64 n, const i64* __restric
 
 template<class V>
 i64 fcg(hipStream_t s, nlf_matrix A, const V* val, nlf_precond M, const double* b, double* x, double tol, i64 max_it,
-        double* true_res, i64* updates, int window, KernelTimer& timer, const int16_t* lo = nullptr) {
+        double* true_res, i64* updates, int window, KernelTimer& timer, bool* on_slices, const int16_t* lo = nullptr) {
     const i64 n = A->rows;
     LearnedGraph& g = *learned_of(M);
     const unsigned vb = grid_stride_blocks(n), rb = spmv_blocks(64, n);       // no product has more blocks than rb
@@ -1573,7 +1573,7 @@ i64 fcg(hipStream_t s, nlf_matrix A, const V* val, nlf_precond M, const double* 
     // the products read the upper triangle once (the symmetric storage), when it applies
     const SymValues which = std::is_same_v<V, double> ? SYM_FP64 : lo ? SYM_SPLIT : SYM_FP32;
     const SymSolve slices(A, which, s);
-    const bool sym = slices.on;
+    const bool sym = *on_slices = slices.on;
     // the lane count (and with it the partial-sum grid) the full-storage layout would take; the symmetric
     // storage applies only where every offset is below 2^15, as the 16-bit one does, so it is known
     // without building that layout
@@ -1902,21 +1902,24 @@ int nlf_fcg_solve(nlf_matrix A, nlf_precond M, nlf_precond fallback, const doubl
         out.preconditioner = NLF_PRECOND_LEARNED;
         KernelTimer timer;
         i64 it = 0;
+        bool on_slices = false;
         if (mode == NLF_MODE_MIXED) {
             NLF_CHECK(A->val32.p, NLF_ERR_STATE, "mixed mode needs nlf_matrix_make_fp32 first");
-            it = fcg<float>(s, A, A->val32.p, M, b, x, tol, max_it, &out.true_residual, &out.outer_iterations, FCG_WINDOW, timer);
+            it = fcg<float>(s, A, A->val32.p, M, b, x, tol, max_it, &out.true_residual, &out.outer_iterations, FCG_WINDOW, timer,
+                            &on_slices);
         } else if (mode == NLF_MODE_SPLIT) {
             NLF_CHECK(A->split_ready, NLF_ERR_STATE, "split mode needs nlf_matrix_make_split first");
             it = fcg<float>(s, A, A->val32.p, M, b, x, tol, max_it, &out.true_residual, &out.outer_iterations, FCG_WINDOW, timer,
-                            A->val_lo.p);
+                            &on_slices, A->val_lo.p);
         } else {
             NLF_CHECK(mode == NLF_MODE_FP64, NLF_ERR_ARGUMENT, "unknown mode");
-            it = fcg<double>(s, A, A->val.p, M, b, x, tol, max_it, &out.true_residual, &out.outer_iterations, FCG_WINDOW, timer);
+            it = fcg<double>(s, A, A->val.p, M, b, x, tol, max_it, &out.true_residual, &out.outer_iterations, FCG_WINDOW, timer,
+                            &on_slices);
         }
         out.spmv_ms = timer.avg(0);
         out.precond_ms = timer.avg(1);
         out.spmv_samples = timer.count[0];
-        out.spmv_bytes = spmv_stream_bytes(A, mode == NLF_MODE_MIXED ? 4 : mode == NLF_MODE_SPLIT ? 6 : 8, 8);
+        out.spmv_bytes = spmv_stream_bytes(A, mode == NLF_MODE_MIXED ? 4 : mode == NLF_MODE_SPLIT ? 6 : 8, 8, on_slices);
         if (it < 0) {
             // stagnation: fall back to PCG with the fallback preconditioner from the current iterate
             out.fallbacks = 1;

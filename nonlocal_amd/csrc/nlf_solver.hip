@@ -1301,10 +1301,10 @@ using namespace nlf;
 
 namespace nlf {
 
-// HBM bytes one SpMV streams: values, column source, row pointers, x once and y.
-i64 spmv_stream_bytes(const nlf_matrix_s* a, size_t sv, size_t sx) {
+// HBM bytes one SpMV streams: values, column source, row pointers, x once and y.  slices: it reads a->symv.
+i64 spmv_stream_bytes(const nlf_matrix_s* a, size_t sv, size_t sx, bool slices) {
     const i64 n = a->rows;
-    if (a->symv && a->ctx->spmv_symmetric && a->symv->version == a->val_version) {
+    if (slices) {
         // slice values, the strips written and read, the direct sums written and read, x once and y
         const nlf_symv_s& v = *a->symv;
         return v.slots * 64 * i64(sv) + 2 * v.part_size * i64(sizeof(double)) + n * i64(4 * sizeof(double));
@@ -1699,7 +1699,7 @@ int nlf_cg_solve_noalloc(nlf_matrix a, nlf_precond p, const double* b, double* x
         cg.set_cols(a);
         cg.indefinite = a->neumann;
         out.iterations = cg.solve(b, x, tol, max_it, &out.residual, &breakdown);
-        out.spmv_bytes = spmv_stream_bytes(a, sizeof(double), sizeof(double));
+        out.spmv_bytes = spmv_stream_bytes(a, sizeof(double), sizeof(double), false);
         // FP64 true residual ||b - A x|| / ||b||, with z and the partial arrays of the work memory
         const unsigned rb = spmv_blocks(64, n);
         residual64(n, a->outer.p, spmv_cols(a), a->val.p, pick_lpr(a), x, b, cg.z, cg.part1, cg.part2, rb, s);
@@ -1726,11 +1726,11 @@ int nlf_cg_solve(nlf_matrix a, nlf_precond p, const double* b, double* x, double
         nlf_solve_stats out{};
         out.preconditioner = p ? p->kind : NLF_PRECOND_IDENTITY;
         int breakdown = 0;
-        auto timings = [&](const KernelTimer& t, size_t sv, size_t sx) {
+        auto timings = [&](const KernelTimer& t, size_t sv, size_t sx, bool slices) {
             out.spmv_ms = t.avg(0);
             out.precond_ms = t.avg(1);
             out.spmv_samples = t.count[0];
-            out.spmv_bytes = spmv_stream_bytes(a, sv, sx);
+            out.spmv_bytes = spmv_stream_bytes(a, sv, sx, slices);
         };
         if (mode == NLF_MODE_FP64) {
             CG<double, double> cg(s, n, a->nnz_full, a->outer.p, a->cols.p, a->val.p, p);
@@ -1738,7 +1738,7 @@ int nlf_cg_solve(nlf_matrix a, nlf_precond p, const double* b, double* x, double
             if (symv_prepare(a, s)) cg.set_symmetric(a);
             else cg.set_cols(a);
             out.iterations = cg.solve(b, x, tol, max_it, &out.residual, &breakdown);
-            timings(cg.timer, sizeof(double), sizeof(double));
+            timings(cg.timer, sizeof(double), sizeof(double), cg.sym != nullptr);
         } else {
             NLF_CHECK(mode == NLF_MODE_MIXED || mode == NLF_MODE_SPLIT, NLF_ERR_ARGUMENT, "unknown mode");
             NLF_CHECK(a->val32.p, NLF_ERR_STATE, "mixed mode needs nlf_matrix_make_fp32 first");
@@ -1757,7 +1757,7 @@ int nlf_cg_solve(nlf_matrix a, nlf_precond p, const double* b, double* x, double
             out.iterations = cg.solve_reliable(a->outer.p, a->cols.p, a->val.p, b, x, tol, max_it, 0.1,
                                                &out.true_residual, &out.outer_iterations, &breakdown);
             out.residual = out.true_residual;
-            timings(cg.timer, mode == NLF_MODE_SPLIT ? sizeof(float) + sizeof(int16_t) : sizeof(float), sizeof(double));
+            timings(cg.timer, mode == NLF_MODE_SPLIT ? sizeof(float) + sizeof(int16_t) : sizeof(float), sizeof(double), sym.on);
         }
         // FP64 true residual ||b - A x|| / ||b||
         {

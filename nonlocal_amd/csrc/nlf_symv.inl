@@ -583,6 +583,28 @@ static void symv_fill_low(nlf_matrix_s* a, SymValues which, hipStream_t s) {
     NLF_HIP(hipGetLastError());
 }
 
+// Whether a solve with these values is faster on the slices.  Small systems are not: a slice is a chain of trips
+// and a reduction follows, while the full storage comes from the cache.  us per iteration, slices / full storage:
+//   FP32 values, by their size in the full storage, Jacobi: 24 MB (120 x 120 nodes, 9.3 elements' reach) 36.4 / 24.7,
+//   51 MB (300 x 300, 4.1) 34.4 / 33.4, 93 MB (233 x 233, 9.3) 42.2 / 44.1, 155 MB (300 x 300, 9.3) 54.9 / 59.7,
+//   283 MB (700 x 700, 4.1) 78 / 112;
+//   split values, whose remainders are a second stream: 139 MB 59.6 / 48.1, 233 MB 70.5 / 65.9, 318 MB (700 x 700,
+//   3.1) 101 / 125, 417 MB (400 x 400, 9.3) 106 / 137.
+// FP64 values take the slices at any size (120 x 120, 9.3: 33.4 / 25.5; 300 x 300, 9.3: 65.9 / 85.2).
+constexpr i64 SYMV_FP32_BYTES = i64(96) << 20, SYMV_SPLIT_BYTES = i64(256) << 20;
+static bool symv_pays(const nlf_matrix_s* a, SymValues which) {
+    if (which == SYM_FP32) return a->nnz_full * i64(sizeof(float)) >= SYMV_FP32_BYTES;
+    if (which == SYM_SPLIT) return a->nnz_full * i64(sizeof(float) + sizeof(int16_t)) >= SYMV_SPLIT_BYTES;
+    return true;
+}
+
+// A batch's full-storage product is slower (a nonzero at a time), so its limit is lower, where about two slices fall
+// to a compute unit.  ms per solve, slices / full storage, FP64 and FP32 values, by slices: 125 (5 instances of 32 to
+// 45 a side) 3.6 / 2.5 and 4.9 / 3.2; 550 (32 of 24 to 40) 3.3 / 3.3 and 4.5 / 4.1; 652 (5 of 32 to 150) 10.5 / 15.1
+// and 15.8 / 21.4; 817 (48 of 32) 3.0 / 3.4 and 4.2 / 4.5; 1089 (64 of 32) 4.0 / 5.6 and 5.7 / 8.1.
+constexpr i64 SYMV_BATCH_SLICES = 600;
+static bool symv_pays_batch(const nlf_matrix_s* a) { return (a->rows + 63) / 64 >= SYMV_BATCH_SLICES; }
+
 // The slices of one solve, with the values it reads.  Reduced values are filled anew for each solve (one pass over
 // the upper triangle), so they never lag behind the matrix's, and given back at its end.  What the solve allocates
 // itself it allocates first: a solve that fits with the full storage then runs with it where the slices do not fit
@@ -591,7 +613,8 @@ struct SymSolve {
     nlf_matrix_s* a;
     SymValues which;
     bool on;
-    SymSolve(nlf_matrix_s* a_, SymValues w, hipStream_t s) : a(a_), which(w), on(symv_prepare(a_, s)) {
+    SymSolve(nlf_matrix_s* a_, SymValues w, hipStream_t s, bool batch = false)
+        : a(a_), which(w), on((batch ? symv_pays_batch(a_) : symv_pays(a_, w)) && symv_prepare(a_, s)) {
         if (!on || which == SYM_FP64) return;
         try {
             symv_fill_low(a, which, s);

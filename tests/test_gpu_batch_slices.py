@@ -10,9 +10,10 @@ from tests.helpers import direct_solution, oracle_assembly, rel_l2
 
 pytestmark = pytest.mark.gpu
 
-SIDES = [40, 32, 37, 33]
+SIDES = [140, 97, 113, 89]                 # 792 slices of 64 rows: a batch reads them from 600
 BAD = 1
-BOUND = {A.NLF_MODE_FP64: 1e-10, A.NLF_MODE_MIXED: 1e-8}
+TOL = 1e-12
+BOUND = 4 * 140 ** 2 * TOL                 # the error of a solution: the condition number times its residual
 
 
 def _instances(lam=1.0):
@@ -46,11 +47,11 @@ def test_instances_stay_apart(gpu_ctx, references, precond, mode, what):
     if what != "conductivity":
         (solver.b if what == "load" else x0)[(begin + end) // 2] = float("nan")
         (solver.b if what == "load" else x0)[[begin, end - 1]] = float("nan")
-    x, its, res, st = solver.solve(tol=1e-12, mode=mode, x0=x0)
+    x, its, res, st = solver.solve(tol=TOL, mode=mode, x0=x0)
     for i, (xi, ref) in enumerate(zip(solver.split(x), references)):
         if i != BAD:
-            assert res[i] <= 1e-12, f"instance {i}"
-            assert rel_l2(xi.cpu().numpy(), ref) < BOUND[mode], f"instance {i}"
+            assert res[i] <= TOL, f"instance {i}"
+            assert rel_l2(xi.cpu().numpy(), ref) < BOUND, f"instance {i}"
 
 
 def test_autotuner_has_nothing_to_choose(gpu_ctx, tmp_path):
