@@ -398,7 +398,6 @@ struct nlf_batch_s {
     nlf_matrix A = nullptr;
     nlf::BatchPlan plan;
     nlf::DevBuf<double> invd;
-    nlf::DevBuf<float> invd32;
     double tune_seconds = 0.0;
     nlf_precond precond = nullptr;       // ILLT of the batch's local matrix (nlf_batch_set_preconditioner), or Jacobi
 };
@@ -548,9 +547,8 @@ int nlf_batch_create(nlf_matrix a, int count, const int64_t* row_begin, nlf_batc
         B->plan.row_begin_h.assign(row_begin, row_begin + count + 1);
         upload(B->plan.row_begin, row_begin, size_t(count) + 1, s);
         B->invd.alloc(size_t(a->rows));
-        B->invd32.alloc(size_t(a->rows));
         hipLaunchKernelGGL(k_inv_diag, dim3(blocks_for(a->rows, 256)), dim3(256), 0, s, a->rows, a->diag.p, a->val.p,
-                           B->invd.p, B->invd32.p);
+                           B->invd.p);
         batch_build_plan(B->plan, a, 4.0, s);
         NLF_HIP(hipGetLastError());
         NLF_HIP(hipStreamSynchronize(s));

@@ -446,14 +446,11 @@ __global__ void k_first_kind(i64 rows, const i64* __restrict__ bo, const i32* __
     f[r] = inner[r] ? f[r] - s : xD[r];
 }
 
-__global__ void k_inv_diag(i64 rows, const i64* __restrict__ diag, const double* __restrict__ val, double* __restrict__ inv,
-                           float* __restrict__ inv32) {
+__global__ void k_inv_diag(i64 rows, const i64* __restrict__ diag, const double* __restrict__ val, double* __restrict__ inv) {
     const i64 r = i64(blockIdx.x) * blockDim.x + threadIdx.x;
     if (r >= rows) return;
     const double d = val[diag[r]];
-    const double v = d != 0.0 ? 1.0 / d : 1.0;      // Eigen::DiagonalPreconditioner: 1 for zero diagonals
-    inv[r] = v;
-    inv32[r] = float(v);
+    inv[r] = d != 0.0 ? 1.0 / d : 1.0;              // Eigen::DiagonalPreconditioner: 1 for zero diagonals
 }
 
 // ---- IC(0) ------------------------------------------------------------------------------------
@@ -482,13 +479,11 @@ __global__ void k_ic_init(i64 rows, const i64* __restrict__ outer, const i32* __
     F[diag[r]] += shift;
 }
 
-__global__ void k_scale_from_diag(i64 rows, const i64* __restrict__ diag, const double* __restrict__ a, double* __restrict__ s,
-                                  float* __restrict__ s32) {
+__global__ void k_scale_from_diag(i64 rows, const i64* __restrict__ diag, const double* __restrict__ a, double* __restrict__ s) {
     const i64 r = i64(blockIdx.x) * blockDim.x + threadIdx.x;
     if (r >= rows) return;
     const double d = fabs(a[diag[r]]);
     s[r] = d > 0.0 ? 1.0 / sqrt(d) : 1.0;
-    s32[r] = float(s[r]);
 }
 
 // Up-looking IC(0): for row k (all rows i < k it depends on are done and mirrored into row k's
@@ -638,7 +633,6 @@ struct nlf_precond_s {
     double setup_seconds = 0.0;
     // Jacobi
     nlf::DevBuf<double> invd;
-    nlf::DevBuf<float> invd32;
     // ILLT
     int fw_levels = 0, bw_levels = 0;
     int blocks = 1;                      // independent diagonal blocks
@@ -1289,7 +1283,6 @@ struct CG {
 };
 
 template<> const double* CG<double, double>::invd() const { return P->invd.p; }
-template<> const float* CG<float, float>::invd() const { return P->invd32.p; }
 template<> const double* CG<float, double>::invd() const { return P->invd.p; }
 
 }  // namespace nlf
@@ -1443,9 +1436,7 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
         const i64 n = a->rows;
         if (kind == NLF_PRECOND_JACOBI) {
             P->invd.alloc(size_t(n));
-            P->invd32.alloc(size_t(n));
-            hipLaunchKernelGGL(k_inv_diag, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, a->diag.p, a->val.p, P->invd.p,
-                               P->invd32.p);
+            hipLaunchKernelGGL(k_inv_diag, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, a->diag.p, a->val.p, P->invd.p);
             NLF_HIP(hipGetLastError());
         } else if (kind == NLF_PRECOND_ILLT) {
             // pattern copy + level sets (host analysis of the pattern only)
@@ -1467,9 +1458,7 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
             hipLaunchKernelGGL(k_transpose_pos, dim3(blocks_for(n, 4)), dim3(256), 0, s, n, d_outer, d_cols, tpos.p);
             P->scale.alloc(size_t(n));
             P->F.alloc(cols.size());
-            DevBuf<float> scale32{size_t(n)};
-            hipLaunchKernelGGL(k_scale_from_diag, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, d_diag, a->val.p,
-                               P->scale.p, scale32.p);
+            hipLaunchKernelGGL(k_scale_from_diag, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, d_diag, a->val.p, P->scale.p);
             DevBuf<int> fail{1};
             // factorisation with growing shift until no pivot fails
             auto factor = [&](auto&& attempt_with) {
