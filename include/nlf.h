@@ -152,7 +152,7 @@ int         nlf_ctx_create(int device, void* stream, nlf_ctx* out);
 int         nlf_ctx_destroy(nlf_ctx ctx);
 const char* nlf_last_error(nlf_ctx ctx);
 int         nlf_ctx_synchronize(nlf_ctx ctx);
-#define NLF_OPT_ASSEMBLY_PAIRS 1     /* 1: MFMA element-pair contractions (thermal Q4), 0: node-centric */
+#define NLF_OPT_ASSEMBLY_PAIRS 1     /* 1: MFMA element-pair contractions (thermal Q4, and Q8 in FP64), 0: node-centric */
 #define NLF_OPT_ROW_PATTERNS   2     /* 1: SpMV column offsets from a dictionary of distinct rows, 0: per nonzero */
 #define NLF_OPT_ASSEMBLY_THREADS 3   /* threads per node workgroup of the value pass: 64 (default), 128, 256, 512 */
 #define NLF_OPT_PATTERN_THREADS  4   /* threads per node workgroup of the pattern build: 64, 128 (default), 256 */
@@ -327,7 +327,8 @@ int nlf_precond_info(nlf_precond p, int* ok, double* shift, int* fw_levels, int*
 int nlf_precond_sweep_info(nlf_precond p, int32_t out[8]);
 /* No reference counterpart: the independent diagonal blocks an ILLT found in its matrix (contiguous
  * row ranges with no entry between them, such as a batch's instances, of at least 1024 rows each),
- * factored and swept side by side in chunks of their own; 1 for a connected matrix. */
+ * factored and swept side by side in chunks of their own (with a row of more than 32 dependencies: factored
+ * by a workgroup each, swept by one workgroup for all); 1 for a connected matrix. */
 int nlf_precond_blocks(nlf_precond p, int32_t* blocks);
 int nlf_precond_apply(nlf_precond p, const double* r_dev, double* z_dev);
 int nlf_precond_export_factor(nlf_precond p, double* values, double* scale);

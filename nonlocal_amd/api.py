@@ -409,7 +409,8 @@ class preconditioner:
 
     def blocks(self):
         """Independent diagonal blocks of an ILLT's matrix, factored and swept side by side in chunks
-        of their own (nlf_precond_blocks)."""
+        of their own; with a row of more than 32 dependencies factored by a workgroup each and swept by
+        one for all (nlf_precond_blocks)."""
         out = C.c_int32()
         self.ctx.check(load().nlf_precond_blocks(self.h, C.byref(out)))
         return out.value

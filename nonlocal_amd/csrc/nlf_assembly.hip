@@ -514,9 +514,9 @@ struct AssemblyArgs {
     double* b_val;
     float* val32;        // FP32 value pass: inner values only (the bound part stays FP64)
     int local_only;      // assemble_part::LOCAL: every group treated as LOCAL
-    const double* pairs; // thermal Q4: nonlocal pair blocks from k_pairs_mfma (null = compute in place)
+    const double* pairs; // thermal: nonlocal pair blocks of k_pairs_mfma or k_pairs8_mfma (null = compute in place)
     const float* pairs32;
-    i64 plane;           // pairs[i * plane + (eoff[eL] + t) * 4 + j], t = position in eL's neighbour list
+    i64 plane;           // pairs[i * plane + (eoff[eL] + t) * nn + j], t = position in eL's neighbour list
     const i64* eoff;
     i64 node0;           // nodes [node0, node0 + grid) of this launch
     int mass;            // heat capacity matrix: rho c int N_i N_j (groups' c[0] = rho c)
@@ -640,7 +640,7 @@ __device__ void nonlocal_row(const AssemblyArgs& a, const GroupParams& g, const 
         for (int k = 0; k < DOF * DOF; ++k) v[j][k] *= s;
 }
 
-// ---- MFMA element-pair contractions (thermal Q4) -------------------------------------------------
+// ---- MFMA element-pair contractions (thermal Q4; Q8 in FP64: k_pairs8_mfma) -----------------------
 // For a pair (eL, eNL) of one group the nonlocal block is
 //   K_ij = (1 - p1) sum_k sum_qn sum_ql Phi[ql][qn] HL_k[i][ql] HN_k[j][qn]
 // with HL_k[i][q] = w_q D_i(q)_k and HN_k[j][q] = w_q (C D_j(q))_k (conductivity_matrix_2d.hpp:132-164,
@@ -1020,7 +1020,7 @@ __global__ __launch_bounds__(THREADS) void k_assemble(AssemblyArgs a) {
         // ITEMS neighbours per thread and step: item u covers [base + u blockDim, base + (u + 1) blockDim),
         // their loads are issued before either is used, and they are added item after item, so the
         // order of the additions is that of ITEMS consecutive single-item steps
-        // (PAIRS: the nonlocal rows come from the pair blocks of k_pairs_mfma, thermal Q4 only)
+        // (PAIRS: the nonlocal rows come from the pair blocks, thermal Q4, and Q8 in FP64)
         constexpr int ITEMS = PAIRS ? NLF_ASM_PAIR_ITEMS : 1;
         const T* pairs = nullptr;
         if constexpr (F64) pairs = a.pairs; else pairs = a.pairs32;
@@ -1663,11 +1663,12 @@ void border_neumann(nlf_matrix_s* mat, hipStream_t s) {
 
 // Value pass on the matrix's pattern.  T = double fills val and b_val (and the 16-bit column
 // offsets); T = float fills val32 with FP32 contractions and FP32 accumulation.  Thermal Q4
-// nonlocal blocks go through the MFMA pair kernel when its pair buffer (16 values per neighbour
-// pair) fits in half of the free device memory; option NLF_OPT_ASSEMBLY_PAIRS = 0 forces the
-// node-centric contraction.
+// nonlocal blocks, and Q8 ones in FP64, go through the MFMA pair kernels (nn * nn values per
+// neighbour pair, within the budget of pair_budget, chunk by chunk where they need more); option
+// NLF_OPT_ASSEMBLY_PAIRS = 0 forces the node-centric contraction, which also takes over where there
+// is no memory for the blocks.
 // Node chunks of the MFMA pair assembly.  An element's blocks take its neighbour count rounded up
-// to a multiple of four slots (k_pairs_mfma writes runs of four).  single: every element's blocks
+// to a multiple of four slots (k_pairs_mfma writes runs of four; Q8 keeps the same slots).  single: every element's blocks
 // (all_pairs slots) fit the budget, one pass over all elements.  Otherwise a chunk is a run of nodes [n0, n1) whose
 // elements' blocks fit the budget: list[lbeg, lend) are its elements (each once, ascending by first
 // touching node) and cofs their first block slot within the chunk.

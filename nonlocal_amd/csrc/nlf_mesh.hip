@@ -346,7 +346,7 @@ int nlf_ctx_destroy(nlf_ctx ctx) {
 const char* nlf_last_error(nlf_ctx ctx) { return ctx ? ctx->error.c_str() : "null context"; }
 
 // Context options (no reference counterpart): NLF_OPT_ASSEMBLY_PAIRS 1 = MFMA element-pair
-// contractions where implemented (thermal Q4, default), 0 = node-centric contraction;
+// contractions where implemented (thermal Q4, and Q8 in FP64; default), 0 = node-centric contraction;
 // NLF_OPT_ROW_PATTERNS 1 = shared row-pattern dictionary for the SpMV of matrices assembled
 // afterwards (default), 0 = per-nonzero 16-bit offsets; NLF_OPT_ASSEMBLY_THREADS = threads per
 // node workgroup of the node-centric value pass (64 default, 128, 256, 512); NLF_OPT_PATTERN_THREADS

@@ -11,8 +11,9 @@
 // ILLT: IC(0) of the local matrix, diagonal scaling s = 1/sqrt|a_ii| and shift retries (our choice:
 // Eigen::IncompleteCholesky is not vendored, so its factor is not reproduced).  Rows are grouped by
 // dependency level (computed once on the host from the pattern).  The factorisation and the triangular
-// sweeps run as dataflows over chunks of rows (nlf_sweep.inl); with more than 32 dependencies in a row, as one
-// 1024-thread workgroup per independent block with a barrier between levels.
+// sweeps run as dataflows over chunks of rows (nlf_sweep.inl).  With more than 32 dependencies in a row the levels
+// are taken one after the other with a barrier between them: the factorisation by a 1024-thread workgroup for each
+// independent block, the sweeps by one workgroup for all rows.
 #include "nlf_internal.hpp"
 
 #include <mutex>
@@ -454,10 +455,10 @@ __global__ void k_inv_diag(i64 rows, const i64* __restrict__ diag, const double*
 }
 
 // ---- IC(0) ------------------------------------------------------------------------------------
-// One independent diagonal block of a block-diagonal factor, factored and swept by a workgroup of
-// its own: its level count, sweep window depth and first level offset (into the shared offsets).
+// One independent diagonal block of a block-diagonal factor, factored by a workgroup of its own: its
+// level count and first level offset (into the shared offsets).
 struct SweepBlock {
-    i32 levels, K, lptr_off, pad;
+    i32 levels, lptr_off;
 };
 
 struct LevelArgs {
@@ -1077,7 +1078,9 @@ constexpr i64 SYMV_REDUCE_BLOCKS = 2048;
 // Above this size the full storage's values bypass the caches in a solve with sweeps: the last-level cache
 // holds 256 MB, a smaller matrix is read from it again, a larger one only drives out the factor that the
 // sweeps read next, whose loads' latency bounds them.  Q8 sheets, us per iteration without / with: 31 000
-// rows (112 MB) 259 / 271, 44 000 (204 MB) 352 / 363, 59 000 (352 MB) 550 / 447, 121 000 (1264 MB) 978 / 809.
+// rows (112 MB) 259 / 271, 44 000 (204 MB) 352 / 363, 59 000 (352 MB) 550 / 447, 121 000 (1264 MB) 978 / 809; with
+// FP32 values 77 000 (302 MB) 647 / 539, 98 000 (451 MB) 780 / 640, 121 000 (663 MB) 926 / 766.  Split values are not
+// read so.
 constexpr i64 SPMV_NT_BYTES = i64(256) << 20;
 
 // Preconditioned CG on device vectors (conjugate_gradient::solve).  Vectors of type X, matrix values V.
@@ -1491,7 +1494,7 @@ int nlf_precond_create(nlf_matrix a, int kind, nlf_precond* out) {
                 std::vector<SweepBlock> bd;
                 if (P->blocks > 1) {
                     bl = block_levels(fr, fp, bounds);
-                    for (int b = 0; b < P->blocks; ++b) bd.push_back(SweepBlock{bl.levels[size_t(b)], 0, i32(bl.seg[size_t(b)]), 0});
+                    for (int b = 0; b < P->blocks; ++b) bd.push_back(SweepBlock{bl.levels[size_t(b)], i32(bl.seg[size_t(b)])});
                     upload(blk, bd.data(), bd.size(), s);
                     upload(lrows, bl.rows.data(), bl.rows.size(), s);
                     upload(lptr, bl.ptr.data(), bl.ptr.size(), s);

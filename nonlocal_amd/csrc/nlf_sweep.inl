@@ -600,8 +600,10 @@ static bool plan_sweep(const std::vector<i64>& outer, const std::vector<i32>& co
 // a memory round trip per level: with one workgroup and one thread per row, a row's entries and merges were
 // serial loads (30 us per level at 200 x 200 Q8).  No barrier: like the sweeps, a value is its own flag and
 // is read again until it is there, each wave going through the steps by itself.  Whole set-up of the
-// preconditioner, host analysis included, before and after: 200 x 200 Q8 57 -> 14.5 ms, 220 x 220 plane
-// stress 58 -> 12.6 ms, 500 x 500 Q4 30 -> 15 ms, 1000 x 1000 Q4 152 -> 109 ms, 40 x 40 Q4 1.4 -> 0.6 ms.
+// preconditioner, host analysis included, before and after: 200 x 200 Q8 59 -> 25 ms, 220 x 220 plane
+// stress 49 -> 19.5 ms (of these two, 11 and 7 ms are the host's, for merging rows and for a plan of the
+// factorisation without merged ones), 500 x 500 Q4 26 -> 15 ms, 1000 x 1000 Q4 154 -> 106 ms, 40 x 40 Q4
+// 1.2 -> 0.6 ms.
 //
 // Entry m of lane l's list: the position in row j (the column of entry l above the diagonal) of column
 // cols[outer[k] + m], -1 where row j lacks it.

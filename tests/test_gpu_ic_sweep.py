@@ -4,10 +4,10 @@ layout, with nlf_precond_sweep_info naming the kernel that ran:
 
 - the 1000 x 1000 composite of the benchmark: its level 0 (the rows with no dependency, the
   first-kind column among them) is twice as wide as any other level and is split, so both sweeps
-  take the prefetching kernel at a width of 512;
+  have levels of at most 512 records;
 - a square with first-kind conditions on all four sides, whose level 0 is wider than the largest
   workgroup (split into several levels);
-- Q8 and plane-stress rows (up to 16 entries below the diagonal), which take shallower prefetch.
+- Q8 and plane-stress rows (up to 16 entries below the diagonal), which hold fewer steps in flight.
 
 The arithmetic of every record is the same in every kernel, so z is held to 1e-12 relative to the
 oracle as for the other layouts."""
@@ -52,7 +52,7 @@ def test_ic_sweep_matches_oracle(gpu_ctx, name, build, width, split):
     info = Pg.sweep_info()
     print(f"  sweeps {info}", flush=True)
     for sweep in ("forward", "backward"):
-        assert info[sweep]["kernel"] == 2, f"{sweep} sweep did not take the prefetching kernel"
+        assert info[sweep]["kernel"] == 2, f"{sweep} sweep did not take the chunked kernel"
         if width is not None:
             assert info[sweep]["width"] == width
     if split:
@@ -70,7 +70,7 @@ def test_ic_sweep_matches_oracle(gpu_ctx, name, build, width, split):
 
 def test_ic_of_independent_blocks(gpu_ctx):
     """A block-diagonal matrix (four thermal instances of 1089 to 1681 nodes concatenated as in a
-    batch) is factored and swept block by block, one workgroup per block: its IC(0) is the blocks'
+    batch) is factored and swept in chunks that end with a block: its IC(0) is the blocks'
     own, so z is every instance's oracle apply in turn."""
     from nonlocal_amd import batch
     problems = [configs.thermal_q4(n, 0.6, 2.0 / n, 1.0 + 0.1 * k, name=f"i{k}") for k, n in enumerate([35, 32, 40, 33])]
