@@ -31,6 +31,24 @@ def references():
     return refs
 
 
+@pytest.mark.parametrize("mode", [A.NLF_MODE_FP64, A.NLF_MODE_MIXED])
+@pytest.mark.parametrize("precond", [A.NLF_PRECOND_JACOBI, A.NLF_PRECOND_ILLT])
+def test_graph_replays_and_solutions(gpu_ctx, references, precond, mode):
+    """The oracle's solutions from graph replays, the same bits from eager launches and from a second graph."""
+    print(f"[batch slices] graph, precond {precond} mode {mode}", flush=True)
+    solver = batch.BatchSolver(_instances(), gpu_ctx, precond=precond)
+    assert solver.K.symv_info() is not None
+    x, its, res, st = solver.solve(tol=TOL, mode=mode)
+    assert res.max() <= TOL and st.preconditioner == precond
+    for i, (xi, ref) in enumerate(zip(solver.split(x), references)):
+        assert rel_l2(xi.cpu().numpy(), ref) < BOUND, f"instance {i}"
+    eager, its_e, _, _ = solver.solve(tol=TOL, mode=mode, use_graph=False)
+    torch.cuda.synchronize()
+    again, its_a, _, _ = solver.solve(tol=TOL, mode=mode)
+    assert torch.equal(x, eager) and torch.equal(x, again)
+    assert np.array_equal(its, its_e) and np.array_equal(its, its_a)
+
+
 # (no ILLT with the conductivity: one factorisation serves the batch, fails and says so)
 @pytest.mark.parametrize("precond,what", [(A.NLF_PRECOND_JACOBI, "load"), (A.NLF_PRECOND_JACOBI, "start"),
                                           (A.NLF_PRECOND_JACOBI, "conductivity"), (A.NLF_PRECOND_ILLT, "load"),
