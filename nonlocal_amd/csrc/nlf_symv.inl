@@ -452,8 +452,10 @@ void symv_release(nlf_matrix_s* a) {
 
 // Longest window of a slice (doubles, 56 KB of the 64 KB of LDS that a launch may ask for): a reach of about
 // 30 elements on a structured mesh.  256 x 256 nodes with 25.6 elements' reach: 270 us from the full storage,
-// 163 us here (windows of 4600 doubles, four workgroups to a compute unit).
-constexpr i64 SYMV_WINDOW = 7168;
+// 163 us here (windows of 4600 doubles, four workgroups to a compute unit).  A long window is a long chain, so one
+// over SYMV_NARROW takes two slices to a compute unit: us per product, here / full storage, at 30.3 elements' reach,
+// 100 x 100 nodes (160 slices) 105 / 37, 160 x 160 (406) 128 / 128, 180 x 180 (512) 133 / 164, 300 x 300 308 / 473.
+constexpr i64 SYMV_WINDOW = 7168, SYMV_NARROW = 2048, SYMV_WIDE_SLICES = 512;
 
 // The storage where it applies, in a->symv; false where it does not.
 static bool symv_build(nlf_matrix_s* a, hipStream_t s) {
@@ -485,7 +487,7 @@ static bool symv_build(nlf_matrix_s* a, hipStream_t s) {
     const i64 upper_offdiag = a->nnz_upper - rows;
     // bytes: 8 per slot of 64 values and the strips twice, against 8 per full-storage value
     const double sym_bytes = double(slots) * 64.0 * 8.0 + 2.0 * 8.0 * double(std::accumulate(hW.begin(), hW.end(), i64(0)));
-    if (maxb > 255 || maxw > SYMV_WINDOW || sym_bytes > 0.75 * 8.0 * double(a->nnz_full) || upper_offdiag <= 0) return refuse();
+    if (maxb > 255 || maxw > (ns < SYMV_WIDE_SLICES ? SYMV_NARROW : SYMV_WINDOW) || sym_bytes > 0.75 * 8.0 * double(a->nnz_full) || upper_offdiag <= 0) return refuse();
     auto sv = std::make_unique<nlf_symv_s>();
     sv->ns = ns;
     sv->wmax = int(maxw);
@@ -547,7 +549,7 @@ static bool symv_refuse(nlf_matrix_s* a) {
 
 // Builds (or rebuilds, when the values changed) the symmetric SpMV storage of a FP64 matrix.  Returns
 // false, with nothing kept, where it does not apply: offsets of 2^15 or more, more than 255 bands in a
-// slice, a window over SYMV_WINDOW doubles, padding that leaves less than a quarter of the traffic saved, or no
+// slice, a window over SYMV_WINDOW doubles (SYMV_NARROW in a small system), padding that leaves less than a quarter of the traffic saved, or no
 // memory for it.
 bool symv_prepare(nlf_matrix_s* a, hipStream_t s) {
     if (!a->ctx->spmv_symmetric || a->rows <= 0 || !a->val.p || a->nnz_full <= 0) return false;
@@ -584,17 +586,19 @@ static void symv_fill_low(nlf_matrix_s* a, SymValues which, hipStream_t s) {
 }
 
 // Whether a solve with these values is faster on the slices.  Small systems are not: a slice is a chain of trips
-// and a reduction follows, while the full storage comes from the cache.  us per iteration, slices / full storage:
-//   FP32 values, by their size in the full storage, Jacobi: 24 MB (120 x 120 nodes, 9.3 elements' reach) 36.4 / 24.7,
-//   51 MB (300 x 300, 4.1) 34.4 / 33.4, 93 MB (233 x 233, 9.3) 42.2 / 44.1, 155 MB (300 x 300, 9.3) 54.9 / 59.7,
-//   283 MB (700 x 700, 4.1) 78 / 112;
-//   split values, whose remainders are a second stream: 139 MB 59.6 / 48.1, 233 MB 70.5 / 65.9, 318 MB (700 x 700,
-//   3.1) 101 / 125, 417 MB (400 x 400, 9.3) 106 / 137.
-// FP64 values take the slices at any size (120 x 120, 9.3: 33.4 / 25.5; 300 x 300, 9.3: 65.9 / 85.2).
-constexpr i64 SYMV_FP32_BYTES = i64(96) << 20, SYMV_SPLIT_BYTES = i64(256) << 20;
+// and a reduction follows, while the full storage comes from the cache.  us per iteration with Jacobi, slices / full
+// storage, on n x n nodes with a reach of r elements, (n + 1)^2 / 64 slices:
+//   FP32 values, MiB in the full storage: n 120 r 9.3 (23) 36.4 / 24.7; 190, 22.3 (241) 99 / 81; 190, 28.3 (361) 132 /
+//   153; 233, 13.3 (156) 59 / 57; 250, 17.3 (280) 85 / 120; 260, 9.3 (111) 47 / 52; 270, 7.3 (85) 41 / 45; 300, 4.1
+//   (49) 34.4 / 33.4; 300, 25.3 (780) 166 / 320; 700, 0.6 (70) 53.8 / 51.7; 700, 4.1 (270) 78 / 112;
+//   split values, whose remainders are a second stream: 190, 28.3 (541) 240 / 180; 250, 22.3 (644) 193 / 191; 270,
+//   17.3 (492) 144 / 169; 300, 9.3 (222) 70 / 65; 300, 12.3 (349) 94 / 112; 700, 3.1 (303) 101 / 125.
+// FP64 values take the slices at any size (n 120 r 9.3: 33.4 / 25.5; 300, 9.3: 65.9 / 85.2).
 static bool symv_pays(const nlf_matrix_s* a, SymValues which) {
-    if (which == SYM_FP32) return a->nnz_full * i64(sizeof(float)) >= SYMV_FP32_BYTES;
-    if (which == SYM_SPLIT) return a->nnz_full * i64(sizeof(float) + sizeof(int16_t)) >= SYMV_SPLIT_BYTES;
+    const i64 ns = (a->rows + 63) / 64, mib = i64(1) << 20;
+    const i64 full = a->nnz_full * i64(which == SYM_FP32 ? sizeof(float) : sizeof(float) + sizeof(int16_t));
+    if (which == SYM_FP32) return (ns >= 1024 && full >= 80 * mib) || (ns >= 512 && full >= 256 * mib);
+    if (which == SYM_SPLIT) return ns >= 1024 && full >= 256 * mib;
     return true;
 }
 

@@ -52,7 +52,7 @@ def without_slices(ctx, make, solve, reduced):
 @pytest.mark.parametrize("mode,reduced", [(m, False) for m in MODES] + [(m, True) for m in MODES[1:]])
 def test_cg(gpu_ctx, mode, reduced):
     print(f"[memory limit] cg mode {mode} reduced {reduced}", flush=True)
-    n = {A.NLF_MODE_FP64: 100, A.NLF_MODE_MIXED: 250, A.NLF_MODE_SPLIT: 330}[mode]     # sizes that take the slices
+    n = {A.NLF_MODE_FP64: 100, A.NLF_MODE_MIXED: 270, A.NLF_MODE_SPLIT: 380}[mode]     # sizes that take the slices
     problem = configs.thermal_q4(n, 0.5, 9.3 / n)
     g = api.mesh_2d(problem.mesh, gpu_ctx)
     api._search(g, problem.models)
@@ -81,7 +81,7 @@ def test_flexible_cg(gpu_ctx, mode, reduced):
     print(f"[memory limit] flexible cg mode {mode} reduced {reduced}", flush=True)
 
     def make():
-        n = 96 if mode == A.NLF_MODE_FP64 else 250
+        n = 96 if mode == A.NLF_MODE_FP64 else 270
         tp = learned.TrainingProblem(n, seed=1, ctx=gpu_ctx, count=3, r=(5.3 if n == 96 else 11.3) / n)
         tp.K.make_fp32()
         tp.K.problem = tp
