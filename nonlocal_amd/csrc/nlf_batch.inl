@@ -424,7 +424,7 @@ i64 batch_cg(nlf_batch B, const V* val, const double* b, double* x, double tol, 
     // a side, FP32 values: 630 -> 297 ms for assembly and solve, 560 ms of it left with the full storage); a slice whose instances are all done is passed over.
     DevBuf<int2> slice_inst{size_t((n + 63) / 64)};
     const SymValues which = std::is_same_v<V, double> ? SYM_FP64 : SYM_FP32;
-    const SymSolve slices(A, which, s, true);
+    const SymSolve slices(A, which, s, count);
     const bool sym = slices.on;
     SymSkip live{nullptr, nullptr, 0};
     if (sym) {
@@ -594,7 +594,7 @@ int nlf_batch_autotune(nlf_batch b, const char* cache_path, double* chosen) {
             }
         }
         const auto t0 = std::chrono::steady_clock::now();
-        if (!found && symv_pays_batch(A) && symv_prepare(A, s)) {
+        if (!found && symv_pays_batch(A, P.count) && symv_prepare(A, s)) {
             best_t = P.target;
         } else if (!found) {
             DevBuf<double> x{size_t(A->rows)}, y{size_t(A->rows)};

@@ -603,11 +603,15 @@ static bool symv_pays(const nlf_matrix_s* a, SymValues which) {
 }
 
 // A batch's full-storage product is slower (a nonzero at a time), so its limit is lower, where about two slices fall
-// to a compute unit.  ms per solve, slices / full storage, FP64 and FP32 values, by slices: 125 (5 instances of 32 to
-// 45 a side) 3.6 / 2.5 and 4.9 / 3.2; 550 (32 of 24 to 40) 3.3 / 3.3 and 4.5 / 4.1; 652 (5 of 32 to 150) 10.5 / 15.1
-// and 15.8 / 21.4; 817 (48 of 32) 3.0 / 3.4 and 4.2 / 4.5; 1089 (64 of 32) 4.0 / 5.6 and 5.7 / 8.1.
-constexpr i64 SYMV_BATCH_SLICES = 600;
-static bool symv_pays_batch(const nlf_matrix_s* a) { return (a->rows + 63) / 64 >= SYMV_BATCH_SLICES; }
+// to a compute unit; small instances, whose slices span rows of nodes of two of them and pad more, reach it later.
+// ms per solve, slices / full storage, FP64 and FP32 values, by slices: 125 (5 instances of 32 to 45 a side) 3.6 / 2.5
+// and 4.9 / 3.2; 355 (3 of 86, 12 elements' reach) 10.1 / 9.5 and 15.9 / 14.0; 462 (7 of 64) 4.2 / 5.0 and 7.2 / 7.7;
+// 462 (5 of 32 to 120) 7.5 / 10.0 and 11.7 / 14.3; 529 (16 of 45) 6.2 / 6.4 and 9.9 / 9.9; 550 (32 of 24 to 40) 3.3 /
+// 3.3 and 4.5 / 4.1; 817 (48 of 32) 3.0 / 3.4 and 4.2 / 4.5; 1089 (64 of 32) 4.0 / 5.6 and 5.7 / 8.1.
+static bool symv_pays_batch(const nlf_matrix_s* a, int count) {
+    const i64 ns = (a->rows + 63) / 64;
+    return ns >= 600 || (ns >= 400 && a->rows >= 4096 * i64(count));
+}
 
 // The slices of one solve, with the values it reads.  Reduced values are filled anew for each solve (one pass over
 // the upper triangle), so they never lag behind the matrix's, and given back at its end.  What the solve allocates
@@ -617,8 +621,9 @@ struct SymSolve {
     nlf_matrix_s* a;
     SymValues which;
     bool on;
-    SymSolve(nlf_matrix_s* a_, SymValues w, hipStream_t s, bool batch = false)
-        : a(a_), which(w), on((batch ? symv_pays_batch(a_) : symv_pays(a_, w)) && symv_prepare(a_, s)) {
+    // batch: the instances of a batch, 0: no batch
+    SymSolve(nlf_matrix_s* a_, SymValues w, hipStream_t s, int batch = 0)
+        : a(a_), which(w), on((batch ? symv_pays_batch(a_, batch) : symv_pays(a_, w)) && symv_prepare(a_, s)) {
         if (!on || which == SYM_FP64) return;
         try {
             symv_fill_low(a, which, s);

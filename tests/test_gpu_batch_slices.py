@@ -10,7 +10,7 @@ from tests.helpers import direct_solution, oracle_assembly, rel_l2
 
 pytestmark = pytest.mark.gpu
 
-SIDES = [140, 97, 113, 89]                 # 792 slices of 64 rows: a batch reads them from 600
+SIDES = [140, 97, 113, 89]                 # 792 slices of 64 rows: a batch reads them from 600 at the latest
 BAD = 1
 TOL = 1e-12
 BOUND = 4 * 140 ** 2 * TOL                 # the error of a solution: the condition number times its residual
@@ -70,6 +70,26 @@ def test_instances_stay_apart(gpu_ctx, references, precond, mode, what):
         if i != BAD:
             assert res[i] <= TOL, f"instance {i}"
             assert rel_l2(xi.cpu().numpy(), ref) < BOUND, f"instance {i}"
+
+
+@pytest.mark.parametrize("sides,slices", [([32] * 35, False), ([32] * 36, True), ([72] * 4, False), ([64] * 7, True)])
+def test_storage_by_size(gpu_ctx, sides, slices):
+    """Small batches read the full storage, larger ones (600 slices; 400 with 4096 rows an instance) the slices: the
+    bits tell which, and the solutions are the same."""
+    problems = [configs.thermal_q4(n, 0.5, 3.3 / n, 1.0 + 0.01 * k, name=f"t{k}") for k, n in enumerate(sides)]
+    solver = batch.BatchSolver(problems, gpu_ctx)
+    rows = int(solver.node_begin[-1])
+    print(f"[batch slices] {len(sides)} of {sides[0]}: {(rows + 63) // 64} slices, {rows // len(sides)} rows each", flush=True)
+    x, its, res, st = solver.solve(tol=TOL, mode=A.NLF_MODE_MIXED)
+    gpu_ctx.set_option(A.NLF_OPT_SPMV_SYMMETRIC, 0)
+    try:
+        y, its_y, res_y, _ = solver.solve(tol=TOL, mode=A.NLF_MODE_MIXED)
+    finally:
+        gpu_ctx.set_option(A.NLF_OPT_SPMV_SYMMETRIC, 1)
+    assert max(res.max(), res_y.max()) <= TOL
+    # the slices add in another order; the full storage gives the same bits again
+    assert torch.equal(x, y) == (not slices)
+    assert float((x - y).norm() / y.norm()) < BOUND
 
 
 def test_autotuner_has_nothing_to_choose(gpu_ctx, tmp_path):
